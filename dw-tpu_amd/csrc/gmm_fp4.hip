@@ -707,6 +707,19 @@ static int balanced_tiles() {
   return (*end == 0 && v >= 0 && v <= (1l << 30)) ? (int)v : kGmmBalancedTiles;
 }
 
+// Few rows per expert: the streaming kernel (gmm_stream.hip).  Measured
+// against the tiles below (both with streaming weight loads), us:
+//   32 experts, K = 7168, N = 4096: 1 token 49 -> 23; 4 rows an expert 81 -> 79, 10 rows 82 -> 91;
+//   256 experts, K = N = 4096: 3 rows an expert 398 -> 339, 7 rows 414 -> 386, 12 rows 412 -> 446;
+// so it is taken up to 6 rows per local expert; and, while an expert's rows
+// make one tile, also where even 256-column tiles would leave half of the CUs
+// idle (8 experts of 50 rows, K = 3072, N = 2560: 31 -> 26; K = 1024,
+// N = 640: 16 -> 8).
+static bool stream_rule(int64_t M, int64_t N, int64_t E_local, int ncu) {
+  if (M <= 6 * E_local) return true;
+  return M <= 64 * E_local && (M / 96 + E_local) * ((N + 255) / 256) <= ncu / 2;
+}
+
 // The bf16 grouped matmul (arguments checked by the caller).
 int launch_gmm_bf16(const uint16_t *lhs, const int32_t *row_idx, int64_t lhs_rows, int64_t M, int64_t K,
                     const uint8_t *weight, const uint8_t *scale, const int32_t *group_sizes, int num_groups,
@@ -720,6 +733,9 @@ int launch_gmm_bf16(const uint16_t *lhs, const int32_t *row_idx, int64_t lhs_row
   // local and full) leave CUs idle; larger launches never split, and run the
   // kernel without the narrow producers.
   const int ncu = device_cu_count();
+  if (stream_rule(M, N, E_local, ncu))
+    return launch_gmm_stream(lhs, row_idx, lhs_rows, M, K, weight, scale, group_sizes, num_groups, group_offset,
+                             E_local, N, out, out_f32, gated, ep, st);
   const bool narrow = ((M + 95) / 96) * ((N + 511) / 512) < ncu;
 #define DWM_GMM_WS(ACT, NARROW)                                                                                   \
   launch_gmm_ws<3, 8, 2, 4, 4, ACT, NARROW>(lhs, row_idx, lhs_rows, M, K, weight, scale, group_sizes, num_groups, \

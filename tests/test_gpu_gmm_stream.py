@@ -1,0 +1,115 @@
+"""The streaming kernel of the grouped matmul (csrc/gmm_stream.hip), which
+takes launches with few rows per expert: against the float64 oracle under the
+stated bound, and bit for bit against the 96-row tiles, which the same rows
+take when every group is padded with further rows (a row's result depends on
+its own lhs row and expert only)."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import bf16_bits, bf16_tensor
+from oracle import fp4 as ofp4
+from oracle import gmm as ogmm
+from oracle.numerics import bf16_bits as f32_to_bf16_bits
+from oracle.numerics import bf16_to_f32
+
+pytestmark = pytest.mark.gpu
+
+
+def _sizes(E, pattern):
+    return np.array([pattern[i % len(pattern)] for i in range(E)], np.int32)
+
+
+# K: 1, 2, 3, 4, 5, 7, 8 and 11 K blocks around the register ring's depths (3
+# and 4); N: ragged 64-column groups; groups past 64 and 256 (4 and 16 sizes
+# per lane); one- and four-wave blocks (the 300 groups); rows 15 / 16 / 17 and
+# 31 / 32 / 33 around the 16- and 32-row tiles; a few groups of many rows.
+CASES = [
+    (4, 128, 16, [1, 0, 2, 1], None, False, "none"),
+    (8, 256, 80, [1, 3, 0, 4], None, False, "f32"),
+    (12, 384, 272, [17, 0, 1, 0, 1, 2], None, False, "bias"),
+    (12, 512, 128, [16, 0, 15, 0, 1, 2], None, True, "none"),
+    (24, 640, 192, [31, 0, 0, 33, 0, 1, 0, 0, 0, 5, 0, 0], None, True, "bias"),
+    (40, 896, 320, [32, 0, 0, 0, 0, 70, 0, 0, 0, 0, 0, 0, 0, 1, 2, 3, 0, 0, 0, 0], None, False, "gather"),
+    (100, 1024, 64, [0, 1, 2, 0, 16, 0, 17, 3] + [0] * 12, (30, 40), False, "none"),
+    (300, 1408, 1280, [1, 0, 0, 2], None, False, "gather"),
+    (300, 128, 1040, [0, 1, 3, 0, 8], (7, 290), False, "f32"),
+    (1024, 256, 128, [0, 0, 1], None, True, "gather"),
+]
+
+
+@pytest.mark.parametrize("E,K,N,pattern,window,act,form", CASES)
+def test_stream_kernel_against_oracle_and_tiles(dev, rng, E, K, N, pattern, window, act, form):
+    from dw_tpu_amd import fp4_weight_to_codes, gmm_v2
+    sizes = _sizes(E, pattern)
+    go, e_local = window if window else (0, E)
+    M = int(sizes.sum())
+    assert 0 < M <= 6 * e_local, "the launch takes the streaming kernel"
+    rhs = rng.integers(0, 256, (e_local, K, N // 2), dtype=np.uint8)
+    sc = rng.integers(123, 130, (e_local, K // 32, 1, N), dtype=np.uint8)
+    pw = fp4_weight_to_codes(torch.from_numpy(rhs).to(dev), torch.from_numpy(sc).to(dev), gate_up=act)
+    bits = f32_to_bf16_bits(rng.standard_normal((M, K)).astype(np.float32))
+    bias = torch.from_numpy(rng.standard_normal((e_local, N)).astype(np.float32)).to(dev) if form == "bias" else None
+    kw = dict(rhs_bias=bias, group_offset=go if window else None,
+              preferred_element_type=torch.float32 if form == "f32" else None,
+              fuse_act="silu_and_mul_with_clamp" if act else None)
+    gs = torch.from_numpy(sizes).to(dev)
+    lhs = bf16_tensor(bits, dev)
+    if form == "gather":
+        idx = rng.permutation(M).astype(np.int32)
+        src = np.empty_like(bits)
+        src[idx] = bits
+        y = gmm_v2(bf16_tensor(src, dev), pw, gs, lhs_row_indices=torch.from_numpy(idx).to(dev), **kw)
+    else:
+        y = gmm_v2(lhs, pw, gs, **kw)
+    # The same rows at the head of groups padded to more than 72 rows each.
+    pad = 80
+    big = sizes + pad
+    assert big.sum() > 64 * e_local
+    starts = np.concatenate([[0], np.cumsum(big)[:-1]])
+    at = np.concatenate([s + np.arange(n) for s, n in zip(starts, sizes)]).astype(np.int64)
+    rows = np.zeros((int(big.sum()), K), np.uint16)
+    rows[at] = bits
+    at = torch.from_numpy(at).to(dev)
+    yb = gmm_v2(bf16_tensor(rows, dev), pw, torch.from_numpy(big).to(dev), **kw)[at]
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int32 if form == "f32" else torch.int16),
+                       yb.view(torch.int32 if form == "f32" else torch.int16))
+    lo, hi = int(sizes[:go].sum()), int(sizes[:go + e_local].sum())
+    assert (y[:lo] == 0).all() and (y[hi:] == 0).all()
+    if act or form == "bias":
+        return  # the epilogue is the tiles' own, compared bit for bit above
+    x = bf16_to_f32(bits)[lo:hi]
+    loc = sizes[go:go + e_local]
+    w = ogmm.dequant_rhs(ofp4.e2m1_to_codes(ofp4.unpack_nibbles(rhs)), ofp4.e8m0_decode(sc))
+    y64, _ = ogmm.gmm(x, None, None, loc, out_dtype="float64", w=w)
+    got = y[lo:hi].cpu().numpy() if form == "f32" else bf16_to_f32(bf16_bits(y[lo:hi]))
+    err = np.abs(got.astype(np.float64) - y64)
+    assert np.all(err <= ogmm.error_bound(y64, ogmm.abs_product(x, w, loc), K,
+                                          "float32" if form == "f32" else "bfloat16")), ogmm.error_stats(got, y64)
+
+
+def test_stream_kernel_skips_rows_past_m(dev, rng):
+    """Device group sizes whose sum passes M: no row past M is read or
+    written (lhs and out are padded), and rows below M are those of sizes cut
+    to fit."""
+    import ctypes
+    from dw_tpu_amd import _lib, fp4_weight_to_codes
+    E, K, N, M, pad = 16, 256, 128, 60, 64
+    sizes = _sizes(E, [5, 0, 40, 3])
+    assert M <= 6 * E and sizes.sum() > M + 40
+    pw = fp4_weight_to_codes(torch.from_numpy(rng.integers(0, 256, (E, K, N // 2), dtype=np.uint8)).to(dev),
+                             torch.from_numpy(rng.integers(123, 130, (E, K // 32, 1, N), dtype=np.uint8)).to(dev))
+    lhs = bf16_tensor(f32_to_bf16_bits(rng.standard_normal((M + pad, K)).astype(np.float32)), dev)
+    fit = np.minimum(sizes, np.maximum(0, M - np.concatenate([[0], np.cumsum(sizes)[:-1]]))).astype(np.int32)
+    outs = []
+    for s in (sizes, fit):
+        gs = torch.from_numpy(s).to(dev)
+        out = torch.full((M + pad, N), 0x1234, dtype=torch.int16, device=dev)
+        P = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+        _lib.call("dwm_gmm_fp4", P(lhs), M, K, P(pw.weight), P(pw.scale), P(gs), E, None, E, N, P(out), _lib.BF16, 0,
+                  _lib.ACT_NONE, _lib.stream_handle(dev))
+        torch.cuda.synchronize()
+        assert (out[M:] == 0x1234).all()
+        outs.append(out[:M])
+    assert torch.equal(outs[0], outs[1])

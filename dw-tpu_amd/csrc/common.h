@@ -114,6 +114,15 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *base, ui
 #define buffer_load_lds(SIZE, rsrc, lds, voffset, soffset) ((void)(rsrc), (void)(lds), (void)(voffset), (void)(soffset))
 #endif
 
+// 16 bytes per lane from src into LDS at lds + 16 * lane with cache policy AUX
+// (kAux*; a no-op in the host pass, like buffer_load_lds).
+#if defined(__HIP_DEVICE_COMPILE__)
+#define global_load_lds16(AUX, src, lds) \
+  __builtin_amdgcn_global_load_lds((const void *)(src), (lds_void_t *)(lds), 16, 0, AUX)
+#else
+#define global_load_lds16(AUX, src, lds) ((void)(src), (void)(lds))
+#endif
+
 // s_waitcnt immediate (gfx9 encoding): vmcnt <= vm, lgkmcnt == 0, expcnt untouched.
 __host__ __device__ constexpr int waitcnt_vm_lgkm0(int vm) { return (vm & 15) | ((vm >> 4) << 14) | (7 << 4); }
 

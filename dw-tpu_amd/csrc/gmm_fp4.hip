@@ -165,8 +165,9 @@ struct WsCfg {
 
 // Producer wave pw: NA of its A_LOADS lhs row groups hold rows of the tile;
 // the others are zero in every stage and never loaded.  It loads GL of the
-// tile's 64-column weight groups (G_LOADS in a wide tile, half in a narrow one).
-template <class C, int NA, int GL>
+// tile's 64-column weight groups (G_LOADS in a wide tile, half in a narrow one),
+// their weights with cache policy AUX (kAuxStream or 0: launch_gmm_bf16).
+template <class C, int NA, int GL, int AUX>
 __device__ __forceinline__ void ws_producer(const uint16_t *__restrict__ lhs, const int32_t *__restrict__ row_idx,
                                             int64_t lhs_rows, int64_t row0, int rows, int K, int T,
                                             int KB, const uint8_t *__restrict__ wexp,
@@ -217,9 +218,8 @@ __device__ __forceinline__ void ws_producer(const uint16_t *__restrict__ lhs, co
     for (int c = 0; c < GL; ++c) {
       const int gi = pw + NP * c;
       const uint8_t *const w = wsrc[c] + (int64_t)t * 2048;
-      __builtin_amdgcn_global_load_lds((const void *)w, (lds_void_t *)(st + C::W + gi * 2048), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((const void *)(w + 1024), (lds_void_t *)(st + C::W + gi * 2048 + 1024), 16,
-                                       0, 0);
+      global_load_lds16(AUX, w, st + C::W + gi * 2048);
+      global_load_lds16(AUX, w + 1024, st + C::W + gi * 2048 + 1024);
       __builtin_amdgcn_global_load_lds((const void *)(ssrc[c] + (int64_t)(t >> 1) * 256),
                                        (lds_void_t *)(st + C::S + gi * 256), 4, 0, 0);
     }
@@ -508,20 +508,20 @@ __device__ __forceinline__ void ws_idle_consumer(int T) {
 }
 
 // Producer dispatch on the number of lhs row groups that hold rows.
-template <class C, int GL>
+template <class C, int GL, int AUX>
 __device__ __forceinline__ void ws_produce(int na, const uint16_t *lhs, const int32_t *row_idx, int64_t lhs_rows,
                                            int64_t row0, int rows, int K, int T, int KB, const uint8_t *wexp,
                                            const uint8_t *sexp, int g0, int G, uint8_t *s_lds, int pw) {
   constexpr int AL = C::A_LOADS;
-  if (na >= AL) ws_producer<C, AL, GL>(lhs, row_idx, lhs_rows, row0, rows, K, T, KB, wexp, sexp, g0, G, s_lds, pw);
-  else if (na == 2) ws_producer<C, (AL > 2 ? 2 : AL), GL>(lhs, row_idx, lhs_rows, row0, rows, K, T, KB, wexp, sexp, g0, G, s_lds, pw);
-  else if (na == 1) ws_producer<C, (AL > 1 ? 1 : AL), GL>(lhs, row_idx, lhs_rows, row0, rows, K, T, KB, wexp, sexp, g0, G, s_lds, pw);
-  else ws_producer<C, 0, GL>(lhs, row_idx, lhs_rows, row0, rows, K, T, KB, wexp, sexp, g0, G, s_lds, pw);
+  if (na >= AL) ws_producer<C, AL, GL, AUX>(lhs, row_idx, lhs_rows, row0, rows, K, T, KB, wexp, sexp, g0, G, s_lds, pw);
+  else if (na == 2) ws_producer<C, (AL > 2 ? 2 : AL), GL, AUX>(lhs, row_idx, lhs_rows, row0, rows, K, T, KB, wexp, sexp, g0, G, s_lds, pw);
+  else if (na == 1) ws_producer<C, (AL > 1 ? 1 : AL), GL, AUX>(lhs, row_idx, lhs_rows, row0, rows, K, T, KB, wexp, sexp, g0, G, s_lds, pw);
+  else ws_producer<C, 0, GL, AUX>(lhs, row_idx, lhs_rows, row0, rows, K, T, KB, wexp, sexp, g0, G, s_lds, pw);
 }
 
 // NARROW: the tile list may cut its costliest classes into 256-column tiles
 // (find_tile) when the 512-column tiles leave some of the ncu CUs idle.
-template <class C, int MB, bool ACT, bool NARROW>
+template <class C, int MB, bool ACT, bool NARROW, int AUX>
 __global__ __launch_bounds__(C::THREADS) void gmm_fp4_ws_kernel(
     const uint16_t *__restrict__ lhs, const int32_t *__restrict__ row_idx, int64_t lhs_rows, int64_t M, int K,
     const uint8_t *__restrict__ wpk,
@@ -580,9 +580,9 @@ __global__ __launch_bounds__(C::THREADS) void gmm_fp4_ws_kernel(
     // Row groups pw + NP i with 8 (pw + NP i) < rows are loaded.
     const int na = min(C::A_LOADS, (rows + 8 * C::NPROD - 1 - 8 * pw) / (8 * C::NPROD));
     if (NARROW && narrow)
-      ws_produce<C, C::G_LOADS / 2>(na, lhs, row_idx, lhs_rows, row0, rows, K, T, KB, wexp, sexp, g0, G, s_lds, pw);
+      ws_produce<C, C::G_LOADS / 2, AUX>(na, lhs, row_idx, lhs_rows, row0, rows, K, T, KB, wexp, sexp, g0, G, s_lds, pw);
     else
-      ws_produce<C, C::G_LOADS>(na, lhs, row_idx, lhs_rows, row0, rows, K, T, KB, wexp, sexp, g0, G, s_lds, pw);
+      ws_produce<C, C::G_LOADS, AUX>(na, lhs, row_idx, lhs_rows, row0, rows, K, T, KB, wexp, sexp, g0, G, s_lds, pw);
     DWM_GS(gs_role(1u | (uint64_t)rows << 8 | (uint64_t)narrow << 24);)
     tl_exit();
     return;
@@ -670,7 +670,7 @@ static int device_cu_count() {
   return n;
 }
 
-template <int MB, int CW, int JW, int NP, int NS, bool ACT, bool NARROW>
+template <int MB, int CW, int JW, int NP, int NS, bool ACT, bool NARROW, int AUX>
 static int launch_gmm_ws(const uint16_t *lhs, const int32_t *row_idx, int64_t lhs_rows, int64_t M, int64_t K,
                          const uint8_t *w, const uint8_t *s,
                          const int32_t *gs, int ng, const int32_t *go, int64_t e_local, int64_t N, void *out,
@@ -685,7 +685,7 @@ static int launch_gmm_ws(const uint16_t *lhs, const int32_t *row_idx, int64_t lh
   const int64_t grid = ((entries + 7) / 8 + NC) * 8;
   DWM_UNSUPPORTED_IF(grid > (1ll << 31) - 1, "gmm_fp4: too many tiles (%lld)", (long long)grid);
   DWM_UNSUPPORTED_IF(K > (1 << 24), "gmm_fp4: K <= 2^24 required");
-  hipLaunchKernelGGL((gmm_fp4_ws_kernel<C, MB, ACT, NARROW>), dim3((unsigned)grid), dim3(C::THREADS), 0, st, lhs,
+  hipLaunchKernelGGL((gmm_fp4_ws_kernel<C, MB, ACT, NARROW, AUX>), dim3((unsigned)grid), dim3(C::THREADS), 0, st, lhs,
                      row_idx, lhs_rows, M, (int)K, w, s, gs, ng, go, e_local, (int)N, out, out_f32, ep, ncu, bal);
   return launch_status("gmm_fp4");
 }
@@ -737,11 +737,15 @@ int launch_gmm_bf16(const uint16_t *lhs, const int32_t *row_idx, int64_t lhs_row
     return launch_gmm_stream(lhs, row_idx, lhs_rows, M, K, weight, scale, group_sizes, num_groups, group_offset,
                              E_local, N, out, out_f32, gated, ep, st);
   const bool narrow = ((M + 95) / 96) * ((N + 511) / 512) < ncu;
-#define DWM_GMM_WS(ACT, NARROW)                                                                                   \
-  launch_gmm_ws<3, 8, 2, 4, 4, ACT, NARROW>(lhs, row_idx, lhs_rows, M, K, weight, scale, group_sizes, num_groups, \
-                                             group_offset, E_local, N, out, out_f32, ep, ncu, balanced_tiles(), st)
-  if (gated) return narrow ? DWM_GMM_WS(true, true) : DWM_GMM_WS(true, false);
-  return narrow ? DWM_GMM_WS(false, true) : DWM_GMM_WS(false, false);
+#define DWM_GMM_WS(ACT, NARROW, AUX)                                                                          \
+  launch_gmm_ws<3, 8, 2, 4, 4, ACT, NARROW, AUX>(lhs, row_idx, lhs_rows, M, K, weight, scale, group_sizes,    \
+                                                 num_groups, group_offset, E_local, N, out, out_f32, ep, ncu, \
+                                                 balanced_tiles(), st)
+#define DWM_GMM_WS_AUX(ACT, NARROW) \
+  (weights_read_once(M, E_local) ? DWM_GMM_WS(ACT, NARROW, kAuxStream) : DWM_GMM_WS(ACT, NARROW, 0))
+  if (gated) return narrow ? DWM_GMM_WS_AUX(true, true) : DWM_GMM_WS_AUX(true, false);
+  return narrow ? DWM_GMM_WS_AUX(false, true) : DWM_GMM_WS_AUX(false, false);
+#undef DWM_GMM_WS_AUX
 #undef DWM_GMM_WS
 }
 

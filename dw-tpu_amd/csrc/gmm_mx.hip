@@ -174,8 +174,10 @@ __global__ __launch_bounds__(256) void mx_quant_e2m1_kernel(const uint16_t *__re
 // AF4: the lhs is e2m1 (MXFP4: 32 bytes per row and 64-deep step, one
 // 16-byte A operand per lane, A format 4 in the MFMA) instead of e4m3 (64
 // bytes per row and step).
-template <int MB, int CW, int NP, int NS, int RH = 1, bool AF4 = false>
+// WAUX: cache policy of the weight loads (kAuxStream or 0).
+template <int MB, int CW, int NP, int NS, int RH, bool AF4, int WAUX>
 struct MxCfg {
+  static constexpr int AUX = WAUX;
   static constexpr int CONS = CW, NPROD = NP, STAGES = NS, HALVES = RH;
   static constexpr bool A_FP4 = AF4;
   static constexpr int GT = CW / RH;                     // 64-column groups per tile
@@ -275,9 +277,8 @@ __device__ __forceinline__ void mx_producer(const uint8_t *__restrict__ lhs, con
     for (int c = 0; c < C::G_LOADS; ++c) {
       const int gi = pw + NP * c;
       const uint8_t *const w = wsrc[c] + (int64_t)t * 2048;
-      __builtin_amdgcn_global_load_lds((const void *)w, (lds_void_t *)(st + C::W + gi * 2048), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((const void *)(w + 1024), (lds_void_t *)(st + C::W + gi * 2048 + 1024), 16,
-                                       0, 0);
+      global_load_lds16(C::AUX, w, st + C::W + gi * 2048);
+      global_load_lds16(C::AUX, w + 1024, st + C::W + gi * 2048 + 1024);
     }
     if ((t & 1) == 0) {
 #pragma unroll
@@ -511,8 +512,9 @@ __global__ __launch_bounds__(C::THREADS) void gmm_mx_kernel(
 // AF4: e2m1 lhs (MXFP4): 64 bytes per row and 128-deep step in four 16-byte
 // chunks, chunk c of row r at physical chunk c ^ ((r >> 2) & 3) (the e4m3
 // layout of the 64-deep kernel), 16 rows per 1 KiB load.
-template <int MB, int CW, int NP, int NS, bool AF4 = false>
+template <int MB, int CW, int NP, int NS, bool AF4, int WAUX>
 struct Mx128Cfg {
+  static constexpr int AUX = WAUX;
   static constexpr int CONS = CW, NPROD = NP, STAGES = NS;
   static constexpr bool A_FP4 = AF4;
   static constexpr int GT = CW;
@@ -597,8 +599,7 @@ __device__ __forceinline__ void mx128_producer(const uint8_t *__restrict__ lhs, 
       const uint8_t *const w = wsrc[c] + (int64_t)t * 4096;
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        __builtin_amdgcn_global_load_lds((const void *)(w + 1024 * q),
-                                         (lds_void_t *)(st + C::W + gi * 4096 + 1024 * q), 16, 0, 0);
+        global_load_lds16(C::AUX, w + 1024 * q, st + C::W + gi * 4096 + 1024 * q);
       __builtin_amdgcn_global_load_lds((const void *)(ssrc[c] + (int64_t)t * 256),
                                        (lds_void_t *)(st + C::S + gi * 256), 4, 0, 0);
     }
@@ -780,40 +781,49 @@ static int launch_mx(const uint8_t *lhs, const uint8_t *lsc, const int32_t *row_
   return launch_status("gmm_fp4_mx");
 }
 
+// One form of the MX grouped matmul: 96-row x 512-column tiles, 8 consumer +
+// 4 producer waves.  64-deep K steps in a five-stage ring (two published per
+// barrier, two in flight), or 128-deep steps in a three-stage ring (one
+// published, one in flight).  Below K = 4096, groups of 97 .. 192 rows on
+// average run 192 x 256 tiles (two stacked row halves), so their weights are
+// read once: decode_down (~128 rows per group) 111 -> 106 us, measured against
+// the 96 x 512 tiles; seven stages in place of five were slower (110 us).
+// Larger groups read their weights once per row tile either way.  Weights
+// that no other row tile of the expert reads are loaded with the streaming
+// policy (kAuxStream).  AF4: MXFP4 lhs, the same kernels with e2m1 A operands.
+template <bool ACT, bool AF4>
+static int launch_mx_form(const uint8_t *lhs, const uint8_t *lhs_scale, const int32_t *row_idx, int64_t lhs_rows,
+                          int64_t M, int64_t K, const uint8_t *weight, const uint8_t *scale,
+                          const int32_t *group_sizes, int num_groups, const int32_t *group_offset, int64_t E_local,
+                          int64_t N, void *out, int out_f32, const GmmEpilogue &ep, hipStream_t st) {
+  using H = MxCfg<3, 8, 4, 5, 2, AF4, 0>;  // streaming loads measured 98.4 -> 102.7 us at decode_down
+  using D0 = Mx128Cfg<3, 8, 4, 3, AF4, 0>;
+  using D1 = Mx128Cfg<3, 8, 4, 3, AF4, kAuxStream>;
+  using S0 = MxCfg<3, 8, 4, 5, 1, AF4, 0>;
+  using S1 = MxCfg<3, 8, 4, 5, 1, AF4, kAuxStream>;
+  const bool deep = K >= kMx128MinK;
+  const bool halves = !deep && M > 96 * E_local && M <= 192 * E_local;
+  const bool once = weights_read_once(M, E_local);
+#define DWM_MX(CFG, TMB, DEEP)                                                                                    \
+  launch_mx<CFG, TMB, ACT, DEEP>(lhs, lhs_scale, row_idx, lhs_rows, M, K, weight, scale, group_sizes, num_groups, \
+                                 group_offset, E_local, N, out, out_f32, ep, st)
+  if (halves) return DWM_MX(H, 6, false);
+  if (deep) return once ? DWM_MX(D1, 3, true) : DWM_MX(D0, 3, true);
+  return once ? DWM_MX(S1, 3, false) : DWM_MX(S0, 3, false);
+#undef DWM_MX
+}
+
 // The MX grouped matmul (arguments checked by the caller).
 int launch_gmm_mx(const uint8_t *lhs, const uint8_t *lhs_scale, const int32_t *row_idx, int64_t lhs_rows, int64_t M,
                   int64_t K, const uint8_t *weight, const uint8_t *scale, const int32_t *group_sizes, int num_groups,
                   const int32_t *group_offset, int64_t E_local, int64_t N, void *out, int out_f32, bool gated,
                   const GmmEpilogue &ep, hipStream_t st, bool lhs_fp4) {
-  // 96-row x 512-column tiles, 8 consumer + 4 producer waves.  64-deep K
-  // steps in a five-stage ring (two published per barrier, two in flight),
-  // or 128-deep steps in a three-stage ring (one published, one in flight).
-  // Below K = 4096, groups of 97 .. 192 rows on average run 192 x 256
-  // tiles (two stacked row halves), so their weights are read once:
-  // decode_down (~128 rows per group) 111 -> 106 us, measured against the
-  // 96 x 512 tiles; seven stages in place of five were slower (110 us).
-  // Larger groups read their weights once per row tile either way.
-  using C64 = MxCfg<3, 8, 4, 5>;
-  using C64H = MxCfg<3, 8, 4, 5, 2>;
-  using C128 = Mx128Cfg<3, 8, 4, 3>;
-  // MXFP4 lhs: the same kernels with e2m1 A operands.
-  using F64 = MxCfg<3, 8, 4, 5, 1, true>;
-  using F64H = MxCfg<3, 8, 4, 5, 2, true>;
-  using F128 = Mx128Cfg<3, 8, 4, 3, true>;
-  const bool deep = K >= kMx128MinK;
-  const bool halves = !deep && M > 96 * E_local && M <= 192 * E_local;
-#define DWM_MX(CFG, TMB, ACT, DEEP)                                                                                \
-  launch_mx<CFG, TMB, ACT, DEEP>(lhs, lhs_scale, row_idx, lhs_rows, M, K, weight, scale, group_sizes, num_groups, \
-                                 group_offset, E_local, N, out, out_f32, ep, st)
-  if (lhs_fp4) {
-    if (gated)
-      return deep ? DWM_MX(F128, 3, true, true) : halves ? DWM_MX(F64H, 6, true, false) : DWM_MX(F64, 3, true, false);
-    return deep ? DWM_MX(F128, 3, false, true) : halves ? DWM_MX(F64H, 6, false, false) : DWM_MX(F64, 3, false, false);
-  }
-  if (gated)
-    return deep ? DWM_MX(C128, 3, true, true) : halves ? DWM_MX(C64H, 6, true, false) : DWM_MX(C64, 3, true, false);
-  return deep ? DWM_MX(C128, 3, false, true) : halves ? DWM_MX(C64H, 6, false, false) : DWM_MX(C64, 3, false, false);
-#undef DWM_MX
+#define DWM_MX_FORM(ACT, AF4)                                                                                     \
+  launch_mx_form<ACT, AF4>(lhs, lhs_scale, row_idx, lhs_rows, M, K, weight, scale, group_sizes, num_groups,       \
+                           group_offset, E_local, N, out, out_f32, ep, st)
+  if (lhs_fp4) return gated ? DWM_MX_FORM(true, true) : DWM_MX_FORM(false, true);
+  return gated ? DWM_MX_FORM(true, false) : DWM_MX_FORM(false, false);
+#undef DWM_MX_FORM
 }
 
 }  // namespace dwm

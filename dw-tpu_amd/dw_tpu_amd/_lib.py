@@ -148,9 +148,21 @@ def ptr(t):
     return None if t is None else ctypes.c_void_p(t.data_ptr())
 
 
+def addr(t):
+    """Device address of a tensor as an int (None for None): what ctypes
+    takes for a pointer argument with no c_void_p object in between."""
+    return None if t is None else t.data_ptr()
+
+
 def stream_handle(device=None):
     """The current torch stream of ``device`` as a hipStream_t."""
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+
+
+def raw_stream(device):
+    """``stream_handle`` of a tensor's device as an int, with no Stream
+    object made (0.2 us of host time against 1.5)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def dtype_code(dt):

@@ -19,6 +19,7 @@ Modes: "native", "wide", "flipped" and "megablox" are one arithmetic on
 MI355X; "pre" (``matmul_pre``) is the reference's other rounding.
 """
 import ctypes
+import functools
 import warnings
 from dataclasses import dataclass
 
@@ -55,20 +56,34 @@ def prepack_fp8(weight: torch.Tensor) -> Fp8Weight:
     dev = _lib.require_cuda(w)
     k, n = w.shape
     out = torch.empty(k * n, dtype=torch.uint8, device=dev)
-    _lib.call("dwm_dense_fp8_prepack", _lib.ptr(w), k, n, _lib.ptr(out), _lib.stream_handle(dev))
+    _lib.call("dwm_dense_fp8_prepack", _lib.addr(w), k, n, _lib.addr(out), _lib.raw_stream(dev))
     return Fp8Weight(out, k, n)
+
+
+@functools.lru_cache(maxsize=4096)
+def _default_workspace(m, k, n):
+    """Workspace bytes of the library's own plans (host arithmetic on the sizes alone)."""
+    b = ctypes.c_int64(0)
+    _lib.call("dwm_dense_fp8_workspace_size", m, k, n, ctypes.byref(b))
+    return b.value
 
 
 def _plan_and_workspace(m, k, n, dev, tile, w8a8):
     """(plan pointer or None, workspace tensor or None, workspace bytes)."""
-    plan = None if tile is None else tile_to_plan(tile, max(m, 1), k, n, w8a8)
-    b = ctypes.c_int64(0)
-    if plan is None:
-        _lib.call("dwm_dense_fp8_workspace_size", m, k, n, ctypes.byref(b))
+    if tile is None:
+        plan, need = None, _default_workspace(m, k, n)
     else:
-        _lib.call("dwm_dense_fp8_plan_workspace_size", m, k, n, ctypes.byref(plan), ctypes.byref(b))
-    ws = None if b.value == 0 else torch.empty(b.value, dtype=torch.uint8, device=dev)
-    return (None if plan is None else ctypes.byref(plan)), ws, b.value
+        p = tile_to_plan(tile, max(m, 1), k, n, w8a8)
+        b = ctypes.c_int64(0)
+        _lib.call("dwm_dense_fp8_plan_workspace_size", m, k, n, ctypes.byref(p), ctypes.byref(b))
+        plan, need = ctypes.byref(p), b.value
+    ws = None if need == 0 else torch.empty(need, dtype=torch.uint8, device=dev)
+    return plan, ws, need
+
+
+def _f32(t):
+    """``t`` as a contiguous f32 tensor (itself when it is one)."""
+    return t if t.dtype == torch.float32 and t.is_contiguous() else t.to(torch.float32).contiguous()
 
 
 def _aligned(t):
@@ -112,7 +127,7 @@ def matmul(x, w, s, *, tn=None, tk=None, tm=None, mode="native", stages=0):
     if k != pw.k:
         raise ValueError(f"x K={k} does not match weight K={pw.k}")
     x = _aligned(x)
-    sc = s.reshape(k // 128, n).to(torch.float32).contiguous()
+    sc = _f32(s.reshape(k // 128, n))
     dev = _lib.require_cuda(x, pw.weight, sc)
     tile = None if (tm, tk, tn) == (None, None, None) else DenseTile(mode, tm, tk, tn, stages)
     try:
@@ -122,8 +137,8 @@ def matmul(x, w, s, *, tn=None, tk=None, tm=None, mode="native", stages=0):
                       f"using the library's own plan", stacklevel=2)
         plan, ws, wsb = _plan_and_workspace(m, k, n, dev, None, False)
     out = torch.empty((m, n), dtype=torch.bfloat16, device=dev)
-    _lib.call("dwm_dense_fp8_w8a16_plan", _lib.ptr(x), m, k, n, _lib.ptr(pw.weight), _lib.ptr(sc), _lib.ptr(out),
-              plan, _lib.ptr(ws), wsb, _lib.stream_handle(dev))
+    _lib.call("dwm_dense_fp8_w8a16_plan", x.data_ptr(), m, k, n, pw.weight.data_ptr(), sc.data_ptr(), out.data_ptr(),
+              plan, _lib.addr(ws), wsb, _lib.raw_stream(dev))
     return out
 
 
@@ -146,8 +161,8 @@ def matmul_pre(x, w, s):
     _lib.call("dwm_dense_fp8_workspace_size", m, k, n, ctypes.byref(b))
     ws = None if b.value == 0 else torch.empty(b.value, dtype=torch.uint8, device=dev)
     out = torch.empty((m, n), dtype=torch.bfloat16, device=dev)
-    _lib.call("dwm_dense_fp8_w8a16_pre", _lib.ptr(x), m, k, n, _lib.ptr(pw.weight), _lib.ptr(sc), _lib.ptr(out),
-              _lib.ptr(ws), b.value, _lib.stream_handle(dev))
+    _lib.call("dwm_dense_fp8_w8a16_pre", _lib.addr(x), m, k, n, _lib.addr(pw.weight), _lib.addr(sc), _lib.addr(out),
+              _lib.addr(ws), b.value, _lib.raw_stream(dev))
     return out
 
 
@@ -163,13 +178,12 @@ def matmul_w8a8(xq, sx, w, sw, *, tile=None):
     if k != pw.k or tuple(sx.shape) != (m, k // 128) or tuple(sw.shape) != (k // 128, n // 128):
         raise ValueError("matmul_w8a8: shapes of xq, sx, w, sw do not match")
     xq = _aligned(xq)
-    sx = sx.to(torch.float32).contiguous()
-    sw = sw.to(torch.float32).contiguous()
+    sx, sw = _f32(sx), _f32(sw)
     dev = _lib.require_cuda(xq, sx, pw.weight, sw)
     plan, ws, wsb = _plan_and_workspace(m, k, n, dev, tile, True)
     out = torch.empty((m, n), dtype=torch.bfloat16, device=dev)
-    _lib.call("dwm_dense_fp8_w8a8_plan", _lib.ptr(xq), _lib.ptr(sx), m, k, n, _lib.ptr(pw.weight), _lib.ptr(sw),
-              _lib.ptr(out), plan, _lib.ptr(ws), wsb, _lib.stream_handle(dev))
+    _lib.call("dwm_dense_fp8_w8a8_plan", xq.data_ptr(), sx.data_ptr(), m, k, n, pw.weight.data_ptr(), sw.data_ptr(),
+              out.data_ptr(), plan, _lib.addr(ws), wsb, _lib.raw_stream(dev))
     return out
 
 
@@ -192,9 +206,13 @@ def select_tile(m, k, n):
     table = overrides()
     if (m, k, n) in table:
         return table[m, k, n]
-    if m < 1 or k < 128 or k % 128 or n < 16 or n % 16:
+    if not _takes(m, k, n):
         return None
     return plan_to_tile(default_plan(m, k, n), k)
+
+
+def _takes(m, k, n):
+    return m >= 1 and k >= 128 and k % 128 == 0 and n >= 16 and n % 16 == 0
 
 
 def try_dense_fp8(x, weight, scale):
@@ -208,15 +226,21 @@ def try_dense_fp8(x, weight, scale):
         return None
     m, k = x.shape
     wk, n = (weight.k, weight.n) if isinstance(weight, Fp8Weight) else weight.shape
-    entry = select_tile(m, k, n)
-    if entry is None or wk != k:
+    # select_tile's choice; without an override it is the library's own plan,
+    # which a launch with no tile makes by itself.
+    table = overrides()
+    own = (m, k, n) not in table
+    entry = None if own else table[m, k, n]
+    if (not _takes(m, k, n) if own else entry is None) or wk != k:
         return None
     if tuple(scale.shape) not in ((k // 128, 1, n), (1, k // 128, 1, n)):
         return None
     if not x.is_cuda:
         return None
-    mode, tm, tk, tn = entry
     try:
+        if own:
+            return matmul(x, weight, scale)
+        mode, tm, tk, tn = entry
         return matmul(x, weight, scale.reshape(k // 128, 1, n), tm=tm, tk=tk, tn=tn, mode=mode,
                       stages=getattr(entry, "stages", 0))
     except _lib.Unsupported:

@@ -105,8 +105,8 @@ def mx_quantize(x: torch.Tensor, fmt: str = "e4m3") -> MxLhs:
     dev = _lib.require_cuda(x)
     codes = torch.empty((rows, k // 2 if fmt == "e2m1" else k), dtype=torch.uint8, device=dev)
     scales = torch.empty((rows, k // MX_BLOCK), dtype=torch.uint8, device=dev)
-    _lib.call("dwm_mx_quant_e2m1" if fmt == "e2m1" else "dwm_mx_quant_e4m3", _lib.ptr(x), rows, k, _lib.ptr(codes),
-              _lib.ptr(scales), _lib.stream_handle(dev))
+    _lib.call("dwm_mx_quant_e2m1" if fmt == "e2m1" else "dwm_mx_quant_e4m3", _lib.addr(x), rows, k, _lib.addr(codes),
+              _lib.addr(scales), _lib.raw_stream(dev))
     return MxLhs(codes, scales, fmt)
 
 
@@ -150,7 +150,7 @@ def e2m1_to_codes(rhs: torch.Tensor) -> torch.Tensor:
     src = _as_bytes(rhs).contiguous()
     _lib.require_cuda(src)
     out = torch.empty_like(src, dtype=torch.uint8)
-    _lib.call("dwm_e2m1_to_codes", _lib.ptr(src), _lib.ptr(out), src.numel(), _lib.stream_handle(src.device))
+    _lib.call("dwm_e2m1_to_codes", _lib.addr(src), _lib.addr(out), src.numel(), _lib.raw_stream(src.device))
     return out
 
 
@@ -168,8 +168,8 @@ def decode_fp4(packed: torch.Tensor, fmt: int, scales: torch.Tensor = None, chec
             raise ValueError("scales must be uint8 e8m0 codes, one per 32 values")
     out = torch.empty(src.shape[:-1] + (src.shape[-1] * 2,), dtype=torch.bfloat16, device=src.device)
     flags = torch.zeros(1, dtype=torch.int32, device=src.device)
-    _lib.call("dwm_fp4_decode", _lib.ptr(src), fmt, n, _lib.ptr(scales), _lib.ptr(out), _lib.ptr(flags),
-              _lib.stream_handle(src.device))
+    _lib.call("dwm_fp4_decode", _lib.addr(src), fmt, n, _lib.addr(scales), _lib.addr(out), _lib.addr(flags),
+              _lib.raw_stream(src.device))
     if check and int(flags.item()) & 1:
         raise ValueError("e8m0 scale code 255 (not a finite power of two)")
     return out
@@ -251,13 +251,13 @@ def prepack_fp4(rhs: torch.Tensor, rhs_scale: torch.Tensor, rhs_fp4_codes: bool 
     flags = torch.zeros(1, dtype=torch.int32, device=src.device)
     fmt = _lib.FP4_CODES if rhs_fp4_codes else _lib.FP4_E2M1
     if transpose_rhs:
-        _lib.call("dwm_gmm_fp4_prepack_transposed", _lib.ptr(src), fmt, _lib.ptr(sc), _lib.dtype_code(sc.dtype), e,
-                  k, n, 1 if gate_up else 0, _lib.ptr(wout), _lib.ptr(sout), _lib.ptr(flags),
-                  _lib.stream_handle(src.device))
+        _lib.call("dwm_gmm_fp4_prepack_transposed", _lib.addr(src), fmt, _lib.addr(sc), _lib.dtype_code(sc.dtype), e,
+                  k, n, 1 if gate_up else 0, _lib.addr(wout), _lib.addr(sout), _lib.addr(flags),
+                  _lib.raw_stream(src.device))
     else:
         entry = "dwm_gmm_fp4_prepack_gate_up" if gate_up else "dwm_gmm_fp4_prepack"
-        _lib.call(entry, _lib.ptr(src), fmt, _lib.ptr(sc), _lib.dtype_code(sc.dtype), e, k, n,
-                  _lib.ptr(wout), _lib.ptr(sout), _lib.ptr(flags), _lib.stream_handle(src.device))
+        _lib.call(entry, _lib.addr(src), fmt, _lib.addr(sc), _lib.dtype_code(sc.dtype), e, k, n,
+                  _lib.addr(wout), _lib.addr(sout), _lib.addr(flags), _lib.raw_stream(src.device))
     f = int(flags.item())
     if f & 1:
         raise ValueError("rhs_scale holds a value that is not +0.0 or a power of two in the e8m0 range "
@@ -431,19 +431,19 @@ def gmm_v2(lhs: torch.Tensor,
     out = torch.empty((m, w.n // 2 if fused else w.n), dtype=out_dtype, device=dev)
     if mx_fmt == "e2m1":
         codes, scales = lhs.codes.contiguous(), lhs.scales.contiguous()
-        _lib.call("dwm_gmm_fp4_mxfp4", _lib.ptr(codes), _lib.ptr(scales), codes.shape[0], _lib.ptr(idx), m, w.k,
-                  _lib.ptr(w.weight), _lib.ptr(w.scale), _lib.ptr(bias),
-                  _lib.dtype_code(bias.dtype) if bias is not None else 0, _lib.ptr(gs), gs.numel(), _lib.ptr(go),
-                  w.num_experts, w.n, _lib.ptr(out), _lib.dtype_code(out_dtype), 1 if zero_initialize else 0,
-                  _lib.FUSE_ACTS[fuse_act], _lib.stream_handle(dev))
+        _lib.call("dwm_gmm_fp4_mxfp4", _lib.addr(codes), _lib.addr(scales), codes.shape[0], _lib.addr(idx), m, w.k,
+                  _lib.addr(w.weight), _lib.addr(w.scale), _lib.addr(bias),
+                  _lib.dtype_code(bias.dtype) if bias is not None else 0, _lib.addr(gs), gs.numel(), _lib.addr(go),
+                  w.num_experts, w.n, _lib.addr(out), _lib.dtype_code(out_dtype), 1 if zero_initialize else 0,
+                  _lib.FUSE_ACTS[fuse_act], _lib.raw_stream(dev))
         return out
     if mx:
         codes, scales = lhs.codes.contiguous(), lhs.scales.contiguous()
         desc = _lib.GmmLhs(codes.data_ptr(), scales.data_ptr(), codes.shape[0], None if idx is None else idx.data_ptr())
     else:
         desc = _lib.GmmLhs(lhs.data_ptr(), None, lhs.shape[0], None if idx is None else idx.data_ptr())
-    _lib.call("dwm_gmm_fp4_ex", ctypes.byref(desc), m, w.k, _lib.ptr(w.weight), _lib.ptr(w.scale), _lib.ptr(bias),
-              _lib.dtype_code(bias.dtype) if bias is not None else 0, _lib.ptr(gs), gs.numel(), _lib.ptr(go),
-              w.num_experts, w.n, _lib.ptr(out), _lib.dtype_code(out_dtype), 1 if zero_initialize else 0,
-              _lib.FUSE_ACTS[fuse_act], _lib.stream_handle(dev))
+    _lib.call("dwm_gmm_fp4_ex", ctypes.byref(desc), m, w.k, _lib.addr(w.weight), _lib.addr(w.scale), _lib.addr(bias),
+              _lib.dtype_code(bias.dtype) if bias is not None else 0, _lib.addr(gs), gs.numel(), _lib.addr(go),
+              w.num_experts, w.n, _lib.addr(out), _lib.dtype_code(out_dtype), 1 if zero_initialize else 0,
+              _lib.FUSE_ACTS[fuse_act], _lib.raw_stream(dev))
     return out

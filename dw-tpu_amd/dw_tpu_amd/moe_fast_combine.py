@@ -35,9 +35,9 @@ def _combine(x, indices, topk_weights, topk, out_dtype):
     idx = indices.reshape(-1).to(torch.int32).contiguous()
     dev = _lib.require_cuda(x, idx, w)
     out = torch.empty((num_tokens, x.shape[1]), dtype=out_dtype, device=dev)
-    _lib.call("dwm_moe_combine", _lib.ptr(x), _lib.dtype_code(x.dtype), x.shape[0], x.shape[1], _lib.ptr(idx),
-              _lib.ptr(w), _lib.dtype_code(w.dtype), num_tokens, topk, _lib.ptr(out),
-              _lib.dtype_code(out_dtype), _lib.stream_handle(dev))
+    _lib.call("dwm_moe_combine", _lib.addr(x), _lib.dtype_code(x.dtype), x.shape[0], x.shape[1], _lib.addr(idx),
+              _lib.addr(w), _lib.dtype_code(w.dtype), num_tokens, topk, _lib.addr(out),
+              _lib.dtype_code(out_dtype), _lib.raw_stream(dev))
     return out
 
 

@@ -48,10 +48,10 @@ def moe_dispatch(topk_indices: torch.Tensor, num_experts: int, check: bool = Fal
     rev = torch.empty(n, dtype=torch.int32, device=dev)
     gs = torch.empty(num_experts, dtype=torch.int32, device=dev)
     go = torch.empty(num_experts + 1, dtype=torch.int32, device=dev)
-    flags = torch.zeros(1, dtype=torch.int32, device=dev)
-    _lib.call("dwm_moe_dispatch", _lib.ptr(ids), t, topk, num_experts, _lib.ptr(perm), _lib.ptr(tok),
-              _lib.ptr(rev), _lib.ptr(gs), _lib.ptr(go), _lib.ptr(flags), _lib.ptr(workspace),
-              _lib.stream_handle(dev))
+    flags = torch.zeros(1, dtype=torch.int32, device=dev) if check else None  # a fill launch of its own
+    _lib.call("dwm_moe_dispatch", _lib.addr(ids), t, topk, num_experts, _lib.addr(perm), _lib.addr(tok),
+              _lib.addr(rev), _lib.addr(gs), _lib.addr(go), _lib.addr(flags), _lib.addr(workspace),
+              _lib.raw_stream(dev))
     if check and int(flags.item()):
         raise ValueError(f"topk_indices holds expert ids outside [0, {num_experts})")
     return Dispatch(perm, tok, rev, gs, go)
@@ -86,8 +86,8 @@ def row_gather(src: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
     dev = _lib.require_cuda(src, idx)
     rows = idx.numel()
     out = torch.empty((rows, src.shape[1]), dtype=src.dtype, device=dev)
-    _lib.call("dwm_row_gather", _lib.ptr(src), src.shape[0], src.shape[1] * src.element_size(),
-              _lib.ptr(idx), rows, _lib.ptr(out), _lib.stream_handle(dev))
+    _lib.call("dwm_row_gather", _lib.addr(src), src.shape[0], src.shape[1] * src.element_size(),
+              _lib.addr(idx), rows, _lib.addr(out), _lib.raw_stream(dev))
     return out
 
 
@@ -108,6 +108,6 @@ def fast_dispatch_gather(hidden: torch.Tensor, topk_argsort_indices: torch.Tenso
     dev = _lib.require_cuda(src, idx)
     rows = idx.numel()
     out = torch.empty((rows, src.shape[1]), dtype=src.dtype, device=dev)
-    _lib.call("dwm_dispatch_gather", _lib.ptr(src), src.shape[0], src.shape[1] * src.element_size(),
-              _lib.ptr(idx), rows, int(topk), _lib.ptr(out), _lib.stream_handle(dev))
+    _lib.call("dwm_dispatch_gather", _lib.addr(src), src.shape[0], src.shape[1] * src.element_size(),
+              _lib.addr(idx), rows, int(topk), _lib.addr(out), _lib.raw_stream(dev))
     return out

@@ -83,9 +83,9 @@ def fused_moe_fp4_routing(gating_output: torch.Tensor, top_k: int, renormalize: 
         num_valid = num_valid.to(device=dev, dtype=torch.int32).reshape(1).contiguous()
     w = torch.empty((t, top_k), dtype=dtype, device=dev)
     ids = torch.empty((t, top_k), dtype=torch.int32, device=dev)
-    _lib.call("dwm_route_topk", _lib.ptr(logits), _lib.dtype_code(logits.dtype), t, e, int(top_k),
-              _lib.SCORE_FNS[scoring_fn], _lib.ptr(bias), _lib.ptr(hash_ids), 1 if renormalize else 0,
-              _lib.ptr(num_valid), _lib.ptr(w), _lib.dtype_code(dtype), _lib.ptr(ids), _lib.stream_handle(dev))
+    _lib.call("dwm_route_topk", _lib.addr(logits), _lib.dtype_code(logits.dtype), t, e, int(top_k),
+              _lib.SCORE_FNS[scoring_fn], _lib.addr(bias), _lib.addr(hash_ids), 1 if renormalize else 0,
+              _lib.addr(num_valid), _lib.addr(w), _lib.dtype_code(dtype), _lib.addr(ids), _lib.raw_stream(dev))
     return w, ids
 
 
@@ -100,6 +100,6 @@ def dedupe_topk(topk_weights: torch.Tensor, topk_ids: torch.Tensor, num_experts:
     ids = topk_ids.to(torch.int32).contiguous()
     w_out = torch.empty_like(w)
     ids_out = torch.empty_like(ids)
-    _lib.call("dwm_dedupe_topk", _lib.ptr(w), _lib.ptr(ids), t, k, int(num_experts), _lib.ptr(w_out),
-              _lib.ptr(ids_out), _lib.stream_handle(w.device))
+    _lib.call("dwm_dedupe_topk", _lib.addr(w), _lib.addr(ids), t, k, int(num_experts), _lib.addr(w_out),
+              _lib.addr(ids_out), _lib.raw_stream(w.device))
     return w_out, ids_out

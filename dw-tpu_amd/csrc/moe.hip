@@ -4,7 +4,7 @@
 // one_hot(...).sum(0) (patches/tpu-inference-ext/0405-moe-fast-dispatch.patch:70-98,
 // kernels/tpu_inference/layers/common/moe_fast_dispatch.py:41-44) with a
 // counting sort that is bit-exact to a stable argsort, in three launches
-// (one block for batches of up to 8192 ids, dispatch_fused_kernel):
+// (one launch for batches of up to kWideMax ids, dispatch_wide_kernel):
 //   1. per 1024-id chunk, an LDS histogram -> counts[chunk][expert]
 //   2. one block: group sizes, exclusive offsets, per-(chunk, expert) bases
 //   3. per chunk, in id order (256 ids per step, wave by wave): each lane's
@@ -166,81 +166,90 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_kernel(
   }
 }
 
-// Small batches (n <= kFusedMax ids) over 64 or more experts (fewer take
-// dispatch_small_kernel below): one block of 1024 threads runs all three
-// steps -- the LDS histogram, the scan (wave 0) and the stable scatter in
-// 1024-id steps -- in one launch, with no workspace round trip.
-constexpr int kFusedThreads = 1024, kFusedMax = 8192;
+// Up to kWideMax ids in one launch: block b of 1024 threads counts all n ids
+// by key in LDS (those before its portion and the rest apart; every block
+// reads the ids from L2), scans the totals, and places its own 1024 ids.
+// What bounds three launches (count, scan, scatter) is their latency, not
+// their work: 24576 ids over 256 experts took 3.9 + 6.5 + 6.4 us and the gaps
+// between them, this kernel one launch.  The repeated count grows with n (64
+// LDS atomics per thread at kWideMax), so larger batches keep the three.
+// Few experts and few ids take dispatch_small_kernel below.
+constexpr int kFusedThreads = 1024, kSmallMax = 8192, kWideMax = 65536;
 
-__global__ __launch_bounds__(kFusedThreads) void dispatch_fused_kernel(const int32_t *ids, int64_t n, int topk,
-                                                                       int E, int32_t *perm, int32_t *tok_sorted,
-                                                                       int32_t *revert, int32_t *group_sizes,
-                                                                       int32_t *group_offsets, int32_t *flags) {
-  constexpr int W = kFusedThreads / 64;
-  __shared__ int s_run[kMaxExperts + 1];     // counts, then the next position of each key
-  __shared__ int s_wcnt[W][kMaxExperts + 1];  // this step's count of each key per wave
+__global__ __launch_bounds__(kFusedThreads) void dispatch_wide_kernel(const int32_t *ids, int64_t n, int topk, int E,
+                                                                      int32_t *perm, int32_t *tok_sorted,
+                                                                      int32_t *revert, int32_t *group_sizes,
+                                                                      int32_t *group_offsets, int32_t *flags) {
+  constexpr int W = kFusedThreads / 64, U = 8;
+  __shared__ int s_bef[kMaxExperts + 1];      // ids of each key before the portion, then the portion's first position
+  __shared__ int s_rest[kMaxExperts + 1];     // the other ids of each key
+  __shared__ int s_wcnt[W][kMaxExperts + 1];  // the portion's count of each key per wave
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   for (int e = tid; e <= E; e += kFusedThreads) {
-    s_run[e] = 0;
+    s_bef[e] = 0;
+    s_rest[e] = 0;
 #pragma unroll
     for (int w = 0; w < W; ++w) s_wcnt[w][e] = 0;
   }
-  __syncthreads();
+  const int64_t base = (int64_t)blockIdx.x * kFusedThreads, j = base + tid;
+  const bool active = j < n;
   bool bad = false;
-  for (int64_t j = tid; j < n; j += kFusedThreads) atomicAdd(&s_run[dispatch_key(ids[j], E, &bad)], 1);
-  if (bad && flags) atomicOr(flags, 1);
+  const int key = active ? dispatch_key(ids[j], E, &bad) : 0;
+  int nbits = 0;
+  while ((1 << nbits) <= E) ++nbits;  // keys 0..E
+  uint64_t peers = __ballot(active);
+  for (int b = 0; b < nbits; ++b) {
+    const bool bit = (key >> b) & 1;
+    const uint64_t m = __ballot(bit);
+    peers &= bit ? m : ~m;
+  }
+  const int rank = __popcll(peers & ((1ull << lane) - 1ull));
+  __syncthreads();
+  if (active && rank == 0) s_wcnt[wave][key] = __popcll(peers);
+  for (int64_t j0 = 0; j0 < n; j0 += U * kFusedThreads) {
+    int id[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {  // the loads of a round side by side
+      const int64_t i = j0 + u * kFusedThreads + tid;
+      id[u] = i < n ? ids[i] : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t i0 = j0 + u * kFusedThreads;
+      if (i0 + tid < n) atomicAdd(i0 < base ? &s_bef[dispatch_key(id[u], E, &bad)] : &s_rest[dispatch_key(id[u], E, &bad)], 1);
+    }
+  }
+  if (bad && flags && blockIdx.x == 0) atomicOr(flags, 1);
   __syncthreads();
   if (wave == 0) {
     int carry = 0;
     for (int b = 0; b <= E; b += 64) {
       const int e = b + lane;
-      const int v = e <= E ? s_run[e] : 0;
+      const int bef = e <= E ? s_bef[e] : 0;
+      const int v = e <= E ? bef + s_rest[e] : 0;
       const int inc = wave_inclusive_scan(v);
       if (e <= E) {
-        if (e < E) group_sizes[e] = v;
-        if (group_offsets) group_offsets[e] = carry + inc - v;  // entry E = number of valid ids
-        s_run[e] = carry + inc - v;
+        const int off = carry + inc - v;
+        if (blockIdx.x == 0) {
+          if (e < E) group_sizes[e] = v;
+          if (group_offsets) group_offsets[e] = off;  // entry E = number of valid ids
+        }
+        s_bef[e] = off + bef;
       }
       carry += wave_last(inc);
     }
   }
-  int nbits = 0;
-  while ((1 << nbits) <= E) ++nbits;  // keys 0..E
   __syncthreads();
-  for (int64_t base = 0; base < n; base += kFusedThreads) {
-    const int64_t j = base + tid;
-    const bool active = j < n;
-    bool b2 = false;
-    const int key = active ? dispatch_key(ids[j], E, &b2) : 0;
-    uint64_t peers = __ballot(active);
-    for (int b = 0; b < nbits; ++b) {
-      const bool bit = (key >> b) & 1;
-      const uint64_t m = __ballot(bit);
-      peers &= bit ? m : ~m;
-    }
-    const int rank = __popcll(peers & ((1ull << lane) - 1ull));
-    const int cnt = __popcll(peers);
-    const bool leader = active && rank == 0;
-    if (leader) s_wcnt[wave][key] = cnt;
-    __syncthreads();
-    if (active) {
-      int pos = s_run[key] + rank;
-      for (int w = 0; w < wave; ++w) pos += s_wcnt[w][key];
-      perm[pos] = (int32_t)j;
-      tok_sorted[pos] = (int32_t)(j / topk);
-      revert[j] = pos;
-    }
-    __syncthreads();
-    if (leader) {
-      atomicAdd(&s_run[key], cnt);
-      s_wcnt[wave][key] = 0;
-    }
-    __syncthreads();
+  if (active) {
+    int pos = s_bef[key] + rank;
+    for (int w = 0; w < wave; ++w) pos += s_wcnt[w][key];
+    perm[pos] = (int32_t)j;
+    tok_sorted[pos] = (int32_t)(j / topk);
+    revert[j] = pos;
   }
 }
 
-
-// Small batches over few experts (n <= kFusedMax ids, E + 1 <= 64 keys):
+// Small batches over few experts (n <= kSmallMax ids, E + 1 <= 64 keys):
 // the scattered stores, not the ranking, set the time of a one-block
 // dispatch, so the ids are split into portions of 512 over up to 16 blocks.
 // Every block counts all n ids (cheap: 16 waves, one 64-id round each per
@@ -257,7 +266,7 @@ __global__ __launch_bounds__(kFusedThreads) void dispatch_small_kernel(const int
                                                                        int32_t *revert, int32_t *group_sizes,
                                                                        int32_t *group_offsets, int32_t *flags) {
   constexpr int W = kFusedThreads / 64, PR = kSmallPortion / 64;     // waves; rounds per portion
-  constexpr int RMAX = kFusedMax / kFusedThreads;                      // rounds per wave
+  constexpr int RMAX = kSmallMax / kFusedThreads;                      // rounds per wave
   static_assert(PR <= W, "a portion's rounds fall on distinct waves");
   __shared__ int s_tot[W][kSmallMaxKeys], s_bef[W][kSmallMaxKeys];
   __shared__ int s_rc[PR][kSmallMaxKeys];  // per round of the portion: count of each key
@@ -512,15 +521,16 @@ static int dispatch_launch(const int32_t *topk_ids, int64_t n, int topk, int num
                        group_sizes, group_offsets);
     return launch_status("moe_dispatch");
   }
-  if (n <= kFusedMax && num_experts < kSmallMaxKeys) {
+  if (n <= kSmallMax && num_experts < kSmallMaxKeys) {
     const unsigned blocks = (unsigned)((n + kSmallPortion - 1) / kSmallPortion);
     hipLaunchKernelGGL(dispatch_small_kernel, dim3(blocks), dim3(kFusedThreads), 0, st, topk_ids, n, topk,
                        num_experts, perm, tok_sorted, revert, group_sizes, group_offsets, flags);
     return launch_status("moe_dispatch");
   }
-  if (n <= kFusedMax) {
-    hipLaunchKernelGGL(dispatch_fused_kernel, dim3(1), dim3(kFusedThreads), 0, st, topk_ids, n, topk,
-                       num_experts, perm, tok_sorted, revert, group_sizes, group_offsets, flags);
+  if (n <= kWideMax) {
+    hipLaunchKernelGGL(dispatch_wide_kernel, dim3((unsigned)((n + kFusedThreads - 1) / kFusedThreads)),
+                       dim3(kFusedThreads), 0, st, topk_ids, n, topk, num_experts, perm, tok_sorted, revert,
+                       group_sizes, group_offsets, flags);
     return launch_status("moe_dispatch");
   }
   hipLaunchKernelGGL(dispatch_count_kernel, dim3((unsigned)nchunks), dim3(kDispThreads), 0, st,
@@ -612,15 +622,15 @@ extern "C" int dwm_moe_dispatch_noalloc(const int32_t *topk_ids, int64_t T, int 
   if (rc != DWM_OK) return rc;
   const int64_t n = T * topk;
   const int64_t words = (n + kChunk - 1) / kChunk * (int64_t)(num_experts + 1);
-  DWM_UNSUPPORTED_IF(n > kFusedMax && words > kNoAllocWords,
+  DWM_UNSUPPORTED_IF(n > kWideMax && words > kNoAllocWords,
                      "moe_dispatch_noalloc: %lld ids over %d experts need %lld counter words, more than the "
                      "%lld of its static scratch (use dwm_moe_dispatch with a workspace)",
                      (long long)n, num_experts, (long long)words, (long long)kNoAllocWords);
-  // Only the three-launch path (n > kFusedMax) uses the counters: smaller
+  // Only the three-launch path (n > kWideMax) uses the counters: smaller
   // batches never look the array up, so their first call on a device does
   // no runtime lookup (e.g. inside a stream capture).
   int32_t *counts = nullptr;
-  if (n > kFusedMax) {
+  if (n > kWideMax) {
     counts = device_scratch();
     if (!counts) return DWM_ERR_HIP;
   }

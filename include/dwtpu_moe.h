@@ -305,7 +305,7 @@ int dwm_moe_dispatch(const int32_t *topk_ids, int64_t T, int topk, int num_exper
 /* dwm_moe_dispatch without a workspace argument and without allocating: no
  * counterpart in the reference; it is for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops).  The
- * chunk counters of batches above 8192 ids live in a 4 MiB device array of
+ * chunk counters of batches above 65536 ids live in a 4 MiB device array of
  * the library (one per GPU, held until the process ends), so
  * ceil(T*topk / 1024) * (num_experts + 1) must be <= 2^20 (e.g. T*topk <=
  * 4,177,920 at 256 experts); larger requests return DWM_ERR_UNSUPPORTED
@@ -313,7 +313,7 @@ int dwm_moe_dispatch(const int32_t *topk_ids, int64_t T, int topk, int num_exper
  * calls that overlap on one GPU (on different streams) race and must not be
  * issued.  Results are bit-identical to dwm_moe_dispatch's.  The array's
  * address on a device is looked up (hipGetSymbolAddress) by the first call
- * there with more than 8192 ids; batches of at most 8192 ids never use it.
+ * there with more than 65536 ids; batches of at most 65536 ids never use it.
  * A caller that captures a larger batch into a HIP graph makes one such
  * call on that device before the capture. */
 int dwm_moe_dispatch_noalloc(const int32_t *topk_ids, int64_t T, int topk, int num_experts, int32_t *perm,

@@ -461,8 +461,9 @@ __global__ __launch_bounds__(256) void combine_kernel(const void *x, int64_t x_r
 // same arithmetic as combine_kernel, but each row's 8 values stay packed
 // (one 16-byte register quad per row, widened while accumulating), so a
 // thread holds its kCombineKG rows in 32 registers and every block of the
-// decode shapes is resident at once (8 waves per SIMD).
-template <int OF32>
+// decode shapes is resident at once (8 waves per SIMD).  NT: the rows are
+// loaded with the streaming policy (kCombineStreamBytes).
+template <int OF32, int NT>
 __global__ __launch_bounds__(256) void combine_bf16_kernel(const uint16_t *__restrict__ x, int64_t x_rows, int64_t H,
                                                            const int32_t *__restrict__ idx, const void *w,
                                                            int w_dtype, int64_t T, int topk, void *out) {
@@ -480,7 +481,8 @@ __global__ __launch_bounds__(256) void combine_bf16_kernel(const uint16_t *__res
         if (k0 + g < topk) {
           const int64_t r = gather_index(idx[t * topk + k0 + g], x_rows);
           wk[g] = load_f32(w, w_dtype, t * topk + k0 + g);
-          raw[g] = *(const u32x4_t *)(x + r * H + c);
+          const u32x4_t *const p = (const u32x4_t *)(x + r * H + c);
+          raw[g] = NT ? __builtin_nontemporal_load(p) : *p;
         }
       }
 #pragma unroll
@@ -508,6 +510,13 @@ __global__ __launch_bounds__(256) void combine_bf16_kernel(const uint16_t *__res
     }
   }
 }
+
+// Each expert row is read once, so its lines only displace others.  Rows past
+// half of the 256 MB Infinity Cache were not kept there since they were
+// written and stream past it: 201 MB (4096 tokens, top-6, H = 4096) the
+// routing around them 126.6 -> 118.7 us, 229 MB 132.9 -> 126.7; rows that are
+// still cached lose (57 MB 40.3 -> 41.9, 49 MB 37.8 -> 38.9).
+constexpr int64_t kCombineStreamBytes = 128ll << 20;
 
 // The dispatch launches for n = T * topk ids with chunk counters `counts`
 // (nchunks * (E + 1) int32, fully written by the count kernel before they are
@@ -690,12 +699,18 @@ extern "C" int dwm_moe_combine(const void *x, int x_dtype, int64_t x_rows, int64
   hipStream_t st = as_stream(stream);
   const int of32 = out_dtype == DWM_F32;
   if (vec && !xf32) {
-    if (of32)
-      hipLaunchKernelGGL((combine_bf16_kernel<1>), grid, dim3(256), 0, st, (const uint16_t *)x, x_rows, H, idx, w,
-                         w_dtype, T, topk, out);
-    else
-      hipLaunchKernelGGL((combine_bf16_kernel<0>), grid, dim3(256), 0, st, (const uint16_t *)x, x_rows, H, idx, w,
-                         w_dtype, T, topk, out);
+#define DWM_COMBINE(OF32, NT)                                                                                    \
+  hipLaunchKernelGGL((combine_bf16_kernel<OF32, NT>), grid, dim3(256), 0, st, (const uint16_t *)x, x_rows, H,    \
+                     idx, w, w_dtype, T, topk, out)
+    const bool nt = T * topk * H * 2 > kCombineStreamBytes;
+    if (of32) {
+      if (nt) DWM_COMBINE(1, 1);
+      else DWM_COMBINE(1, 0);
+    } else {
+      if (nt) DWM_COMBINE(0, 1);
+      else DWM_COMBINE(0, 0);
+    }
+#undef DWM_COMBINE
     return launch_status("moe_combine");
   }
   if (!xf32 && !of32)

@@ -279,21 +279,25 @@ __global__ __launch_bounds__(kDenseThreads) void dense_fp8_kernel(
 // its lhs fragments (straight from L2, only rows < M) through a D-deep
 // register ring; there is no LDS staging and no barrier in the K loop.
 // The waves' f32 partial sums are added in LDS in wave order (deterministic)
-// and rounded once, in the same launch.
-template <int KS, int D, bool A8>
+// and rounded once, in the same launch.  With NB > 1 the block owns NB
+// 16-column groups and every wave streams all of them for its K steps, so the
+// lhs fragments are loaded once per NB groups; the sums and their order are
+// the same.
+template <int KS, int D, int NB, bool A8>
 __global__ __launch_bounds__(64 * KS) void dense_fp8_skinny_kernel(
     const void *__restrict__ xin, const float *__restrict__ sx, int M, int K, int N,
     const uint8_t *__restrict__ wpk, const float *__restrict__ sw, int sw_ld, uint16_t *__restrict__ out) {
-  __shared__ f32x4_t s_red[KS - 1][64];
+  static_assert(NB <= KS, "one wave sums each column group");
+  __shared__ f32x4_t s_red[KS][NB][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int KB = K >> 7;
-  const int nb = blockIdx.x;
+  const int nb = blockIdx.x * NB;
   const int kb_per = (KB + KS - 1) / KS;
   const int kb_begin = wave * kb_per;
   const int kb_end = min(KB, kb_begin + kb_per);
   const int r = lane & 15, q = lane >> 4;
   const bool rok = r < M;
-  const int64_t col = (int64_t)nb * 16 + r;  // C layout: column lane % 16, rows 4 q .. 4 q + 3
+  const int64_t col = (int64_t)nb * 16 + r;  // C layout: column lane % 16 (of group g: + 16 g), rows 4 q .. 4 q + 3
   const uint8_t *const wp = wpk + (int64_t)nb * KB * 2048 + lane * 32;
   // lhs fragment of MFMA step s: row r, k = 128 kb + 32 q + 8 s .. + 7
   const uint8_t *const xrow = (const uint8_t *)xin + (int64_t)(rok ? r : 0) * K * (A8 ? 1 : 2) + 32 * q * (A8 ? 1 : 2);
@@ -302,12 +306,15 @@ __global__ __launch_bounds__(64 * KS) void dense_fp8_skinny_kernel(
   // the wait for block kb then covers only loads issued before those of
   // block kb + 1 (vector loads complete in order), so D blocks stay in flight.
   constexpr int XW = A8 ? 2 : 4;  // 16-byte lhs loads per K block
-  u32x4_t wlo[D], whi[D], xa[D][XW];
-  float wsc[D], xsc[D][4];
+  u32x4_t wlo[D][NB], whi[D][NB], xa[D][XW];
+  float wsc[D][NB], xsc[D][4];
   auto load = [&](int slot, int kb) {
-    const u32x4_t *p = (const u32x4_t *)(wp + (int64_t)kb * 2048);
-    wlo[slot] = p[0];
-    whi[slot] = p[1];
+#pragma unroll
+    for (int g = 0; g < NB; ++g) {
+      const u32x4_t *p = (const u32x4_t *)(wp + ((int64_t)g * KB + kb) * 2048);
+      wlo[slot][g] = p[0];
+      whi[slot][g] = p[1];
+    }
     if (rok) {
       const u32x4_t *xp = (const u32x4_t *)(xrow + (int64_t)kb * (A8 ? 128 : 256));
 #pragma unroll
@@ -316,7 +323,9 @@ __global__ __launch_bounds__(64 * KS) void dense_fp8_skinny_kernel(
 #pragma unroll
       for (int s = 0; s < XW; ++s) xa[slot][s] = u32x4_t{0u, 0u, 0u, 0u};
     }
-    wsc[slot] = A8 ? sw[(int64_t)kb * sw_ld + (col >> 7)] : sw[(int64_t)kb * sw_ld + col];
+#pragma unroll
+    for (int g = 0; g < NB; ++g)
+      wsc[slot][g] = A8 ? sw[(int64_t)kb * sw_ld + ((col + 16 * g) >> 7)] : sw[(int64_t)kb * sw_ld + col + 16 * g];
     if (A8) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) xsc[slot][i] = sx[(int64_t)min(4 * q + i, M - 1) * KB + kb];
@@ -325,7 +334,9 @@ __global__ __launch_bounds__(64 * KS) void dense_fp8_skinny_kernel(
 #pragma unroll
   for (int d = 0; d < D; ++d)
     if (kb_begin + d < kb_end) load(d, kb_begin + d);
-  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+  f32x4_t acc[NB];
+#pragma unroll
+  for (int g = 0; g < NB; ++g) acc[g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   for (int kb0 = kb_begin; kb0 < kb_end; kb0 += D) {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
@@ -344,36 +355,45 @@ __global__ __launch_bounds__(64 * KS) void dense_fp8_skinny_kernel(
 #pragma unroll
         for (int s = 0; s < 4; ++s) a[s] = xa[d][s];
       }
-      const u32x4_t lo = wlo[d], hi = whi[d];
-      const float wscale = wsc[d];
-      float f[4];
+      u32x4_t lo[NB], hi[NB];
+      float f[NB][4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) f[i] = A8 ? xsc[d][i] * wscale : wscale;
-      if (kb + D < kb_end) load(d, kb + D);
-      f32x4_t part = {0.f, 0.f, 0.f, 0.f};
+      for (int g = 0; g < NB; ++g) {
+        lo[g] = wlo[d][g];
+        hi[g] = whi[d][g];
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const uint32_t w0 = s < 2 ? lo[2 * s] : hi[2 * s - 4];
-        const uint32_t w1 = s < 2 ? lo[2 * s + 1] : hi[2 * s - 3];
-        const u32x4_t b = {cvt_fp8x2_bf16<false>(w0), cvt_fp8x2_bf16<true>(w0), cvt_fp8x2_bf16<false>(w1),
-                           cvt_fp8x2_bf16<true>(w1)};
-        part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[s]),
-                                                       __builtin_bit_cast(bf16x8_t, b), part, 0, 0, 0);
+        for (int i = 0; i < 4; ++i) f[g][i] = A8 ? xsc[d][i] * wsc[d][g] : wsc[d][g];
       }
-      // acc += part * scale (f32 multiply, then f32 add)
+      if (kb + D < kb_end) load(d, kb + D);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] = acc[i] + part[i] * f[i];
+      for (int g = 0; g < NB; ++g) {
+        f32x4_t part = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const uint32_t w0 = s < 2 ? lo[g][2 * s] : hi[g][2 * s - 4];
+          const uint32_t w1 = s < 2 ? lo[g][2 * s + 1] : hi[g][2 * s - 3];
+          const u32x4_t b = {cvt_fp8x2_bf16<false>(w0), cvt_fp8x2_bf16<true>(w0), cvt_fp8x2_bf16<false>(w1),
+                             cvt_fp8x2_bf16<true>(w1)};
+          part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[s]),
+                                                         __builtin_bit_cast(bf16x8_t, b), part, 0, 0, 0);
+        }
+        // acc += part * scale (f32 multiply, then f32 add)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[g][i] = acc[g][i] + part[i] * f[g][i];
+      }
     }
   }
-  if (wave > 0) s_red[wave - 1][lane] = acc;
-  __syncthreads();
-  if (wave > 0) return;
 #pragma unroll
-  for (int w = 0; w < KS - 1; ++w) acc = acc + s_red[w][lane];
+  for (int g = 0; g < NB; ++g) s_red[wave][g][lane] = acc[g];
+  __syncthreads();
+  if (wave >= NB) return;
+  f32x4_t sum = s_red[0][wave][lane];
+#pragma unroll
+  for (int w = 1; w < KS; ++w) sum = sum + s_red[w][wave][lane];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int m = 4 * q + i;
-    if (m < M) out[(int64_t)m * N + col] = f32_to_bf16_bits(acc[i]);
+    if (m < M) out[(int64_t)m * N + col + 16 * wave] = f32_to_bf16_bits(sum[i]);
   }
 }
 
@@ -1045,8 +1065,20 @@ static int run_dense(const void *x, const float *sx, int64_t M, int64_t K, int64
   float *const partial = need ? (float *)workspace : nullptr;
   const int ks = p.ksplit;
   if (p.kernel == DWM_DENSE_SKINNY) {
-    hipLaunchKernelGGL((dense_fp8_skinny_kernel<16, 2, A8>), dim3((unsigned)(N / 16)), dim3(1024), 0, st, x, sx,
-                       (int)M, (int)K, (int)N, w, sw, sw_ld, out);
+    // One K block per wave up to K = 2048: no more waves than K blocks, so that
+    // none is idle and more blocks share a CU (the same sums in the same order).
+    // Wide and shallow (at least two blocks per CU of 64 columns), a block
+    // takes four column groups.
+#define DWM_SKINNY(KS, D, NB)                                                                                   \
+  hipLaunchKernelGGL((dense_fp8_skinny_kernel<KS, D, NB, A8>), dim3((unsigned)(N / (16 * NB))), dim3(64 * KS), 0, \
+                     st, x, sx, (int)M, (int)K, (int)N, w, sw, sw_ld, out)
+    const bool wide = N % 64 == 0 && N / 64 >= 512;
+    if (K <= 512 && wide) DWM_SKINNY(4, 1, 4);
+    else if (K <= 512) DWM_SKINNY(4, 1, 1);
+    else if (K <= 1024 && wide) DWM_SKINNY(8, 1, 4);
+    else if (K <= 1024) DWM_SKINNY(8, 1, 1);
+    else DWM_SKINNY(16, 2, 1);
+#undef DWM_SKINNY
   } else if (p.kernel == DWM_DENSE_MFMA) {
     if constexpr (A8) {
       if (p.tile_m == 256) launch_mfma<DenseMfmaCfg<4, 2, true>, true, 3>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);

@@ -1,0 +1,53 @@
+"""The dense FP8 launches for few rows: the skinny kernel's forms for shallow K
+(fewer waves) and wide N (four column groups per block), against the float64
+oracle under the stated bound, with the plan the library launched."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import bf16_bits, bf16_tensor
+from oracle import dense_fp8 as odf
+from oracle import gmm as ogmm
+from oracle.numerics import bf16_to_f32
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(out, y64, ap, K):
+    y = bf16_to_f32(bf16_bits(out)).astype(np.float64)
+    err = np.abs(y - y64)
+    assert np.all(np.isfinite(y))
+    assert np.all(err <= odf.error_bound(y64, ap, K)), ogmm.error_stats(y, y64)
+
+
+@pytest.mark.parametrize("a8", [False, True])
+@pytest.mark.parametrize("M,K,N", [(1, 128, 48), (16, 512, 128), (5, 640, 256), (16, 1024, 80), (7, 1152, 128),
+                                   (3, 256, 32768), (16, 512, 32832), (9, 896, 32768), (16, 1024, 33024)])
+def test_skinny_forms_against_oracle(dev, a8, M, K, N):
+    from dw_tpu_amd.dense_fp8 import last_plan, matmul, matmul_w8a8
+    from dw_tpu_amd.workloads import make_dense_workload
+    if a8:
+        N = -(-N // 128) * 128
+    wl = make_dense_workload(M, K, N, seed=M + K + 1)
+    cols = np.unique(np.r_[0, 15, 16, 63, N - 17, N - 1, np.random.default_rng(1).integers(0, N, 200)] % N)
+    if a8:
+        out = matmul_w8a8(*(torch.from_numpy(v).to(dev) for v in (wl.xq, wl.sx, wl.wq, wl.sw)))
+        sw = np.repeat(wl.sw, 128, axis=1)[:, cols]
+        y64 = np.zeros((M, len(cols)))
+        ap = np.zeros_like(y64)
+        from oracle.numerics import E4M3_VALUES
+        xv, wv = E4M3_VALUES[wl.xq].astype(np.float64), E4M3_VALUES[wl.wq[:, cols]].astype(np.float64)
+        for kb in range(K // 128):
+            sl = slice(kb * 128, kb * 128 + 128)
+            f = wl.sx[:, kb][:, None].astype(np.float64) * sw[kb][None, :]
+            y64 += (xv[:, sl] @ wv[sl]) * f
+            ap += (np.abs(xv[:, sl]) @ np.abs(wv[sl])) * np.abs(f)
+    else:
+        out = matmul(bf16_tensor(wl.x_bits, dev), torch.from_numpy(wl.wq).to(dev).view(torch.float8_e4m3fn),
+                     torch.from_numpy(wl.s_w8a16).to(dev))
+        xf, wc, sc = bf16_to_f32(wl.x_bits), wl.wq[:, cols], wl.s_w8a16[:, :, cols]
+        y64 = odf.matmul_w8a16(xf, wc, sc, out_dtype="float64")
+        ap = odf.abs_product_w8a16(xf, wc, sc)
+    torch.cuda.synchronize()
+    assert last_plan().astuple() == (1, 16, 16, 16, 2)
+    _check(out[:, torch.from_numpy(cols).to(dev)], y64, ap, K)

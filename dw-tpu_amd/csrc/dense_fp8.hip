@@ -13,6 +13,7 @@
 //   (exact: 3 mantissa bits, exponents inside bf16's range) for bf16 MFMA
 //   32x32x16; W8A8 runs the fp8 MFMA 32x32x64 on the codes.
 // - M <= 16: dense_fp8_skinny_kernel (see below).
+// - W8A8, 17 <= M <= 96, N % 128 == 0: dense_fp8_rows_kernel (see below).
 // - Other shapes: dense_fp8_kernel, bf16 MFMA 16x16x32 on decoded codes.
 // Every product is the exact fp8 (or bf16 x fp8) product; the 128-K partial
 // is an f32 sum of them.
@@ -397,6 +398,132 @@ __global__ __launch_bounds__(64 * KS) void dense_fp8_skinny_kernel(
   }
 }
 
+// W8A8, 17 .. 96 rows: dense_fp8_rows_kernel.  What bounds it: the weight
+// stream and latency -- at 64 rows, K = 7168, N = 4096 the weights take 5 us
+// of HBM time and the fp8 MFMAs under 2 us, but the 128-row MFMA tiles took
+// 17 us: half of their rows were padding, every step waited at a barrier for
+// LDS copies of operands that no second wave needs, and the eight K runs of a
+// tile wrote 17 MB of partials.
+// Here nothing is staged: a wave owns 16 MB rows x 16 NB columns and a run of
+// K blocks, and loads its operands straight into registers in the order of
+// the 16x16x128 fp8 MFMA: lane (c, q) takes the 32 codes k = 32 q .. + 31 of
+// its row or column, which is a lane's 32 bytes of the prepacked chunk (lhs
+// and weights agree on k, so every product is formed once).  One K block is
+// one MFMA per 16 x 16 tile, folded once (acc = fma(part, sx * sw, acc)).
+// The KS waves of a block split its K blocks and are added in wave order
+// through LDS; WR row halves share the block's weights through L1.  The row
+// scales of the block's K run are transposed into LDS once ([K block][row],
+// so a lane's four rows are one read).
+constexpr int kRowsKb = 32;  // K blocks per block at most (row-scale buffer)
+
+typedef __attribute__((ext_vector_type(8))) int i32x8_t;
+typedef i32x8_t __attribute__((aligned(16))) i32x8_a16_t;
+
+template <int MB, int NB, int WR, int KS>
+__global__ __launch_bounds__(64 * WR * KS) void dense_fp8_rows_kernel(
+    const uint8_t *__restrict__ x, const float *__restrict__ sx, int M, int K, int N,
+    const uint8_t *__restrict__ wpk, const float *__restrict__ sw, int sw_ld, int ksplit, uint16_t *__restrict__ out,
+    float *__restrict__ partial) {
+  constexpr int W = WR * KS, T = MB * NB, R = 16 * MB * WR, D = 2;
+  static_assert(128 % (16 * NB) == 0, "one weight-scale block per tile");
+  __shared__ f32x4_t s_red[KS][WR][T][64];
+  __shared__ __attribute__((aligned(16))) float s_sx[kRowsKb][R];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kw = wave % KS, wr = wave / KS;
+  const int c16 = lane & 15, q = lane >> 4;
+  const int KB = K >> 7;
+  const int kb_per = (KB + ksplit - 1) / ksplit;
+  const int kb0 = blockIdx.z * kb_per;
+  const int nkb = min(KB, kb0 + kb_per) - kb0;
+  const int lo = kb0 + nkb * kw / KS, hi = kb0 + nkb * (kw + 1) / KS;  // the wave's K blocks
+  const int nb0 = blockIdx.x * NB;
+  uint32_t aoff[MB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+    aoff[i] = (uint32_t)min(16 * (MB * wr + i) + c16, M - 1) * (uint32_t)K + 32u * q;  // rows past M repeat the last
+  const uint32_t woff = lane * 32u;
+  i32x8_t a[D][MB], b[D][NB];
+  float ws[D];
+  auto load = [&](int d, int kb) {
+    const uint8_t *const ab = x + (int64_t)kb * 128;
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const uint8_t *const wb = wpk + ((int64_t)(nb0 + j) * KB + kb) * 2048;
+      b[d][j] = *(const i32x8_a16_t *)(wb + woff);
+    }
+#pragma unroll
+    for (int i = 0; i < MB; ++i) a[d][i] = *(const i32x8_a16_t *)(ab + aoff[i]);
+    ws[d] = sw[(int64_t)kb * sw_ld + (nb0 * 16 >> 7)];
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#pragma unroll
+  for (int d = 0; d < D; ++d) load(d, min(lo + d, KB - 1));
+  // Row scales: row t / kb_pad of the block, K block t % kb_pad.
+  for (int t = tid; t < R * nkb; t += 64 * W) {
+    const int r = t / nkb, kb = t % nkb;
+    s_sx[kb][r] = sx[(int64_t)min(r, M - 1) * KB + kb0 + kb];
+  }
+  __syncthreads();
+  f32x4_t acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  auto consume = [&](int d, int kb) {
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+      const f32x4_t xs = *(const f32x4_t *)&s_sx[kb - kb0][16 * (MB * wr + i) + 4 * q];
+      f32x4_t part[NB];
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+        part[j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a[d][i], b[d][j], f32x4_t{0.f, 0.f, 0.f, 0.f}, 0,
+                                                                   0, 0, 127, 0, 127);
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][j][e] = __builtin_fmaf(part[j][e], xs[e] * ws[d], acc[i][j][e]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  int kb = lo;
+  for (; kb + 2 * D <= hi; kb += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      consume(d, kb + d);
+      load(d, kb + D + d);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < 2 * D - 1; ++t) {
+    if (kb + t < hi) {
+      consume(t % D, kb + t);
+      if (t + D < 2 * D - 1 && kb + t + D < hi) load(t % D, kb + t + D);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) s_red[kw][wr][i * NB + j][lane] = acc[i][j];
+  __syncthreads();
+  // Tile t of row half h: the waves' sums in wave order, rows 4 q .. + 3 of
+  // its 16, column c16.
+  for (int t = wave; t < WR * T; t += W) {
+    const int h = t / T, tt = t % T;
+    f32x4_t v = s_red[0][h][tt][lane];
+#pragma unroll
+    for (int w = 1; w < KS; ++w) v = v + s_red[w][h][tt][lane];
+    const int row = 16 * (MB * h + tt / NB) + 4 * q;
+    const int64_t col = (int64_t)(nb0 + tt % NB) * 16 + c16;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (row + e < M) {
+        if (partial) partial[((int64_t)blockIdx.z * M + row + e) * N + col] = v[e];
+        else out[(int64_t)(row + e) * N + col] = f32_to_bf16_bits(v[e]);
+      }
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Large M: block tiles of BM x BN = (64 WM) x (32 JN WN), each wave a
 // 64 x 32 JN output of 2 x JN MFMA 32x32 tiles (JN = 2; the 128-row W8A16
@@ -451,8 +578,6 @@ struct DenseMfmaCfg {
   static_assert(BN == 128, "one 128-column weight-scale block per tile");
   static_assert(!A8 || JN == 2, "W8A8 waves own two 32-column tiles");
 };
-
-typedef __attribute__((ext_vector_type(8))) int i32x8_t;
 
 // Per-wave step accounting of dense_fp8_mfma_kernel, compiled into the
 // library's timeline build only (-DDWTPU_TIMELINE, libdwtpu_moe_timeline.so;
@@ -931,8 +1056,35 @@ static int whole_runs(int64_t KB, int ks) {
   return (int)((KB + per - 1) / per);
 }
 
+// Rows kernel (W8A8, 17 <= M <= kRowsMax): 16-row blocks per wave and row
+// halves per block.
+constexpr int64_t kRowsMax = 96;
+static int rows_halves(int64_t M) { return M > 64 ? 2 : 1; }
+// 16-column groups per wave: four at two row blocks; more rows leave registers for two.
+constexpr int rows_groups(int mb) { return mb == 2 ? 4 : 2; }
+static int rows_blocks(int64_t M) { return (int)(((M + 15) / 16 + rows_halves(M) - 1) / rows_halves(M)); }
+
+// Measured against the 128-row MFMA tiles (K = 7168, N = 4096, reduce
+// included): M = 17 16.4 -> 11.1 us, 32 17.0 -> 11.6, 48 18.9 -> 12.8, 64
+// 19.2 -> 14.8, 65 19.4 -> 17.7; past 96 rows it loses (100 rows 20.8 ->
+// 21.6).  Above 32 rows a second round of its one-per-CU blocks loses too
+// (64 rows, K = 1024, N = 32768 16.8 -> 27.3), so the column tiles must fit
+// one; up to 32 rows it wins there as well (20 rows 15.0 -> 11.7).
+static bool rows_rule(int64_t M, int64_t N) {
+  return M <= kRowsMax && (M <= 32 || N / (16 * rows_groups(rows_blocks(M))) <= 256);
+}
+
 static dwm_dense_plan default_plan(int64_t M, int64_t K, int64_t N, bool a8) {
   const int64_t KB = K / 128;
+  if (a8 && rows_rule(M, N) && dense_mfma_ok(M, K, N, 128)) {
+    // One block per CU, while every wave keeps a K block; at most kRowsKb per block.
+    const int tn = 16 * rows_groups(rows_blocks(M));
+    const int64_t ct = N / tn, waves = 8 / rows_halves(M);
+    int64_t ks = (256 + ct - 1) / ct;
+    if (ks > KB / waves) ks = KB / waves;
+    if (ks < (KB + kRowsKb - 1) / kRowsKb) ks = (KB + kRowsKb - 1) / kRowsKb;
+    return {DWM_DENSE_ROWS, 16 * rows_blocks(M) * rows_halves(M), tn, whole_runs(KB, (int)ks), 2};
+  }
   if (dense_mfma_ok(M, K, N, 128)) {
     const int tm = (a8 && M >= 256) ? 256 : 128;
     const int64_t tiles = (N / 128) * ((M + tm - 1) / tm);
@@ -983,6 +1135,18 @@ static int check_plan(int64_t M, int64_t K, int64_t N, bool a8, const dwm_dense_
       DWM_UNSUPPORTED_IF(!ok, "dense_fp8 plan: %s %d-row MFMA tiles have no %d-stage ring", v, p.tile_m, p.stages);
       return DWM_OK;
     }
+    case DWM_DENSE_ROWS: {
+      DWM_UNSUPPORTED_IF(!a8 || M > kRowsMax || !dense_mfma_ok(M, K, N, 128),
+                         "dense_fp8 plan: the rows kernel takes W8A8, 17 <= M <= %lld and N %% 128 == 0",
+                         (long long)kRowsMax);
+      DWM_UNSUPPORTED_IF(p.tile_m != 16 * rows_blocks(M) * rows_halves(M) || p.tile_n != 16 * rows_groups(rows_blocks(M)) ||
+                             p.stages != 2,
+                         "dense_fp8 plan: the rows kernel runs %d x %d tiles with ring depth 2 at M=%lld",
+                         16 * rows_blocks(M) * rows_halves(M), 16 * rows_groups(rows_blocks(M)), (long long)M);
+      DWM_UNSUPPORTED_IF((KB + p.ksplit - 1) / p.ksplit > kRowsKb,
+                         "dense_fp8 plan: the rows kernel takes at most %d K blocks per run", kRowsKb);
+      return DWM_OK;
+    }
     case DWM_DENSE_TILED: {
       const bool ok = (p.tile_m == 16 && p.tile_n == 64) || (p.tile_m == 64 && p.tile_n == 128) ||
                       (p.tile_m == 128 && p.tile_n == 128);
@@ -1009,6 +1173,14 @@ static void launch_mfma(const void *x, const float *sx, int64_t M, int64_t K, in
   const dim3 grid((unsigned)(N / C::BN), (unsigned)((M + C::BM - 1) / C::BM), (unsigned)ks);
   hipLaunchKernelGGL((dense_fp8_mfma_kernel<C, A8, NS, A8>), grid, dim3(C::THREADS), 0, st, x, sx, M, (int)K, (int)N,
                      w, sw, sw_ld, ks, out, partial);
+}
+
+template <int MB, int WR>
+static void launch_rows(const void *x, const float *sx, int64_t M, int64_t K, int64_t N, const uint8_t *w,
+                        const float *sw, int sw_ld, int ks, uint16_t *out, float *partial, hipStream_t st) {
+  constexpr int NB = rows_groups(MB);
+  hipLaunchKernelGGL((dense_fp8_rows_kernel<MB, NB, WR, 8 / WR>), dim3((unsigned)(N / (16 * NB)), 1, (unsigned)ks),
+                     dim3(512), 0, st, (const uint8_t *)x, sx, (int)M, (int)K, (int)N, w, sw, sw_ld, ks, out, partial);
 }
 
 template <int MB, int NBW, bool A8, bool PRE = false>
@@ -1079,6 +1251,11 @@ static int run_dense(const void *x, const float *sx, int64_t M, int64_t K, int64
     else if (K <= 1024) DWM_SKINNY(8, 1, 1);
     else DWM_SKINNY(16, 2, 1);
 #undef DWM_SKINNY
+  } else if (p.kernel == DWM_DENSE_ROWS) {
+    if (p.tile_m == 32) launch_rows<2, 1>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
+    else if (p.tile_m == 48) launch_rows<3, 1>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
+    else if (p.tile_m == 64) launch_rows<4, 1>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
+    else launch_rows<3, 2>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
   } else if (p.kernel == DWM_DENSE_MFMA) {
     if constexpr (A8) {
       if (p.tile_m == 256) launch_mfma<DenseMfmaCfg<4, 2, true>, true, 3>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);

@@ -12,6 +12,8 @@ What they mean here is a launch of this library's kernels
   mode "native"    tm = tn = 16: the skinny kernel (M <= 16; its 16 waves
                    split K inside one block, so tk = K);
                    tm = 128 or 256, tn = 128: the MFMA tile kernel;
+                   tn = 64 or 32: the rows kernel (W8A8, 17 <= M <= 96; tm =
+                   M rounded up to 32 (tn = 64), 48, 64 or 96 (32));
   mode "megablox"  the general tiled kernel, tm x tn = 16 x 64, 64 x 128 or
                    128 x 128 (any N % 16 == 0);
   tk               the K depth one block covers: K / tk blocks share an
@@ -87,7 +89,7 @@ def tile_to_plan(tile, m, k, n, w8a8=False):
         raise ValueError(f"tk={tk} must be a positive multiple of 128 (the scale block)")
     kernel = _KERNEL_OF_MODE[mode]
     if kernel is None:
-        kernel = _lib.DENSE_SKINNY if (tm, tn) == (16, 16) else _lib.DENSE_MFMA
+        kernel = (_lib.DENSE_SKINNY if (tm, tn) == (16, 16) else _lib.DENSE_ROWS if tn in (32, 64) else _lib.DENSE_MFMA)
     if kernel == _lib.DENSE_SKINNY:
         if tk != k:
             raise ValueError(f"the skinny kernel covers all of K in one block: tk must be {k}")

@@ -1,6 +1,8 @@
-"""The dense FP8 launches for few rows: the skinny kernel's forms for shallow K
-(fewer waves) and wide N (four column groups per block), against the float64
-oracle under the stated bound, with the plan the library launched."""
+"""The dense FP8 launches for few rows: the W8A8 rows kernel (17 .. 96 rows)
+at the edges of its row tiles, K runs and column tiles, and the skinny
+kernel's forms for shallow K (fewer waves) and wide N (four column groups per
+block), against the float64 oracle under the stated bound, with the plan the
+library launched."""
 import numpy as np
 import pytest
 import torch
@@ -18,6 +20,36 @@ def _check(out, y64, ap, K):
     err = np.abs(y - y64)
     assert np.all(np.isfinite(y))
     assert np.all(err <= odf.error_bound(y64, ap, K)), ogmm.error_stats(y, y64)
+
+
+@pytest.mark.parametrize("M,K,N,plan", [
+    (17, 128, 128, (4, 32, 64, 1, 2)),     # one K block: seven of eight waves have none
+    (32, 4224, 256, (4, 32, 64, 4, 2)),    # 33 K blocks: past the 32 of one run
+    (33, 1152, 384, (4, 48, 32, 1, 2)),
+    (48, 2048, 128, (4, 48, 32, 2, 2)),
+    (49, 3072, 512, (4, 64, 32, 3, 2)),
+    (64, 1408, 256, (4, 64, 32, 1, 2)),
+    (65, 1024, 128, (4, 96, 32, 2, 2)),
+    (95, 2176, 640, (4, 96, 32, 4, 2)),    # 17 K blocks in runs of 5, 5, 5, 2
+    (96, 640, 8192, (4, 96, 32, 1, 2)),    # 256 column tiles
+    (96, 640, 8320, (2, 128, 128, 3, 4)),  # 260: the MFMA tiles
+    (97, 1024, 256, (2, 128, 128, 8, 4)),
+    (32, 256, 16640, (4, 32, 64, 1, 2)),   # two rounds of column tiles
+])
+def test_w8a8_rows_plans_against_oracle(dev, M, K, N, plan):
+    from dw_tpu_amd.dense_fp8 import last_plan, matmul_w8a8
+    from dw_tpu_amd.dense_fp8_tiles import plan_to_tile
+    from dw_tpu_amd.workloads import make_dense_workload
+    wl = make_dense_workload(M, K, N, seed=M + K)
+    args = [torch.from_numpy(v).to(dev) for v in (wl.xq, wl.sx, wl.wq, wl.sw)]
+    out = matmul_w8a8(*args)
+    torch.cuda.synchronize()
+    p = last_plan()
+    assert p.astuple() == plan
+    y64 = odf.matmul_w8a8(wl.xq, wl.sx, wl.wq, wl.sw, out_dtype="float64")
+    _check(out, y64, odf.abs_product_w8a8(wl.xq, wl.sx, wl.wq, wl.sw), K)
+    again = matmul_w8a8(*args, tile=plan_to_tile(p, K))
+    assert torch.equal(again.view(torch.int16), out.view(torch.int16)) and last_plan().astuple() == plan
 
 
 @pytest.mark.parametrize("a8", [False, True])

@@ -13,7 +13,7 @@
 //   (exact: 3 mantissa bits, exponents inside bf16's range) for bf16 MFMA
 //   32x32x16; W8A8 runs the fp8 MFMA 32x32x64 on the codes.
 // - M <= 16: dense_fp8_skinny_kernel (see below).
-// - W8A8, 17 <= M <= 96, N % 128 == 0: dense_fp8_rows_kernel (see below).
+// - 17 <= M <= 32 (W8A8: 96), N % 128 == 0: dense_fp8_rows_kernel (see below).
 // - Other shapes: dense_fp8_kernel, bf16 MFMA 16x16x32 on decoded codes.
 // Every product is the exact fp8 (or bf16 x fp8) product; the 128-K partial
 // is an f32 sum of them.
@@ -398,36 +398,38 @@ __global__ __launch_bounds__(64 * KS) void dense_fp8_skinny_kernel(
   }
 }
 
-// W8A8, 17 .. 96 rows: dense_fp8_rows_kernel.  What bounds it: the weight
-// stream and latency -- at 64 rows, K = 7168, N = 4096 the weights take 5 us
-// of HBM time and the fp8 MFMAs under 2 us, but the 128-row MFMA tiles took
-// 17 us: half of their rows were padding, every step waited at a barrier for
-// LDS copies of operands that no second wave needs, and the eight K runs of a
-// tile wrote 17 MB of partials.
+// 17 .. 96 rows (W8A16: 32): dense_fp8_rows_kernel.  What bounds it: the
+// weight stream and latency -- at 64 rows, K = 7168, N = 4096 the weights take
+// 5 us of HBM time and the MFMAs under 3 us, but the 128-row MFMA tiles took
+// 14-17 us: half of their rows or more were padding, every step waited at a
+// barrier for LDS copies of operands that no second wave needs, and the eight
+// K runs of a tile wrote 17 MB of partials.
 // Here nothing is staged: a wave owns 16 MB rows x 16 NB columns and a run of
-// K blocks, and loads its operands straight into registers in the order of
-// the 16x16x128 fp8 MFMA: lane (c, q) takes the 32 codes k = 32 q .. + 31 of
-// its row or column, which is a lane's 32 bytes of the prepacked chunk (lhs
-// and weights agree on k, so every product is formed once).  One K block is
-// one MFMA per 16 x 16 tile, folded once (acc = fma(part, sx * sw, acc)).
-// The KS waves of a block split its K blocks and are added in wave order
-// through LDS; WR row halves share the block's weights through L1.  The row
-// scales of the block's K run are transposed into LDS once ([K block][row],
-// so a lane's four rows are one read).
-constexpr int kRowsKb = 32;  // K blocks per block at most (row-scale buffer)
+// K blocks, and loads its operands straight into registers in MFMA order:
+// lane (c, q) takes k = 32 q .. + 31 of its row or column, which is a lane's
+// 32 bytes of the prepacked chunk (lhs and weights agree on k, so every
+// product is formed once).  W8A8 runs one 16x16x128 fp8 MFMA per 16 x 16 tile
+// and K block, W8A16 four 16x16x32 bf16 MFMAs on decoded codes; the K block is
+// folded once (acc = fma(part, scale, acc)).  The KS waves of a block split
+// its K blocks and are added in wave order through LDS; WR row halves share
+// the block's weights through L1.  W8A8's row scales of the block's K run are
+// transposed into LDS once ([K block][row], so a lane's four rows are one
+// read).
+constexpr int kRowsKb = 32;  // K blocks per block at most (W8A8's row-scale buffer)
 
 typedef __attribute__((ext_vector_type(8))) int i32x8_t;
 typedef i32x8_t __attribute__((aligned(16))) i32x8_a16_t;
 
-template <int MB, int NB, int WR, int KS>
+template <int MB, int NB, int WR, int KS, bool A8>
 __global__ __launch_bounds__(64 * WR * KS) void dense_fp8_rows_kernel(
     const uint8_t *__restrict__ x, const float *__restrict__ sx, int M, int K, int N,
     const uint8_t *__restrict__ wpk, const float *__restrict__ sw, int sw_ld, int ksplit, uint16_t *__restrict__ out,
     float *__restrict__ partial) {
   constexpr int W = WR * KS, T = MB * NB, R = 16 * MB * WR, D = 2;
+  constexpr int XB = A8 ? 1 : 2, XV = A8 ? 1 : 2;  // bytes per lhs value; 32-byte lhs loads per K block
   static_assert(128 % (16 * NB) == 0, "one weight-scale block per tile");
   __shared__ f32x4_t s_red[KS][WR][T][64];
-  __shared__ __attribute__((aligned(16))) float s_sx[kRowsKb][R];
+  __shared__ __attribute__((aligned(16))) float s_sx[A8 ? kRowsKb : 1][R];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kw = wave % KS, wr = wave / KS;
   const int c16 = lane & 15, q = lane >> 4;
@@ -439,50 +441,89 @@ __global__ __launch_bounds__(64 * WR * KS) void dense_fp8_rows_kernel(
   const int nb0 = blockIdx.x * NB;
   uint32_t aoff[MB];
 #pragma unroll
-  for (int i = 0; i < MB; ++i)
-    aoff[i] = (uint32_t)min(16 * (MB * wr + i) + c16, M - 1) * (uint32_t)K + 32u * q;  // rows past M repeat the last
+  for (int i = 0; i < MB; ++i)  // rows past M repeat the last
+    aoff[i] = (uint32_t)min(16 * (MB * wr + i) + c16, M - 1) * (uint32_t)K * XB + 32u * XB * q;
   const uint32_t woff = lane * 32u;
-  i32x8_t a[D][MB], b[D][NB];
-  float ws[D];
+  i32x8_t a[D][MB][XV], b[D][NB];
+  float ws[D][A8 ? 1 : NB];
   auto load = [&](int d, int kb) {
-    const uint8_t *const ab = x + (int64_t)kb * 128;
+    const uint8_t *const ab = x + (int64_t)kb * 128 * XB;
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
       const uint8_t *const wb = wpk + ((int64_t)(nb0 + j) * KB + kb) * 2048;
       b[d][j] = *(const i32x8_a16_t *)(wb + woff);
     }
 #pragma unroll
-    for (int i = 0; i < MB; ++i) a[d][i] = *(const i32x8_a16_t *)(ab + aoff[i]);
-    ws[d] = sw[(int64_t)kb * sw_ld + (nb0 * 16 >> 7)];
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int p = 0; p < XV; ++p) a[d][i][p] = *(const i32x8_a16_t *)(ab + 32 * p + aoff[i]);
+    if constexpr (A8) {
+      ws[d][0] = sw[(int64_t)kb * sw_ld + (nb0 * 16 >> 7)];
+    } else {
+#pragma unroll
+      for (int j = 0; j < NB; ++j) ws[d][j] = sw[(int64_t)kb * sw_ld + (nb0 + j) * 16 + c16];
+    }
     __builtin_amdgcn_sched_barrier(0);
   };
 #pragma unroll
   for (int d = 0; d < D; ++d) load(d, min(lo + d, KB - 1));
-  // Row scales: row t / kb_pad of the block, K block t % kb_pad.
-  for (int t = tid; t < R * nkb; t += 64 * W) {
-    const int r = t / nkb, kb = t % nkb;
-    s_sx[kb][r] = sx[(int64_t)min(r, M - 1) * KB + kb0 + kb];
+  if constexpr (A8) {
+    // Row scales: row t / nkb of the block, K block t % nkb.
+    for (int t = tid; t < R * nkb; t += 64 * W) {
+      const int r = t / nkb, kb = t % nkb;
+      s_sx[kb][r] = sx[(int64_t)min(r, M - 1) * KB + kb0 + kb];
+    }
+    __syncthreads();
   }
-  __syncthreads();
   f32x4_t acc[MB][NB];
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
     for (int j = 0; j < NB; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   auto consume = [&](int d, int kb) {
+    if constexpr (A8) {
 #pragma unroll
-    for (int i = 0; i < MB; ++i) {
-      const f32x4_t xs = *(const f32x4_t *)&s_sx[kb - kb0][16 * (MB * wr + i) + 4 * q];
-      f32x4_t part[NB];
+      for (int i = 0; i < MB; ++i) {
+        const f32x4_t xs = *(const f32x4_t *)&s_sx[kb - kb0][16 * (MB * wr + i) + 4 * q];
+        f32x4_t part[NB];
 #pragma unroll
-      for (int j = 0; j < NB; ++j)
-        part[j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a[d][i], b[d][j], f32x4_t{0.f, 0.f, 0.f, 0.f}, 0,
-                                                                   0, 0, 127, 0, 127);
+        for (int j = 0; j < NB; ++j)
+          part[j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a[d][i][0], b[d][j], f32x4_t{0.f, 0.f, 0.f, 0.f},
+                                                                     0, 0, 0, 127, 0, 127);
 #pragma unroll
-      for (int j = 0; j < NB; ++j)
+        for (int j = 0; j < NB; ++j)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[i][j][e] = __builtin_fmaf(part[j][e], xs[e] * ws[d], acc[i][j][e]);
-      __builtin_amdgcn_sched_barrier(0);
+          for (int e = 0; e < 4; ++e) acc[i][j][e] = __builtin_fmaf(part[j][e], xs[e] * ws[d][0], acc[i][j][e]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      // Column group by column group: its codes are decoded once, for every
+      // row block; four 16x16x32 MFMAs per row block, then the fold.
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        f32x4_t part[MB];
+#pragma unroll
+        for (int i = 0; i < MB; ++i) part[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {  // k = 32 q + 8 s .. + 7
+          const uint32_t w0 = (uint32_t)b[d][j][2 * s], w1 = (uint32_t)b[d][j][2 * s + 1];
+          const u32x4_t bf = {cvt_fp8x2_bf16<false>(w0), cvt_fp8x2_bf16<true>(w0), cvt_fp8x2_bf16<false>(w1),
+                              cvt_fp8x2_bf16<true>(w1)};
+#pragma unroll
+          for (int i = 0; i < MB; ++i) {
+            const i32x8_t &v = a[d][i][XV > 1 ? s >> 1 : 0];
+            const u32x4_t af = {(uint32_t)v[4 * (s & 1)], (uint32_t)v[4 * (s & 1) + 1], (uint32_t)v[4 * (s & 1) + 2],
+                                (uint32_t)v[4 * (s & 1) + 3]};
+            part[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, af),
+                                                              __builtin_bit_cast(bf16x8_t, bf), part[i], 0, 0, 0);
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[i][j][e] = __builtin_fmaf(part[i][e], ws[d][A8 ? 0 : j], acc[i][j][e]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
   };
   int kb = lo;
@@ -1039,8 +1080,9 @@ static dwm_dense_plan tiled_default(int64_t M, int64_t K, int64_t N) {
   return p;
 }
 
-// MFMA path (M > 16, N % 128 == 0): W8A16 128x128 tiles (8 waves, two or
-// three 25 KB stages: two blocks per CU), 256x128 tiles (8 waves) when those
+// MFMA path (M > 16, N % 128 == 0): W8A16 64x128 tiles up to 64 rows (4
+// waves), 128x128 tiles (8 waves, two or three 25 KB stages: two blocks per
+// CU), 256x128 tiles (8 waves) when those
 // alone fill the grid; W8A8 256x128 tiles (8 waves, three 50 KB stages of
 // one K block each, fragments read one substep ahead) from M >= 256, 128x128
 // below (four 33 KB stages).  K is split over blocks until the grid covers
@@ -1056,7 +1098,7 @@ static int whole_runs(int64_t KB, int ks) {
   return (int)((KB + per - 1) / per);
 }
 
-// Rows kernel (W8A8, 17 <= M <= kRowsMax): 16-row blocks per wave and row
+// Rows kernel (17 <= M <= 32, W8A8 <= kRowsMax): 16-row blocks per wave and row
 // halves per block.
 constexpr int64_t kRowsMax = 96;
 static int rows_halves(int64_t M) { return M > 64 ? 2 : 1; }
@@ -1065,18 +1107,22 @@ constexpr int rows_groups(int mb) { return mb == 2 ? 4 : 2; }
 static int rows_blocks(int64_t M) { return (int)(((M + 15) / 16 + rows_halves(M) - 1) / rows_halves(M)); }
 
 // Measured against the 128-row MFMA tiles (K = 7168, N = 4096, reduce
-// included): M = 17 16.4 -> 11.1 us, 32 17.0 -> 11.6, 48 18.9 -> 12.8, 64
+// included), W8A8: M = 17 16.4 -> 11.1 us, 32 17.0 -> 11.6, 48 18.9 -> 12.8, 64
 // 19.2 -> 14.8, 65 19.4 -> 17.7; past 96 rows it loses (100 rows 20.8 ->
 // 21.6).  Above 32 rows a second round of its one-per-CU blocks loses too
 // (64 rows, K = 1024, N = 32768 16.8 -> 27.3), so the column tiles must fit
 // one; up to 32 rows it wins there as well (20 rows 15.0 -> 11.7).
-static bool rows_rule(int64_t M, int64_t N) {
-  return M <= kRowsMax && (M <= 32 || N / (16 * rows_groups(rows_blocks(M))) <= 256);
+// W8A16 takes it up to 32 rows (17 rows 14.3 -> 10.9, 32 14.9 -> 11.8; K =
+// 1024, N = 32768 20.8 -> 14.6): its lhs fragments are 64 bytes a lane, half
+// lines of every row, and from 48 rows on they cost more than the tiles' LDS
+// copies (48 rows 15.9 -> 16.4, 64 16.7 -> 19.7).
+static bool rows_rule(int64_t M, int64_t N, bool a8) {
+  return M <= 32 || (a8 && M <= kRowsMax && N / (16 * rows_groups(rows_blocks(M))) <= 256);
 }
 
 static dwm_dense_plan default_plan(int64_t M, int64_t K, int64_t N, bool a8) {
   const int64_t KB = K / 128;
-  if (a8 && rows_rule(M, N) && dense_mfma_ok(M, K, N, 128)) {
+  if (rows_rule(M, N, a8) && dense_mfma_ok(M, K, N, 128)) {
     // One block per CU, while every wave keeps a K block; at most kRowsKb per block.
     const int tn = 16 * rows_groups(rows_blocks(M));
     const int64_t ct = N / tn, waves = 8 / rows_halves(M);
@@ -1086,12 +1132,16 @@ static dwm_dense_plan default_plan(int64_t M, int64_t K, int64_t N, bool a8) {
     return {DWM_DENSE_ROWS, 16 * rows_blocks(M) * rows_halves(M), tn, whole_runs(KB, (int)ks), 2};
   }
   if (dense_mfma_ok(M, K, N, 128)) {
-    const int tm = (a8 && M >= 256) ? 256 : 128;
+    const int tm = (a8 && M >= 256) ? 256 : (!a8 && M <= 64) ? 64 : 128;
     const int64_t tiles = (N / 128) * ((M + tm - 1) / tm);
     int ks = 1;
     while (tiles * ks < 256 && ks * 2 <= KB && ks < 16) ks *= 2;
     ks = whole_runs(KB, ks);
     if (a8) return {DWM_DENSE_MFMA, tm, 128, ks, tm == 256 ? 3 : 4};
+    // 33 .. 64 rows: half the MFMAs, lhs copies and barrier partners of a
+    // 128-row tile (K = 7168, N = 4096: 48 rows 15.3 -> 13.9 us, 64 16.1 ->
+    // 14.4; K = 1024, N = 32768 22.3 -> 12.0; twice the K runs lost, 17.7).
+    if (tm == 64) return {DWM_DENSE_MFMA, 64, 128, ks, 4};
     // Enough rows for 256 x 128 tiles to fill the grid: half the weight
     // re-reads of 128-row tiles (8 waves, one block per CU).
     if (ks == 1 && (N / 128) * ((M + 255) / 256) >= 256) return {DWM_DENSE_MFMA, 256, 128, 1, 2};
@@ -1125,19 +1175,21 @@ static int check_plan(int64_t M, int64_t K, int64_t N, bool a8, const dwm_dense_
                      p.ksplit, (long long)KB);
   switch (p.kernel) {
     case DWM_DENSE_MFMA: {
-      DWM_UNSUPPORTED_IF(p.tile_n != 128 || (p.tile_m != 128 && p.tile_m != 256),
-                         "dense_fp8 plan: MFMA tiles are 128 x 128 or 256 x 128 (got %d x %d)", p.tile_m, p.tile_n);
+      DWM_UNSUPPORTED_IF(p.tile_n != 128 || (p.tile_m != 128 && p.tile_m != 256 && (a8 || p.tile_m != 64)),
+                         "dense_fp8 plan: MFMA tiles are 128 x 128, 256 x 128 or (W8A16) 64 x 128 (got %d x %d)", p.tile_m, p.tile_n);
       DWM_UNSUPPORTED_IF(!dense_mfma_ok(M, K, N, p.tile_m),
                          "dense_fp8 plan: the MFMA kernel needs M > 16, N %% 128 == 0 and 32-bit operand offsets");
       // Ring depths that fit 160 KB of LDS (W8A8's prefetching loop needs 3).
       const bool ok = a8 ? (p.tile_m == 128 ? (p.stages == 3 || p.stages == 4) : p.stages == 3)
-                         : (p.tile_m == 128 ? (p.stages >= 2 && p.stages <= 4) : (p.stages == 2 || p.stages == 3));
+                         : (p.tile_m == 64    ? p.stages == 4
+                            : p.tile_m == 128 ? (p.stages >= 2 && p.stages <= 4)
+                                              : (p.stages == 2 || p.stages == 3));
       DWM_UNSUPPORTED_IF(!ok, "dense_fp8 plan: %s %d-row MFMA tiles have no %d-stage ring", v, p.tile_m, p.stages);
       return DWM_OK;
     }
     case DWM_DENSE_ROWS: {
-      DWM_UNSUPPORTED_IF(!a8 || M > kRowsMax || !dense_mfma_ok(M, K, N, 128),
-                         "dense_fp8 plan: the rows kernel takes W8A8, 17 <= M <= %lld and N %% 128 == 0",
+      DWM_UNSUPPORTED_IF(M > (a8 ? kRowsMax : 32) || !dense_mfma_ok(M, K, N, 128),
+                         "dense_fp8 plan: the rows kernel takes 17 <= M <= 32 (W8A8: %lld) and N %% 128 == 0",
                          (long long)kRowsMax);
       DWM_UNSUPPORTED_IF(p.tile_m != 16 * rows_blocks(M) * rows_halves(M) || p.tile_n != 16 * rows_groups(rows_blocks(M)) ||
                              p.stages != 2,
@@ -1175,11 +1227,11 @@ static void launch_mfma(const void *x, const float *sx, int64_t M, int64_t K, in
                      w, sw, sw_ld, ks, out, partial);
 }
 
-template <int MB, int WR>
+template <int MB, int WR, bool A8>
 static void launch_rows(const void *x, const float *sx, int64_t M, int64_t K, int64_t N, const uint8_t *w,
                         const float *sw, int sw_ld, int ks, uint16_t *out, float *partial, hipStream_t st) {
   constexpr int NB = rows_groups(MB);
-  hipLaunchKernelGGL((dense_fp8_rows_kernel<MB, NB, WR, 8 / WR>), dim3((unsigned)(N / (16 * NB)), 1, (unsigned)ks),
+  hipLaunchKernelGGL((dense_fp8_rows_kernel<MB, NB, WR, 8 / WR, A8>), dim3((unsigned)(N / (16 * NB)), 1, (unsigned)ks),
                      dim3(512), 0, st, (const uint8_t *)x, sx, (int)M, (int)K, (int)N, w, sw, sw_ld, ks, out, partial);
 }
 
@@ -1252,17 +1304,20 @@ static int run_dense(const void *x, const float *sx, int64_t M, int64_t K, int64
     else DWM_SKINNY(16, 2, 1);
 #undef DWM_SKINNY
   } else if (p.kernel == DWM_DENSE_ROWS) {
-    if (p.tile_m == 32) launch_rows<2, 1>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
-    else if (p.tile_m == 48) launch_rows<3, 1>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
-    else if (p.tile_m == 64) launch_rows<4, 1>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
-    else launch_rows<3, 2>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
+    if (p.tile_m == 32) launch_rows<2, 1, A8>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
+    if constexpr (A8) {
+      if (p.tile_m == 48) launch_rows<3, 1, true>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
+      else if (p.tile_m == 64) launch_rows<4, 1, true>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
+      else if (p.tile_m == 96) launch_rows<3, 2, true>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
+    }
   } else if (p.kernel == DWM_DENSE_MFMA) {
     if constexpr (A8) {
       if (p.tile_m == 256) launch_mfma<DenseMfmaCfg<4, 2, true>, true, 3>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
       else if (p.stages == 3) launch_mfma<DenseMfmaCfg<2, 2, true>, true, 3>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
       else launch_mfma<DenseMfmaCfg<2, 2, true>, true, 4>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
     } else {
-      if (p.tile_m == 256 && p.stages == 2) launch_mfma<DenseMfmaCfg<4, 2, false>, false, 2>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
+      if (p.tile_m == 64) launch_mfma<DenseMfmaCfg<1, 4, false, 1>, false, 4>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
+      else if (p.tile_m == 256 && p.stages == 2) launch_mfma<DenseMfmaCfg<4, 2, false>, false, 2>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
       else if (p.tile_m == 256) launch_mfma<DenseMfmaCfg<4, 2, false>, false, 3>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
       else if (p.stages == 2) launch_mfma<DenseMfmaCfg<2, 4, false, 1>, false, 2>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
       else if (p.stages == 3) launch_mfma<DenseMfmaCfg<2, 4, false, 1>, false, 3>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);

@@ -11,9 +11,10 @@ What they mean here is a launch of this library's kernels
 
   mode "native"    tm = tn = 16: the skinny kernel (M <= 16; its 16 waves
                    split K inside one block, so tk = K);
-                   tm = 128 or 256, tn = 128: the MFMA tile kernel;
-                   tn = 64 or 32: the rows kernel (W8A8, 17 <= M <= 96; tm =
-                   M rounded up to 32 (tn = 64), 48, 64 or 96 (32));
+                   tm = 64 (W8A16), 128 or 256, tn = 128: the MFMA tile
+                   kernel;
+                   tn = 64 or 32: the rows kernel (17 <= M <= 32, W8A8 <= 96; tm
+                   = M rounded up to 32 (tn = 64), 48, 64 or 96 (32));
   mode "megablox"  the general tiled kernel, tm x tn = 16 x 64, 64 x 128 or
                    128 x 128 (any N % 16 == 0);
   tk               the K depth one block covers: K / tk blocks share an
@@ -62,7 +63,7 @@ def _usual_stages(kernel, tile_m, w8a8):
     if kernel == _lib.DENSE_MFMA:
         if w8a8:
             return 4 if tile_m == 128 else 3
-        return 3 if tile_m == 128 else 2
+        return {64: 4, 128: 3}.get(tile_m, 2)
     return 2
 
 

@@ -403,14 +403,14 @@ enum dwm_dense_kernel {
   /* M <= 16: one block per 16 columns; its 16 waves split K (ksplit = 16)
    * and add their f32 partial sums in wave order; register ring depth 2. */
   DWM_DENSE_SKINNY = 1,
-  /* tile_m x 128 tiles (tile_m 128 or 256), 32x32 MFMA (bf16 for W8A16, fp8
+  /* tile_m x 128 tiles (tile_m 128 or 256; 64 for W8A16), 32x32 MFMA (bf16 for W8A16, fp8
    * for W8A8) fed by an LDS ring of `stages` K steps.  Needs M > 16 and
    * N % 128 == 0. */
   DWM_DENSE_MFMA = 2,
   /* General tiles for any N % 16 == 0: 16 x 64, 64 x 128 or 128 x 128,
    * 16x16x32 bf16 MFMA, double-buffered LDS (stages = 2). */
   DWM_DENSE_TILED = 3,
-  /* W8A8, 17 <= M <= 96, N % 128 == 0: M rounded up to 32 rows x 64
+  /* 17 <= M <= 32 (W8A8: 96), N % 128 == 0: M rounded up to 32 rows x 64
    * columns, or 48, 64 or 96 rows x 32 columns per block, operands
    * straight from memory to registers (ring depth 2), at most 32 K blocks per
    * K run. */

@@ -1,5 +1,5 @@
-"""The dense FP8 launches for few rows: the W8A8 rows kernel (17 .. 96 rows)
-at the edges of its row tiles, K runs and column tiles, and the skinny
+"""The dense FP8 launches for few rows: the rows kernel (17 .. 32 rows, W8A8 .. 96)
+and W8A16's 64-row MFMA tiles at the edges of its row tiles, K runs and column tiles, and the skinny
 kernel's forms for shallow K (fewer waves) and wide N (four column groups per
 block), against the float64 oracle under the stated bound, with the plan the
 library launched."""
@@ -49,6 +49,36 @@ def test_w8a8_rows_plans_against_oracle(dev, M, K, N, plan):
     y64 = odf.matmul_w8a8(wl.xq, wl.sx, wl.wq, wl.sw, out_dtype="float64")
     _check(out, y64, odf.abs_product_w8a8(wl.xq, wl.sx, wl.wq, wl.sw), K)
     again = matmul_w8a8(*args, tile=plan_to_tile(p, K))
+    assert torch.equal(again.view(torch.int16), out.view(torch.int16)) and last_plan().astuple() == plan
+
+
+@pytest.mark.parametrize("M,K,N,plan", [
+    (17, 128, 128, (4, 32, 64, 1, 2)),
+    (32, 4224, 256, (4, 32, 64, 4, 2)),
+    (31, 1152, 384, (4, 32, 64, 1, 2)),
+    (24, 2176, 128, (4, 32, 64, 2, 2)),
+    (32, 256, 16640, (4, 32, 64, 1, 2)),
+    (33, 1024, 256, (2, 64, 128, 8, 4)),   # past 32 rows: 64-row MFMA tiles
+    (64, 1152, 128, (2, 64, 128, 5, 4)),   # runs of 2, 2, 2, 2, 1 K blocks: two steps in a four-stage ring
+    (48, 384, 33024, (2, 64, 128, 1, 4)),
+    (65, 1024, 256, (2, 128, 128, 8, 3)),
+])
+def test_w8a16_rows_plans_against_oracle(dev, M, K, N, plan):
+    from dw_tpu_amd.dense_fp8 import last_plan, matmul, prepack_fp8, try_dense_fp8
+    from dw_tpu_amd.dense_fp8_tiles import plan_to_tile
+    from dw_tpu_amd.workloads import make_dense_workload
+    wl = make_dense_workload(M, K, N, seed=M + K + 2)
+    x, pw = bf16_tensor(wl.x_bits, dev), prepack_fp8(torch.from_numpy(wl.wq).to(dev))
+    s = torch.from_numpy(wl.s_w8a16).to(dev)
+    out = try_dense_fp8(x, pw, s)
+    torch.cuda.synchronize()
+    p = last_plan()
+    assert p.astuple() == plan
+    xf = bf16_to_f32(wl.x_bits)
+    _check(out, odf.matmul_w8a16(xf, wl.wq, wl.s_w8a16, out_dtype="float64"),
+           odf.abs_product_w8a16(xf, wl.wq, wl.s_w8a16), K)
+    t = plan_to_tile(p, K)
+    again = matmul(x, pw, s, mode=t.mode, tm=t.tm, tk=t.tk, tn=t.tn, stages=t.stages)
     assert torch.equal(again.view(torch.int16), out.view(torch.int16)) and last_plan().astuple() == plan
 
 

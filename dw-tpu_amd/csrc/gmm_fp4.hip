@@ -711,13 +711,14 @@ static int balanced_tiles() {
 // against the tiles below (both with streaming weight loads), us:
 //   32 experts, K = 7168, N = 4096: 1 token 49 -> 23; 4 rows an expert 81 -> 79, 10 rows 82 -> 91;
 //   256 experts, K = N = 4096: 3 rows an expert 398 -> 339, 7 rows 414 -> 386, 12 rows 412 -> 446;
+//   e4m3 lhs, 32 experts, K = 7168, N = 4096: half a row an expert 57 -> 40, 4 rows 83 -> 81, 10 rows 85 -> 92;
 // so it is taken up to 6 rows per local expert; and, while an expert's rows
 // make one tile, also where even 256-column tiles would leave half of the CUs
-// idle (8 experts of 50 rows, K = 3072, N = 2560: 31 -> 26; K = 1024,
-// N = 640: 16 -> 8).
-static bool stream_rule(int64_t M, int64_t N, int64_t E_local, int ncu) {
+// idle (8 experts of 50 rows, K = 3072, N = 2560: 31 -> 26, e4m3 lhs 34 -> 24;
+// K = 1024, N = 640: 16 -> 8, 17 -> 10).
+bool gmm_streams(int64_t M, int64_t N, int64_t E_local) {
   if (M <= 6 * E_local) return true;
-  return M <= 64 * E_local && (M / 96 + E_local) * ((N + 255) / 256) <= ncu / 2;
+  return M <= 64 * E_local && (M / 96 + E_local) * ((N + 255) / 256) <= device_cu_count() / 2;
 }
 
 // The bf16 grouped matmul (arguments checked by the caller).
@@ -733,7 +734,7 @@ int launch_gmm_bf16(const uint16_t *lhs, const int32_t *row_idx, int64_t lhs_row
   // local and full) leave CUs idle; larger launches never split, and run the
   // kernel without the narrow producers.
   const int ncu = device_cu_count();
-  if (stream_rule(M, N, E_local, ncu))
+  if (gmm_streams(M, N, E_local))
     return launch_gmm_stream(lhs, row_idx, lhs_rows, M, K, weight, scale, group_sizes, num_groups, group_offset,
                              E_local, N, out, out_f32, gated, ep, st);
   const bool narrow = ((M + 95) / 96) * ((N + 511) / 512) < ncu;

@@ -818,6 +818,9 @@ int launch_gmm_mx(const uint8_t *lhs, const uint8_t *lhs_scale, const int32_t *r
                   int64_t K, const uint8_t *weight, const uint8_t *scale, const int32_t *group_sizes, int num_groups,
                   const int32_t *group_offset, int64_t E_local, int64_t N, void *out, int out_f32, bool gated,
                   const GmmEpilogue &ep, hipStream_t st, bool lhs_fp4) {
+  if (gmm_streams(M, N, E_local))
+    return launch_gmm_mx_stream(lhs, lhs_scale, row_idx, lhs_rows, M, K, weight, scale, group_sizes, num_groups,
+                                group_offset, E_local, N, out, out_f32, gated, ep, st, lhs_fp4);
 #define DWM_MX_FORM(ACT, AF4)                                                                                     \
   launch_mx_form<ACT, AF4>(lhs, lhs_scale, row_idx, lhs_rows, M, K, weight, scale, group_sizes, num_groups,       \
                            group_offset, E_local, N, out, out_f32, ep, st)

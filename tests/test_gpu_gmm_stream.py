@@ -89,6 +89,46 @@ def test_stream_kernel_against_oracle_and_tiles(dev, rng, E, K, N, pattern, wind
                                           "float32" if form == "f32" else "bfloat16")), ogmm.error_stats(got, y64)
 
 
+@pytest.mark.parametrize("E,K,N,pattern,window,act,form", CASES)
+@pytest.mark.parametrize("fmt", ["e4m3", "e2m1"])
+def test_mx_stream_kernel_equals_tiles(dev, rng, E, K, N, pattern, window, act, form, fmt):
+    """The MX form gives the bits of the MX tiles (both K step depths: K below
+    and from 4096 on) for every group and epilogue form above."""
+    from dw_tpu_amd import MxLhs, fp4_weight_to_codes, gmm_v2, mx_quantize
+    if E == 4:
+        K = 4224
+    sizes = _sizes(E, pattern)
+    go, e_local = window if window else (0, E)
+    M = int(sizes.sum())
+    assert 0 < M <= 6 * e_local
+    pw = fp4_weight_to_codes(torch.from_numpy(rng.integers(0, 256, (e_local, K, N // 2), dtype=np.uint8)).to(dev),
+                             torch.from_numpy(rng.integers(123, 130, (e_local, K // 32, 1, N), dtype=np.uint8)).to(dev),
+                             gate_up=act)
+    x = mx_quantize(bf16_tensor(f32_to_bf16_bits(rng.standard_normal((M, K)).astype(np.float32)), dev), fmt)
+    bias = torch.from_numpy(rng.standard_normal((e_local, N)).astype(np.float32)).to(dev) if form == "bias" else None
+    kw = dict(rhs_bias=bias, group_offset=go if window else None,
+              preferred_element_type=torch.float32 if form == "f32" else None,
+              fuse_act="silu_and_mul_with_clamp" if act else None)
+    if form == "gather":
+        p = torch.from_numpy(rng.permutation(M).astype(np.int32)).to(dev)
+        codes, scales = torch.empty_like(x.codes), torch.empty_like(x.scales)
+        codes[p.long()], scales[p.long()] = x.codes, x.scales
+        y = gmm_v2(MxLhs(codes, scales, fmt), pw, torch.from_numpy(sizes).to(dev), lhs_row_indices=p, **kw)
+    else:
+        y = gmm_v2(x, pw, torch.from_numpy(sizes).to(dev), **kw)
+    big = sizes + 80
+    assert big.sum() > 64 * e_local
+    starts = np.concatenate([[0], np.cumsum(big)[:-1]])
+    at = torch.from_numpy(np.concatenate([s + np.arange(n) for s, n in zip(starts, sizes)]).astype(np.int64)).to(dev)
+    codes = torch.zeros((int(big.sum()), x.codes.shape[1]), dtype=torch.uint8, device=dev)
+    scales = torch.full((int(big.sum()), x.scales.shape[1]), 127, dtype=torch.uint8, device=dev)
+    codes[at], scales[at] = x.codes, x.scales
+    yb = gmm_v2(MxLhs(codes, scales, fmt), pw, torch.from_numpy(big).to(dev), **kw)[at]
+    torch.cuda.synchronize()
+    v = torch.int32 if form == "f32" else torch.int16
+    assert torch.equal(y.view(v), yb.view(v)) and bool((y != 0).any())
+
+
 def test_stream_kernel_skips_rows_past_m(dev, rng):
     """Device group sizes whose sum passes M: no row past M is read or
     written (lhs and out are padded), and rows below M are those of sizes cut

@@ -518,6 +518,32 @@ __global__ __launch_bounds__(256) void combine_bf16_kernel(const uint16_t *__res
 // still cached lose (57 MB 40.3 -> 41.9, 49 MB 37.8 -> 38.9).
 constexpr int64_t kCombineStreamBytes = 128ll << 20;
 
+// Copies up to four buffers in one launch (block row y: buffer y): a graph's
+// inputs are a few KB at decode, where a launch per buffer costs more than
+// the bytes.
+struct CopyBuffers {
+  const void *src[4];
+  void *dst[4];
+  int64_t bytes[4];
+};
+
+template <typename V>
+__device__ __forceinline__ void copy_run(const void *src, void *dst, int64_t n) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+    ((V *)dst)[i] = ((const V *)src)[i];
+}
+
+__global__ __launch_bounds__(256) void copy_buffers_kernel(CopyBuffers b) {
+  const int y = blockIdx.y;
+  const void *const src = b.src[y];
+  void *const dst = b.dst[y];
+  const int64_t n = b.bytes[y];
+  const uintptr_t al = (uintptr_t)src | (uintptr_t)dst | (uintptr_t)n;
+  if (al % 16 == 0) copy_run<u32x4_t>(src, dst, n / 16);
+  else if (al % 4 == 0) copy_run<uint32_t>(src, dst, n / 4);
+  else copy_run<uint8_t>(src, dst, n);
+}
+
 // The dispatch launches for n = T * topk ids with chunk counters `counts`
 // (nchunks * (E + 1) int32, fully written by the count kernel before they are
 // read, so they need no clearing).
@@ -666,6 +692,28 @@ static int gather_run(const char *what, const void *src, int64_t src_rows, int64
     hipLaunchKernelGGL(row_gather_kernel<uint8_t>, dim3(grid), dim3(256), 0, st, (const char *)src,
                        src_rows, row_bytes, idx, rows, (char *)out, div);
   return launch_status(what);
+}
+
+extern "C" int dwm_copy_buffers(const void *const *src, void *const *dst, const int64_t *bytes, int count,
+                                void *stream) {
+  clear_error();
+  DWM_CHECK_ARG(count >= 0 && count <= 4, "copy_buffers: 0 .. 4 buffers (got %d)", count);
+  DWM_CHECK_ARG(count == 0 || (src && dst && bytes), "copy_buffers: null pointer");
+  CopyBuffers b{};
+  int n = 0;
+  int64_t most = 0;
+  for (int i = 0; i < count; ++i) {
+    DWM_CHECK_ARG(bytes[i] >= 0 && (bytes[i] == 0 || (src[i] && dst[i])), "copy_buffers: bad buffer %d", i);
+    if (bytes[i] == 0 || src[i] == dst[i]) continue;
+    b.src[n] = src[i];
+    b.dst[n] = dst[i];
+    b.bytes[n++] = bytes[i];
+    if (bytes[i] > most) most = bytes[i];
+  }
+  if (n == 0) return DWM_OK;
+  const int64_t blocks = (most + 4095) / 4096 < 2048 ? (most + 4095) / 4096 : 2048;
+  hipLaunchKernelGGL(copy_buffers_kernel, dim3((unsigned)blocks, (unsigned)n), dim3(256), 0, as_stream(stream), b);
+  return launch_status("copy_buffers");
 }
 
 extern "C" int dwm_row_gather(const void *src, int64_t src_rows, int64_t row_bytes,

@@ -18,11 +18,12 @@ run in the MX mode (gmm_v2.py): ``hidden`` is quantized once, [T, H] before the 
 blocks run along each row, so gmm1 reads exactly the quantized rows of the
 gathered copy), and gmm2 quantizes the activation.
 """
+import ctypes
 from dataclasses import dataclass
 
 import torch
 
-from . import _trace
+from . import _lib, _trace
 from .gmm_v2 import Fp4Weight, _mx_format, gmm_v2, mx_quantize
 from .moe_fast_combine import fast_combine
 from .moe_fast_dispatch import moe_dispatch, row_gather
@@ -114,10 +115,26 @@ class MoeBlockGraph:
                  topk_weights: torch.Tensor = None) -> torch.Tensor:
         """Copies the given inputs (same shapes and dtypes as at construction)
         into the graph's buffers and replays it on the current stream."""
-        for src, dst in ((hidden, self.hidden), (topk_ids, self.topk_ids), (topk_weights, self.topk_weights)):
-            if src is not None:
-                if src.shape != dst.shape:
-                    raise ValueError(f"MoeBlockGraph: shape {tuple(src.shape)} != captured {tuple(dst.shape)}")
+        pairs = [(src, dst) for src, dst in ((hidden, self.hidden), (topk_ids, self.topk_ids),
+                                             (topk_weights, self.topk_weights)) if src is not None]
+        for src, dst in pairs:
+            if src.shape != dst.shape:
+                raise ValueError(f"MoeBlockGraph: shape {tuple(src.shape)} != captured {tuple(dst.shape)}")
+        # Inputs that are plain copies (dense, same dtype, all on the current
+        # device) go in one launch; anything else takes torch's copy.
+        dev = self.hidden.device
+        plain = dev.index == torch.cuda.current_device() and all(
+            type(src) is torch.Tensor and src.device == dst.device == dev and src.dtype == dst.dtype
+            and src.is_contiguous() and dst.is_contiguous() and not (src.requires_grad or dst.requires_grad)
+            for src, dst in pairs)
+        if plain and pairs:
+            n = len(pairs)
+            _lib.call("dwm_copy_buffers", (ctypes.c_void_p * n)(*(src.data_ptr() for src, _ in pairs)),
+                      (ctypes.c_void_p * n)(*(dst.data_ptr() for _, dst in pairs)),
+                      (ctypes.c_int64 * n)(*(dst.numel() * dst.element_size() for _, dst in pairs)), n,
+                      _lib.raw_stream(dev))
+        else:
+            for src, dst in pairs:
                 dst.copy_(src)
         self.graph.replay()
         return self.out

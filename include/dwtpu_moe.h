@@ -302,6 +302,11 @@ int dwm_moe_dispatch(const int32_t *topk_ids, int64_t T, int topk, int num_exper
                      int32_t *perm, int32_t *tok_sorted, int32_t *revert, int32_t *group_sizes,
                      int32_t *group_offsets, int32_t *flags, void *workspace, void *stream);
 
+/* Copies count (at most 4) device buffers of bytes[i] bytes, src[i] -> dst[i]
+ * (not overlapping, or the same address), in one launch: the inputs of a
+ * captured block before its replay.  The arrays are host memory. */
+int dwm_copy_buffers(const void *const *src, void *const *dst, const int64_t *bytes, int count, void *stream);
+
 /* dwm_moe_dispatch without a workspace argument and without allocating: no
  * counterpart in the reference; it is for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops).  The

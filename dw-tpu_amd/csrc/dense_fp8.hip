@@ -591,9 +591,11 @@ __global__ __launch_bounds__(64 * WR * KS) void dense_fp8_rows_kernel(
 // column scales of the step's K block, W8A8 sw[kb, n0/128] (every wave loads
 // it, so each wave issues the same loads per step).  W8A8's row scales sit
 // outside the ring: every SX_KB K blocks the waves load sx[row0 .. + BM - 1,
-// the next SX_KB K blocks] into one of two [BM][SX_KB] f32 buffers, rows of
-// 4 * SX_KB contiguous bytes (a column of sx read per step would touch one
-// line per row).
+// the next SX_KB K blocks] into one of two f32 buffers, rows of 4 * SX_KB
+// contiguous bytes (a column of sx read per step would touch one line per
+// row), stored [BM / 4][SX_KB][4 rows] so that the fold reads the four
+// consecutive rows of a lane at once (one read per row before: M = 1000,
+// K = 7168, N = 4096 47.2 -> 46.2 us, M = 4096 153 -> 148).
 template <int WM, int WN, bool A8, int JN = 2>
 struct DenseMfmaCfg {
   static constexpr int WAVES = WM * WN, THREADS = 64 * WAVES, WCOLS = WN, JCOLS = JN;
@@ -606,7 +608,7 @@ struct DenseMfmaCfg {
   static constexpr int S_BYTES = WAVES * 256;  // one 64-value scale load per wave
   static constexpr int STAGE = (S + S_BYTES + 1023) / 1024 * 1024;
   static constexpr int SX_KB = BM == 256 ? 4 : 8;                  // W8A8: K blocks per row-scale chunk
-  static constexpr int SX_BUF = BM * SX_KB * 4;                    // [BM rows][SX_KB] f32
+  static constexpr int SX_BUF = BM * SX_KB * 4;                    // [BM / 4][SX_KB][4] f32
   static constexpr int SX_BYTES = A8 ? 2 * SX_BUF : 0;
   static constexpr int SX_LOADS = A8 ? SX_BUF / 256 / WAVES : 0;   // 256-byte loads per wave per chunk
   static constexpr int A_LOADS = BM * A_ROW / 1024 / WAVES;        // 1 KiB lhs loads per wave per step
@@ -693,9 +695,9 @@ __global__ __launch_bounds__(C::THREADS) void dense_fp8_mfma_kernel(
   const uint32_t slane = A8 ? (uint32_t)(n0 / 128) * 4u : (uint32_t)min(n0 + 64 * wave + lane, N - 1) * 4u;
   const uint32_t sstride = (uint32_t)sw_ld * 4u;  // bytes per K block
   // W8A8 row scales: load i of this wave covers block rows XR (wave + WAVES i)
-  // .. + XR - 1 (XR = 64 / SX_KB), lane l row + l / SX_KB, K block
-  // kb0 + SX_KB c + l % SX_KB of chunk c (rows past M repeat the last row; K
-  // blocks past the block's run are never read).
+  // .. + XR - 1 (XR = 64 / SX_KB): lane l row + 4 (l / (4 SX_KB)) + l % 4, K
+  // block kb0 + SX_KB c + l / 4 % SX_KB of chunk c (rows past M repeat the last
+  // row; K blocks past the block's run are never read).
   constexpr int XR = 64 / C::SX_KB;
   __amdgpu_buffer_rsrc_t xrsrc;
   uint32_t xoff[C::SX_LOADS > 0 ? C::SX_LOADS : 1];
@@ -703,9 +705,9 @@ __global__ __launch_bounds__(C::THREADS) void dense_fp8_mfma_kernel(
     xrsrc = make_rsrc(sx, (uint32_t)(M * KB * 4));
 #pragma unroll
     for (int i = 0; i < C::SX_LOADS; ++i) {
-      int64_t r = row0 + XR * (wave + C::WAVES * i) + lane / C::SX_KB;
+      int64_t r = row0 + XR * (wave + C::WAVES * i) + 4 * (lane / (4 * C::SX_KB)) + lane % 4;
       if (r >= M) r = M - 1;
-      xoff[i] = (uint32_t)(r * KB) * 4u + (uint32_t)(lane % C::SX_KB) * 4u;
+      xoff[i] = (uint32_t)(r * KB) * 4u + (uint32_t)(lane / 4 % C::SX_KB) * 4u;
     }
   }
   uint8_t *const s_sx = s_lds + NS * C::STAGE;
@@ -944,15 +946,18 @@ __global__ __launch_bounds__(C::THREADS) void dense_fp8_mfma_kernel(
           }
         } else {
           const float swv = *(const float *)(st + C::S);
-          // sx[row, kb0 + t] of block row r at s_sx[t / SX_KB % 2][r][t % SX_KB]
-          const float *const xs = (const float *)(s_sx + ((t / C::SX_KB) & 1) * C::SX_BUF) + t % C::SX_KB;
+          // sx[row, kb0 + t] of block row r at s_sx[t / SX_KB % 2][r / 4][t % SX_KB][r % 4]
+          const float *const xs = (const float *)(s_sx + ((t / C::SX_KB) & 1) * C::SX_BUF) + t % C::SX_KB * 4;
 #pragma unroll
           for (int i = 0; i < 2; ++i) {
             float f[16];
 #pragma unroll
             for (int g = 0; g < 4; ++g)
+            {
+              const f32x4_t x4 = *(const f32x4_t *)(xs + (rA[i] - c32 + 8 * g + 4 * h) * C::SX_KB);
 #pragma unroll
-              for (int q = 0; q < 4; ++q) f[4 * g + q] = xs[(rA[i] - c32 + 8 * g + 4 * h + q) * C::SX_KB] * swv;
+              for (int q = 0; q < 4; ++q) f[4 * g + q] = x4[q] * swv;
+            }
 #pragma unroll
             for (int j = 0; j < JN; ++j)
 #pragma unroll

@@ -13,7 +13,8 @@
 //   (exact: 3 mantissa bits, exponents inside bf16's range) for bf16 MFMA
 //   32x32x16; W8A8 runs the fp8 MFMA 32x32x64 on the codes.
 // - M <= 16: dense_fp8_skinny_kernel (see below).
-// - 17 <= M <= 32 (W8A8: 96), N % 128 == 0: dense_fp8_rows_kernel (see below).
+// - 17 <= M <= 32, or W8A8 up to 96 (its N % 128 == 0): dense_fp8_rows_kernel (see below).
+// - W8A16, M > 64, other N: the MFMA tiles with a clamped last column tile.
 // - Other shapes: dense_fp8_kernel, bf16 MFMA 16x16x32 on decoded codes.
 // Every product is the exact fp8 (or bf16 x fp8) product; the 128-K partial
 // is an f32 sum of them.
@@ -450,7 +451,8 @@ __global__ __launch_bounds__(64 * WR * KS) void dense_fp8_rows_kernel(
     const uint8_t *const ab = x + (int64_t)kb * 128 * XB;
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
-      const uint8_t *const wb = wpk + ((int64_t)(nb0 + j) * KB + kb) * 2048;
+      // column groups past N (W8A16) repeat the last one and are not stored
+      const uint8_t *const wb = wpk + ((int64_t)min(nb0 + j, (N >> 4) - 1) * KB + kb) * 2048;
       b[d][j] = *(const i32x8_a16_t *)(wb + woff);
     }
 #pragma unroll
@@ -461,7 +463,7 @@ __global__ __launch_bounds__(64 * WR * KS) void dense_fp8_rows_kernel(
       ws[d][0] = sw[(int64_t)kb * sw_ld + (nb0 * 16 >> 7)];
     } else {
 #pragma unroll
-      for (int j = 0; j < NB; ++j) ws[d][j] = sw[(int64_t)kb * sw_ld + (nb0 + j) * 16 + c16];
+      for (int j = 0; j < NB; ++j) ws[d][j] = sw[(int64_t)kb * sw_ld + min(nb0 + j, (N >> 4) - 1) * 16 + c16];
     }
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -557,7 +559,7 @@ __global__ __launch_bounds__(64 * WR * KS) void dense_fp8_rows_kernel(
     const int64_t col = (int64_t)(nb0 + tt % NB) * 16 + c16;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      if (row + e < M) {
+      if (row + e < M && (A8 || col < N)) {
         if (partial) partial[((int64_t)blockIdx.z * M + row + e) * N + col] = v[e];
         else out[(int64_t)(row + e) * N + col] = f32_to_bf16_bits(v[e]);
       }
@@ -1092,9 +1094,18 @@ static dwm_dense_plan tiled_default(int64_t M, int64_t K, int64_t N) {
 // one K block each, fragments read one substep ahead) from M >= 256, 128x128
 // below (four 33 KB stages).  K is split over blocks until the grid covers
 // the 256 CUs.
+static bool dense_offsets_ok(int64_t M, int64_t K, int64_t N, int tile_m) {
+  return M * K * 2 < (1ll << 32) && K * N < (1ll << 32) && (M + tile_m - 1) / tile_m <= 65535;
+}
 static bool dense_mfma_ok(int64_t M, int64_t K, int64_t N, int tile_m) {
-  return M > 16 && N % 128 == 0 && M * K * 2 < (1ll << 32) && K * N < (1ll << 32) &&
-         (M + tile_m - 1) / tile_m <= 65535;
+  return M > 16 && N % 128 == 0 && dense_offsets_ok(M, K, N, tile_m);
+}
+// The same tiles for other widths (W8A16): the last column tile's loads are
+// clamped to N and its columns past N are not stored.  Against the general
+// tiled kernel: 100 rows, K = 7168, N = 4000 45.2 -> 17.9 us, 700 rows, K =
+// 5120, N = 4080 123 -> 46, 4000 rows, K = 7168 798 -> 261.
+static bool dense_edge_ok(int64_t M, int64_t K, int64_t N, int tile_m) {
+  return M > 64 && N > 128 && N % 128 != 0 && dense_offsets_ok(M, K, N, tile_m);
 }
 
 // Smallest run count with the same runs: no run is left empty.
@@ -1120,17 +1131,21 @@ static int rows_blocks(int64_t M) { return (int)(((M + 15) / 16 + rows_halves(M)
 // W8A16 takes it up to 32 rows (17 rows 14.3 -> 10.9, 32 14.9 -> 11.8; K =
 // 1024, N = 32768 20.8 -> 14.6): its lhs fragments are 64 bytes a lane, half
 // lines of every row, and from 48 rows on they cost more than the tiles' LDS
-// copies (48 rows 15.9 -> 16.4, 64 16.7 -> 19.7).
+// copies (48 rows 15.9 -> 16.4, 64 16.7 -> 19.7); off the 128-column grid it
+// replaces the general tiled kernel (32 rows, N = 4048 18.0 -> 12.1).
 static bool rows_rule(int64_t M, int64_t N, bool a8) {
   return M <= 32 || (a8 && M <= kRowsMax && N / (16 * rows_groups(rows_blocks(M))) <= 256);
+}
+static bool rows_ok(int64_t M, int64_t K, int64_t N, bool a8) {
+  return M > 16 && M <= (a8 ? kRowsMax : 32) && (!a8 || N % 128 == 0) && dense_offsets_ok(M, K, N, 128);
 }
 
 static dwm_dense_plan default_plan(int64_t M, int64_t K, int64_t N, bool a8) {
   const int64_t KB = K / 128;
-  if (rows_rule(M, N, a8) && dense_mfma_ok(M, K, N, 128)) {
+  if (rows_ok(M, K, N, a8) && rows_rule(M, N, a8)) {
     // One block per CU, while every wave keeps a K block; at most kRowsKb per block.
     const int tn = 16 * rows_groups(rows_blocks(M));
-    const int64_t ct = N / tn, waves = 8 / rows_halves(M);
+    const int64_t ct = (N + tn - 1) / tn, waves = 8 / rows_halves(M);
     int64_t ks = (256 + ct - 1) / ct;
     if (ks > KB / waves) ks = KB / waves;
     if (ks < (KB + kRowsKb - 1) / kRowsKb) ks = (KB + kRowsKb - 1) / kRowsKb;
@@ -1153,6 +1168,13 @@ static dwm_dense_plan default_plan(int64_t M, int64_t K, int64_t N, bool a8) {
     // Two blocks per CU either way; a grid that fits one round takes the
     // deeper ring.
     return {DWM_DENSE_MFMA, 128, 128, ks, tiles * ks <= 512 ? 3 : 2};
+  }
+  if (!a8 && dense_edge_ok(M, K, N, 128)) {
+    const int64_t ct = (N + 127) / 128;
+    if (ct * ((M + 255) / 256) >= 256) return {DWM_DENSE_EDGE, 256, 128, 1, 3};
+    int ks = 1;
+    while (ct * ((M + 127) / 128) * ks < 256 && ks * 2 <= KB && ks < 16) ks *= 2;
+    return {DWM_DENSE_EDGE, 128, 128, whole_runs(KB, ks), 3};
   }
   // 16 waves split K, two K blocks (weights, lhs fragments and scales) in
   // flight per wave; 4/8/16 waves x 2..7 blocks in flight all measured
@@ -1192,9 +1214,16 @@ static int check_plan(int64_t M, int64_t K, int64_t N, bool a8, const dwm_dense_
       DWM_UNSUPPORTED_IF(!ok, "dense_fp8 plan: %s %d-row MFMA tiles have no %d-stage ring", v, p.tile_m, p.stages);
       return DWM_OK;
     }
+    case DWM_DENSE_EDGE: {
+      DWM_UNSUPPORTED_IF(a8 || p.tile_n != 128 || (p.tile_m != 128 && p.tile_m != 256) || p.stages != 3,
+                         "dense_fp8 plan: edge tiles are W8A16, 128 x 128 or 256 x 128 with a 3-stage ring");
+      DWM_UNSUPPORTED_IF(!dense_edge_ok(M, K, N, p.tile_m),
+                         "dense_fp8 plan: edge tiles need M > 64, N > 128, N %% 128 != 0 and 32-bit operand offsets");
+      return DWM_OK;
+    }
     case DWM_DENSE_ROWS: {
-      DWM_UNSUPPORTED_IF(M > (a8 ? kRowsMax : 32) || !dense_mfma_ok(M, K, N, 128),
-                         "dense_fp8 plan: the rows kernel takes 17 <= M <= 32 (W8A8: %lld) and N %% 128 == 0",
+      DWM_UNSUPPORTED_IF(!rows_ok(M, K, N, a8),
+                         "dense_fp8 plan: the rows kernel takes 17 <= M <= 32 (W8A8: %lld, N %% 128 == 0)",
                          (long long)kRowsMax);
       DWM_UNSUPPORTED_IF(p.tile_m != 16 * rows_blocks(M) * rows_halves(M) || p.tile_n != 16 * rows_groups(rows_blocks(M)) ||
                              p.stages != 2,
@@ -1227,7 +1256,7 @@ static thread_local dwm_dense_plan t_last_plan{0, 0, 0, 0, 0};
 template <class C, bool A8, int NS>
 static void launch_mfma(const void *x, const float *sx, int64_t M, int64_t K, int64_t N, const uint8_t *w,
                         const float *sw, int sw_ld, int ks, uint16_t *out, float *partial, hipStream_t st) {
-  const dim3 grid((unsigned)(N / C::BN), (unsigned)((M + C::BM - 1) / C::BM), (unsigned)ks);
+  const dim3 grid((unsigned)((N + C::BN - 1) / C::BN), (unsigned)((M + C::BM - 1) / C::BM), (unsigned)ks);
   hipLaunchKernelGGL((dense_fp8_mfma_kernel<C, A8, NS, A8>), grid, dim3(C::THREADS), 0, st, x, sx, M, (int)K, (int)N,
                      w, sw, sw_ld, ks, out, partial);
 }
@@ -1236,7 +1265,7 @@ template <int MB, int WR, bool A8>
 static void launch_rows(const void *x, const float *sx, int64_t M, int64_t K, int64_t N, const uint8_t *w,
                         const float *sw, int sw_ld, int ks, uint16_t *out, float *partial, hipStream_t st) {
   constexpr int NB = rows_groups(MB);
-  hipLaunchKernelGGL((dense_fp8_rows_kernel<MB, NB, WR, 8 / WR, A8>), dim3((unsigned)(N / (16 * NB)), 1, (unsigned)ks),
+  hipLaunchKernelGGL((dense_fp8_rows_kernel<MB, NB, WR, 8 / WR, A8>), dim3((unsigned)((N + 16 * NB - 1) / (16 * NB)), 1, (unsigned)ks),
                      dim3(512), 0, st, (const uint8_t *)x, sx, (int)M, (int)K, (int)N, w, sw, sw_ld, ks, out, partial);
 }
 
@@ -1315,7 +1344,7 @@ static int run_dense(const void *x, const float *sx, int64_t M, int64_t K, int64
       else if (p.tile_m == 64) launch_rows<4, 1, true>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
       else if (p.tile_m == 96) launch_rows<3, 2, true>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
     }
-  } else if (p.kernel == DWM_DENSE_MFMA) {
+  } else if (p.kernel == DWM_DENSE_MFMA || p.kernel == DWM_DENSE_EDGE) {
     if constexpr (A8) {
       if (p.tile_m == 256) launch_mfma<DenseMfmaCfg<4, 2, true>, true, 3>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
       else if (p.stages == 3) launch_mfma<DenseMfmaCfg<2, 2, true>, true, 3>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);

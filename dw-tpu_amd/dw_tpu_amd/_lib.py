@@ -75,7 +75,7 @@ SIGNATURES = {
 _RESTYPES = {"dwm_last_error": ctypes.c_char_p}
 
 # enum dwm_dense_kernel
-DENSE_SKINNY, DENSE_MFMA, DENSE_TILED, DENSE_ROWS = 1, 2, 3, 4
+DENSE_SKINNY, DENSE_MFMA, DENSE_TILED, DENSE_ROWS, DENSE_EDGE = 1, 2, 3, 4, 5
 
 
 class GmmLhs(ctypes.Structure):

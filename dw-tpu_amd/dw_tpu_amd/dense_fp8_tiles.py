@@ -16,7 +16,8 @@ What they mean here is a launch of this library's kernels
                    tn = 64 or 32: the rows kernel (17 <= M <= 32, W8A8 <= 96; tm
                    = M rounded up to 32 (tn = 64), 48, 64 or 96 (32));
   mode "megablox"  the general tiled kernel, tm x tn = 16 x 64, 64 x 128 or
-                   128 x 128 (any N % 16 == 0);
+                   128 x 128 (any N % 16 == 0); with "stages" 3 the MFMA tiles
+                   of a width off the 128 grid (M > 64, tm = 128 or 256);
   tk               the K depth one block covers: K / tk blocks share an
                    output tile and their f32 partials are added in order;
   "stages"         optional ring depth (LDS stages of the MFMA kernel);
@@ -73,7 +74,7 @@ def plan_to_tile(plan, k):
     if plan.kernel == _lib.DENSE_SKINNY:
         return DenseTile("native", plan.tile_m, k, plan.tile_n, plan.stages)
     tk = 128 * -(-kb // plan.ksplit)
-    mode = "megablox" if plan.kernel == _lib.DENSE_TILED else "native"
+    mode = "megablox" if plan.kernel in (_lib.DENSE_TILED, _lib.DENSE_EDGE) else "native"
     return DenseTile(mode, plan.tile_m, tk, plan.tile_n, plan.stages)
 
 
@@ -89,7 +90,9 @@ def tile_to_plan(tile, m, k, n, w8a8=False):
     if tk <= 0 or tk % 128:
         raise ValueError(f"tk={tk} must be a positive multiple of 128 (the scale block)")
     kernel = _KERNEL_OF_MODE[mode]
-    if kernel is None:
+    if kernel is not None:
+        kernel = _lib.DENSE_EDGE if stages == 3 else kernel
+    else:
         kernel = (_lib.DENSE_SKINNY if (tm, tn) == (16, 16) else _lib.DENSE_ROWS if tn in (32, 64) else _lib.DENSE_MFMA)
     if kernel == _lib.DENSE_SKINNY:
         if tk != k:

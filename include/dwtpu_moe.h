@@ -415,11 +415,14 @@ enum dwm_dense_kernel {
   /* General tiles for any N % 16 == 0: 16 x 64, 64 x 128 or 128 x 128,
    * 16x16x32 bf16 MFMA, double-buffered LDS (stages = 2). */
   DWM_DENSE_TILED = 3,
-  /* 17 <= M <= 32 (W8A8: 96), N % 128 == 0: M rounded up to 32 rows x 64
+  /* 17 <= M <= 32 (W8A8: 96, N % 128 == 0): M rounded up to 32 rows x 64
    * columns, or 48, 64 or 96 rows x 32 columns per block, operands
    * straight from memory to registers (ring depth 2), at most 32 K blocks per
    * K run. */
-  DWM_DENSE_ROWS = 4
+  DWM_DENSE_ROWS = 4,
+  /* W8A16, M > 64, N > 128, N % 128 != 0: the 128 x 128 or 256 x 128 MFMA
+   * tiles (3 stages), the last column tile part-filled. */
+  DWM_DENSE_EDGE = 5
 };
 
 typedef struct dwm_dense_plan {

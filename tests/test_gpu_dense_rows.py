@@ -62,6 +62,16 @@ def test_w8a8_rows_plans_against_oracle(dev, M, K, N, plan):
     (64, 1152, 128, (2, 64, 128, 5, 4)),   # runs of 2, 2, 2, 2, 1 K blocks: two steps in a four-stage ring
     (48, 384, 33024, (2, 64, 128, 1, 4)),
     (65, 1024, 256, (2, 128, 128, 8, 3)),
+    # widths off the 128 grid: rows kernel, general tiles (33 .. 64 rows), MFMA tiles with a part-filled last one
+    (17, 256, 16, (4, 32, 64, 1, 2)),
+    (32, 2048, 208, (4, 32, 64, 2, 2)),
+    (29, 384, 4080, (4, 32, 64, 1, 2)),
+    (64, 512, 144, (3, 64, 128, 4, 2)),
+    (65, 512, 144, (5, 128, 128, 4, 3)),
+    (128, 1152, 240, (5, 128, 128, 5, 3)),
+    (300, 256, 1040, (5, 128, 128, 2, 3)),
+    (200, 512, 112, (3, 128, 128, 4, 2)),   # a single part-filled tile stays on the general kernel
+    (2049, 128, 3600, (5, 256, 128, 1, 3)),
 ])
 def test_w8a16_rows_plans_against_oracle(dev, M, K, N, plan):
     from dw_tpu_amd.dense_fp8 import last_plan, matmul, prepack_fp8, try_dense_fp8

@@ -298,8 +298,8 @@ def prep_dispatch_combine(dev, steps, warmup):
         assert keep
         res = {}
         ms = time_steps(lambda i: call(lib.dwm_moe_dispatch, disp_args), steps, warmup)
-        res["dispatch"] = {"ms": round(ms, 5), "ids": n, "experts": wl.E, "kernels": 1 if n <= 8192 else 3,
-                           "note": "launch-latency bound (one 1024-thread block)"}
+        res["dispatch"] = {"ms": round(ms, 5), "ids": n, "experts": wl.E, "kernels": 1 if n <= 65536 else 3,
+                           "note": "launch-latency bound"}
         ms = time_steps(lambda i: call(lib.dwm_row_gather, gargs[i % gc]), steps, warmup)
         gb = wl.T * wl.K * 2 + n * wl.K * 2 + n * 4
         res["row_gather"] = {"ms": round(ms, 5), "GB_s": round(gb / (ms * 1e-3) / 1e9, 1), "rows": n, "H": wl.K,

@@ -33,39 +33,50 @@ constexpr int kStreamRows = 32;  // rows of a row tile
 // by side on one XCD and share its L2's copy of the weights), column tile ct
 // of n_ct.  The tile list is cut into 8 contiguous runs, one per XCD (blocks
 // whose index is equal mod 8).  Every wave finds its tile alone: lane l holds
-// the sizes of groups l PL .. + PL - 1, two prefix sums over the lanes
-// give row starts and row-tile counts.  Returns false when there is no tile.
+// the sizes of groups l PL .. + PL - 1, and prefix sums over the lanes give
+// row starts, then row-tile counts.  Returns false when there is no tile.
+//
+// Group sizes are not checked by the host: negative ones count as empty, and
+// every group is cut to the rows left below M before its tiles are counted,
+// so the list holds the tiles of rows [0, M) and no others, and fits the grid
+// (stream_grid) whatever the sizes sum to.
 template <int PL>
 __device__ __forceinline__ bool stream_tile(const int32_t *__restrict__ group_sizes, int num_groups, int go,
                                             int64_t e_local, int64_t M, int n_ct, int &g, int64_t &row0, int &rows,
                                             int &ct) {
   const int lane = threadIdx.x & 63;
-  int sz[PL], v[2] = {0, 0};
+  const int m32 = (int)min(M, (int64_t)0x7FFFFFFF);
+  int sz[PL], rows_in = 0, tiles = 0;
 #pragma unroll
   for (int i = 0; i < PL; ++i) sz[i] = group_sizes[min(lane * PL + i, num_groups - 1)];  // loads side by side
 #pragma unroll
-  for (int i = 0; i < PL; ++i) sz[i] = lane * PL + i < num_groups ? max(sz[i], 0) : 0;
+  for (int i = 0; i < PL; ++i) {
+    sz[i] = lane * PL + i < num_groups ? min(max(sz[i], 0), m32) : 0;
+    rows_in += sz[i];
+  }
+  const int start = wave_inclusive_scan(rows_in) - rows_in;  // first row of the lane's first group
+  int left = start >= 0 ? max(m32 - start, 0) : 0;           // (a sum past int32 is past M too)
   auto tiles_of = [&](int gi, int s) {
     return gi >= go && (int64_t)gi < (int64_t)go + e_local ? s / kStreamRows + (s % kStreamRows != 0 ? 1 : 0) : 0;
   };
 #pragma unroll
   for (int i = 0; i < PL; ++i) {
-    v[0] += sz[i];
-    v[1] += tiles_of(lane * PL + i, sz[i]);
+    sz[i] = min(sz[i], left);
+    left -= sz[i];
+    tiles += tiles_of(lane * PL + i, sz[i]);
   }
-  const int own[2] = {v[0], v[1]};
-  wave_inclusive_scan_n<2>(v);
-  const int64_t total = (int64_t)wave_last(v[1]) * n_ct;
+  const int upto = wave_inclusive_scan(tiles), before = upto - tiles;  // row tiles before the lane's groups
+  const int64_t total = (int64_t)wave_last(upto) * n_ct;
   const int64_t run = (total + 7) >> 3;
   const int64_t j = blockIdx.x >> 3;
   const int64_t entry = (int64_t)(blockIdx.x & 7) * run + j;
   if (j >= run || entry >= total || entry > 0x7FFFFFFFll) return false;
   const int trow = (int)((uint32_t)entry / (uint32_t)n_ct);
-  const uint64_t hit = __ballot(v[1] - own[1] <= trow && trow < v[1]);
+  const uint64_t hit = __ballot(before <= trow && trow < upto);
   if (!hit) return false;
   const int sel = __ffsll((unsigned long long)hit) - 1;
-  int rs = __builtin_amdgcn_readlane(v[0] - own[0], sel);  // first row of lane sel's first group
-  int tc = __builtin_amdgcn_readlane(v[1] - own[1], sel);  // row tiles before it
+  int rs = __builtin_amdgcn_readlane(start, sel);
+  int tc = __builtin_amdgcn_readlane(before, sel);
   g = -1;
   int szg = 0;
 #pragma unroll
@@ -86,12 +97,9 @@ __device__ __forceinline__ bool stream_tile(const int32_t *__restrict__ group_si
   const uint32_t n = (uint32_t)tiles_of(g, szg), local = (uint32_t)entry - (uint32_t)tc * (uint32_t)n_ct;
   const int rt = (int)(local % n);
   ct = (int)(local / n);
-  // Group sizes are not checked by the host (find_tile): a row start outside
-  // [0, M) has no tile, and no tile reaches past M.
   row0 = (int64_t)rs + (int64_t)rt * kStreamRows;
-  if (rs < 0 || row0 >= M) return false;
-  rows = (int)min((int64_t)min(szg - rt * kStreamRows, kStreamRows), M - row0);
-  return rows > 0;
+  rows = min(szg - rt * kStreamRows, kStreamRows);
+  return true;
 }
 
 __device__ __forceinline__ bool find_stream_tile(const int32_t *__restrict__ group_sizes, int num_groups, int go,

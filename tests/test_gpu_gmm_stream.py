@@ -153,3 +153,42 @@ def test_stream_kernel_skips_rows_past_m(dev, rng):
         assert (out[M:] == 0x1234).all()
         outs.append(out[:M])
     assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("mx", [False, True])
+@pytest.mark.parametrize("E,sizes,M", [
+    (8, {0: 10000}, 20),                         # the first group alone runs far past M
+    (8, {0: 3, 2: 40, 5: 1 << 30, 6: 1 << 30}, 47),  # the sum leaves int32
+    (300, {7: 5, 40: 33, 120: 2000, 280: 2000}, 60),  # several sizes per lane
+])
+def test_stream_kernel_covers_the_rows_below_m(dev, rng, mx, E, sizes, M):
+    """Device group sizes that sum far past M, with many more tiles than the
+    grid has blocks: every row below M is that of sizes cut to fit, and none
+    past it is written."""
+    import ctypes
+    from dw_tpu_amd import _lib, fp4_weight_to_codes, mx_quantize
+    K, N, pad = 256, 512, 64
+    s = np.zeros(E, np.int64)
+    s[list(sizes)] = list(sizes.values())
+    fit = np.minimum(s, np.maximum(0, M - np.concatenate([[0], np.cumsum(s)[:-1]])))
+    assert M <= 6 * E and fit.sum() == M
+    pw = fp4_weight_to_codes(torch.from_numpy(rng.integers(0, 256, (E, K, N // 2), dtype=np.uint8)).to(dev),
+                             torch.from_numpy(rng.integers(123, 130, (E, K // 32, 1, N), dtype=np.uint8)).to(dev))
+    lhs = bf16_tensor(f32_to_bf16_bits(rng.standard_normal((M + pad, K)).astype(np.float32)), dev)
+    q = mx_quantize(lhs)
+    P = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    outs = []
+    for v in (s, fit):
+        gs = torch.from_numpy(v.astype(np.int32)).to(dev)
+        out = torch.full((M + pad, N), 0x1234, dtype=torch.int16, device=dev)
+        tail = (M, K, P(pw.weight), P(pw.scale), P(gs), E, None, E, N, P(out), _lib.BF16, 0, _lib.ACT_NONE,
+                _lib.stream_handle(dev))
+        if mx:
+            _lib.call("dwm_gmm_fp4_mx", P(q.codes), P(q.scales), M, None, *tail)
+        else:
+            _lib.call("dwm_gmm_fp4", P(lhs), *tail)
+        torch.cuda.synchronize()
+        assert (out[M:] == 0x1234).all()
+        outs.append(out[:M])
+    assert (outs[1] != 0x1234).any(dim=1).all()
+    assert torch.equal(outs[0], outs[1])

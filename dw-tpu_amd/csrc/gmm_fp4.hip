@@ -652,7 +652,7 @@ int launch_gmm_zero_rows(const int32_t *group_sizes, int num_groups, const int32
 
 // Compute units of the current device (looked up once per device).  It only
 // sizes the narrow split; any positive value gives correct results.
-static int device_cu_count() {
+int device_cu_count() {
   constexpr int kMaxDev = 64;
   static std::atomic<int> cache[kMaxDev];
   int dev = 0;

@@ -2,8 +2,9 @@
 // product, layouts and results as gmm_fp4.hip, built for streaming weights.
 //
 // What bounds it: HBM (6.6 TB/s reached at 198 rows over 256 experts, K = N =
-// 4096: 188 us, the tiles 256; one token over 32 experts 49 -> 23).  With at most 32 rows per expert each weight byte
-// feeds at most 64 FLOPs, so the packed weights' stream sets the time.
+// 4096: 188 us, the tiles 256; one token over 32 experts 49 -> 23).  Up to 32
+// rows of an expert a weight byte (two codes) feeds at most 128 FLOPs, so the
+// packed weights' stream sets the time.
 // The 512-column tiles of gmm_fp4.hip leave CUs idle when few experts hold
 // rows (one token with top-8: 64 tiles for 256 CUs) and pay their start and
 // epilogue once per tile with nothing else on the CU.
@@ -26,64 +27,118 @@
 
 namespace dwm {
 
-constexpr int kStreamRows = 32;  // rows of a row tile
+// The wave's tile: `rows` rows from row0 of group g, 64-column group cg;
+// once: no other row tile of the group reads the same weights.
+struct StreamRef {
+  int64_t row0;
+  int g, rows, cg;
+  bool once;
+};
 
-// The wave's tile: row tile rt of group g (row tiles of kStreamRows rows,
-// innermost in the order so that the row tiles of one column tile run side
-// by side on one XCD and share its L2's copy of the weights), column tile ct
-// of n_ct.  The tile list is cut into 8 contiguous runs, one per XCD (blocks
-// whose index is equal mod 8).  Every wave finds its tile alone: lane l holds
-// the sizes of groups l PL .. + PL - 1, and prefix sums over the lanes give
-// row starts, then row-tile counts.  Returns false when there is no tile.
+// A block's first w waves take w adjacent 64-column groups of one row tile.
+// The list runs (group, column tile, row tile) with the row tile innermost,
+// so that the row tiles of one column tile run side by side on one XCD and
+// share its L2's copy of the weights; it is cut into 8 contiguous runs, one
+// per XCD (blocks whose index is equal mod 8).  Every wave finds its tile
+// alone: lane l holds the sizes of groups l PL .. + PL - 1, and prefix sums
+// over the lanes give row starts and row-tile counts.  Returns false when
+// the wave has no tile.
 //
 // Group sizes are not checked by the host: negative ones count as empty, and
-// every group is cut to the rows left below M before its tiles are counted,
-// so the list holds the tiles of rows [0, M) and no others, and fits the grid
-// (stream_grid) whatever the sizes sum to.
-template <int PL>
+// sizes that sum past M are cut to the rows left below M before their tiles
+// are counted, so the list holds the tiles of rows [0, M) and no others, and
+// fits the grid (stream_grid) whatever the sizes sum to.
+//
+// Row tiles hold 16 rows (MX: 32, its MFMA's) or 32.  With 16 the waves are
+// alike: while weights stream from HBM, a wave with twice the rows falls
+// behind and ends alone.  32 are taken where most tiles would share their
+// weights with another one anyway (few groups hold all rows: larger tiles
+// read less from L2), where only they fit one round of waves, and where 16
+// would not fit the grid.  Against 32 throughout, us: 384 rows over 64
+// experts by a Zipf law (1.1), K = N = 4096 100.5 -> 90.5; 192 such rows over
+// 32 experts, K = 2048, N = 7168 50.5 -> 44.0; 32 of 64 rows in one of 32
+// experts, K = 7168 101.5 -> 86.2.  Against 16 throughout: 1536 rows in one
+// of 256 experts 121 -> 109; 192 Zipf rows over 32 experts, K = 7168 94 -> 88.
+//
+// Blocks of four waves share their lhs rows through L1.  A launch of at most
+// one round takes one or two waves a block where that leaves fewer waves on
+// the fullest CU (128 rows in 4 of 64 experts, K = N = 4096 37.6 -> 15.5).
+template <int PL, bool MX, int WPB>
 __device__ __forceinline__ bool stream_tile(const int32_t *__restrict__ group_sizes, int num_groups, int go,
-                                            int64_t e_local, int64_t M, int n_ct, int &g, int64_t &row0, int &rows,
-                                            int &ct) {
+                                            int64_t e_local, int64_t M, int G, int max_rt, int ncu, int wave,
+                                            StreamRef &ref) {
   const int lane = threadIdx.x & 63;
   const int m32 = (int)min(M, (int64_t)0x7FFFFFFF);
-  int sz[PL], rows_in = 0, tiles = 0;
+  int sz[PL];
 #pragma unroll
   for (int i = 0; i < PL; ++i) sz[i] = group_sizes[min(lane * PL + i, num_groups - 1)];  // loads side by side
+  auto tiles_of = [&](int gi, int s, int lg) {
+    return gi >= go && (int64_t)gi < (int64_t)go + e_local ? (s >> lg) + ((s & ((1 << lg) - 1)) != 0 ? 1 : 0) : 0;
+  };
+  int v[3] = {0, 0, 0}, own[3];  // rows, row tiles of 32 rows, of 16
+  auto count = [&]() {
 #pragma unroll
-  for (int i = 0; i < PL; ++i) {
-    sz[i] = lane * PL + i < num_groups ? min(max(sz[i], 0), m32) : 0;
-    rows_in += sz[i];
-  }
-  const int start = wave_inclusive_scan(rows_in) - rows_in;  // first row of the lane's first group
-  int left = start >= 0 ? max(m32 - start, 0) : 0;           // (a sum past int32 is past M too)
-  auto tiles_of = [&](int gi, int s) {
-    return gi >= go && (int64_t)gi < (int64_t)go + e_local ? s / kStreamRows + (s % kStreamRows != 0 ? 1 : 0) : 0;
+    for (int a = 0; a < 3; ++a) v[a] = 0;
+#pragma unroll
+    for (int i = 0; i < PL; ++i) {
+      v[0] += sz[i];
+      v[1] += tiles_of(lane * PL + i, sz[i], 5);
+      if (!MX) v[2] += tiles_of(lane * PL + i, sz[i], 4);
+    }
+#pragma unroll
+    for (int a = 0; a < 3; ++a) own[a] = v[a];
+    wave_inclusive_scan_n<3>(v);  // (MX: v[2] is 0 and folds away)
   };
 #pragma unroll
-  for (int i = 0; i < PL; ++i) {
-    sz[i] = min(sz[i], left);
-    left -= sz[i];
-    tiles += tiles_of(lane * PL + i, sz[i]);
+  for (int i = 0; i < PL; ++i) sz[i] = lane * PL + i < num_groups ? min(max(sz[i], 0), m32) : 0;
+  count();
+  if (__ballot(v[0] < 0 || v[0] > m32) != 0) {
+    // A sum past int32 turns negative there: the lanes after it are past M.
+    const uint64_t neg = __ballot(v[0] < 0);
+    const int start = v[0] - own[0];
+    int left = neg != 0 && lane >= __ffsll((unsigned long long)neg) ? 0 : max(m32 - start, 0);
+#pragma unroll
+    for (int i = 0; i < PL; ++i) {
+      sz[i] = min(sz[i], left);
+      left -= sz[i];
+    }
+    count();
   }
-  const int upto = wave_inclusive_scan(tiles), before = upto - tiles;  // row tiles before the lane's groups
-  const int64_t total = (int64_t)wave_last(upto) * n_ct;
+  const int64_t cap = 8 * (int64_t)ncu;  // waves of one round: 256 VGPRs each
+  const int all32 = wave_last(v[1]), all16 = MX ? 0 : wave_last(v[2]);
+  const bool small = !MX && all16 <= max_rt && 2 * (int64_t)all16 < 3 * (int64_t)all32 &&
+                     (all16 * (int64_t)G <= cap || all32 * (int64_t)G > cap);
+  const int lg = small ? 4 : 5, all = small ? all16 : all32;
+  const int upto = small ? v[2] : v[1], before = upto - (small ? own[2] : own[1]);
+  const int j = blockIdx.x >> 3;
+  if (j >= (all * (int64_t)G + 7) >> 3) return false;  // past the run of every w
+  int w = WPB;
+  if (WPB == 4 && all * (int64_t)G <= cap) {
+    // Waves on the fullest CU with k a block; the list has to fit the grid.
+    auto fullest = [&](int k) {
+      const int blocks = all * ((G + k - 1) / k);
+      return blocks <= (int)gridDim.x ? (blocks + ncu - 1) / ncu * k : 1 << 30;
+    };
+    if (fullest(2) < fullest(w)) w = 2;
+    if (fullest(1) < fullest(w)) w = 1;
+  }
+  const int n_ct = w == 1 ? G : w == 2 ? (G + 1) >> 1 : (G + 3) >> 2;
+  const int64_t total = (int64_t)all * n_ct;
   const int64_t run = (total + 7) >> 3;
-  const int64_t j = blockIdx.x >> 3;
   const int64_t entry = (int64_t)(blockIdx.x & 7) * run + j;
-  if (j >= run || entry >= total || entry > 0x7FFFFFFFll) return false;
+  if (wave >= w || j >= run || entry >= total || entry > 0x7FFFFFFFll) return false;
   const int trow = (int)((uint32_t)entry / (uint32_t)n_ct);
   const uint64_t hit = __ballot(before <= trow && trow < upto);
   if (!hit) return false;
   const int sel = __ffsll((unsigned long long)hit) - 1;
-  int rs = __builtin_amdgcn_readlane(start, sel);
-  int tc = __builtin_amdgcn_readlane(before, sel);
-  g = -1;
-  int szg = 0;
+  int rs = __builtin_amdgcn_readlane(v[0] - own[0], sel);  // first row of lane sel's first group
+  int tc = __builtin_amdgcn_readlane(before, sel);         // row tiles before it
+  int g = -1, szg = 0;
 #pragma unroll
   for (int i = 0; i < PL; ++i) {
     if (g < 0) {
       const int s = __builtin_amdgcn_readlane(sz[i], sel);
-      const int n = tiles_of(sel * PL + i, s);
+      const int n = tiles_of(sel * PL + i, s, lg);
       if (trow < tc + n) {
         g = sel * PL + i;
         szg = s;
@@ -94,24 +149,36 @@ __device__ __forceinline__ bool stream_tile(const int32_t *__restrict__ group_si
     }
   }
   if (g < 0) return false;
-  const uint32_t n = (uint32_t)tiles_of(g, szg), local = (uint32_t)entry - (uint32_t)tc * (uint32_t)n_ct;
+  const uint32_t n = (uint32_t)tiles_of(g, szg, lg), local = (uint32_t)entry - (uint32_t)tc * (uint32_t)n_ct;
   const int rt = (int)(local % n);
-  ct = (int)(local / n);
-  row0 = (int64_t)rs + (int64_t)rt * kStreamRows;
-  rows = min(szg - rt * kStreamRows, kStreamRows);
-  return true;
+  ref.g = g;
+  ref.cg = (int)(local / n) * w + wave;
+  ref.row0 = (int64_t)rs + ((int64_t)rt << lg);
+  ref.rows = min(szg - (rt << lg), 1 << lg);
+  ref.once = n == 1;
+  return ref.cg < G;
 }
 
+template <bool MX, int WPB>
 __device__ __forceinline__ bool find_stream_tile(const int32_t *__restrict__ group_sizes, int num_groups, int go,
-                                                 int64_t e_local, int64_t M, int n_ct, int &g, int64_t &row0,
-                                                 int &rows, int &ct) {
-  if (num_groups <= 64) return stream_tile<1>(group_sizes, num_groups, go, e_local, M, n_ct, g, row0, rows, ct);
-  if (num_groups <= 256) return stream_tile<4>(group_sizes, num_groups, go, e_local, M, n_ct, g, row0, rows, ct);
-  return stream_tile<kMaxGroups / 64>(group_sizes, num_groups, go, e_local, M, n_ct, g, row0, rows, ct);
+                                                 int64_t e_local, int64_t M, int G, int max_rt, int ncu, int wave,
+                                                 StreamRef &ref) {
+  if (num_groups <= 64) return stream_tile<1, MX, WPB>(group_sizes, num_groups, go, e_local, M, G, max_rt, ncu, wave, ref);
+  if (num_groups <= 256) return stream_tile<4, MX, WPB>(group_sizes, num_groups, go, e_local, M, G, max_rt, ncu, wave, ref);
+  return stream_tile<kMaxGroups / 64, MX, WPB>(group_sizes, num_groups, go, e_local, M, G, max_rt, ncu, wave, ref);
+}
+
+// NT: weights that no other row tile of the group reads stream past the caches
+// (the plain policy there: half of 1536 rows in one of 256 experts 512 -> 467
+// us, 384 Zipf rows over 64 experts 107 -> 100, both K = N = 4096; all rows in
+// one or a few experts lose 3-8%).
+template <bool NT>
+__device__ __forceinline__ u32x4_t load_weights(const u32x4_t *p) {
+  return NT ? __builtin_nontemporal_load(p) : *p;
 }
 
 // One row tile of NH 16-row blocks x the wave's 64 columns.
-template <int NH, int D, bool ACT>
+template <int NH, int D, bool NT, bool ACT>
 __device__ __forceinline__ void stream_columns(const uint16_t *__restrict__ lhs, const int32_t *__restrict__ row_idx,
                                                int64_t lhs_rows, int64_t row0, int rows, int K,
                                                const uint8_t *__restrict__ w, const uint8_t *__restrict__ s,
@@ -137,7 +204,7 @@ __device__ __forceinline__ void stream_columns(const uint16_t *__restrict__ lhs,
     const uint8_t *const sb = s + (int64_t)kb * 256;
     const uint8_t *const ab = abase + (int64_t)kb * 256;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) wr[d][i] = __builtin_nontemporal_load((const u32x4_t *)(wb + 1024 * i + woff));
+    for (int i = 0; i < 4; ++i) wr[d][i] = load_weights<NT>((const u32x4_t *)(wb + 1024 * i + woff));
 #pragma unroll
     for (int i = 0; i < 2; ++i) sr[d][i] = *(const uint32_t *)(sb + 64 * i + soff);
 #pragma unroll
@@ -208,43 +275,47 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(2))) v
     const uint16_t *__restrict__ lhs, const int32_t *__restrict__ row_idx, int64_t lhs_rows, int64_t M, int K,
     const uint8_t *__restrict__ wpk, const uint8_t *__restrict__ spk, const int32_t *__restrict__ group_sizes,
     int num_groups, const int32_t *__restrict__ group_offset, int64_t e_local, int N, void *__restrict__ out,
-    int out_f32, GmmEpilogue ep) {
+    int out_f32, GmmEpilogue ep, int max_rt, int ncu) {
   __shared__ __attribute__((aligned(16))) float s_ep[WPB][16 * 72];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int G = (N + 63) >> 6, n_ct = (G + WPB - 1) / WPB;
+  const int G = (N + 63) >> 6;
   const int go = group_offset ? group_offset[0] : 0;
-  int g, rows, ct;
-  int64_t row0;
-  if (!find_stream_tile(group_sizes, num_groups, go, e_local, M, n_ct, g, row0, rows, ct)) return;
-  const int cg = ct * WPB + wave;  // the wave's 64-column group
-  if (cg >= G) return;
-  const int64_t e = g - go;
+  StreamRef ref;
+  if (!find_stream_tile<false, WPB>(group_sizes, num_groups, go, e_local, M, G, max_rt, ncu, wave, ref)) return;
+  const int rows = ref.rows, cg = ref.cg;
+  const int64_t e = ref.g - go;
   const uint8_t *const w = wpk + (e * G + cg) * (int64_t)(K >> 6) * 2048;
   const uint8_t *const s = spk + (e * G + cg) * (int64_t)(K >> 7) * 256;
   const void *const bias = expert_bias(ep, e, N);
-  if (rows <= 16)
-    stream_columns<1, 4, ACT>(lhs, row_idx, lhs_rows, row0, rows, K, w, s, (int64_t)cg * 64, N, out, out_f32, bias,
-                              ep, s_ep[wave]);
-  else
-    stream_columns<2, 3, ACT>(lhs, row_idx, lhs_rows, row0, rows, K, w, s, (int64_t)cg * 64, N, out, out_f32, bias,
-                              ep, s_ep[wave]);
+#define DWM_COLUMNS(NH, D, NT)                                                                              \
+  stream_columns<NH, D, NT, ACT>(lhs, row_idx, lhs_rows, ref.row0, rows, K, w, s, (int64_t)cg * 64, N, out, \
+                                 out_f32, bias, ep, s_ep[wave])
+  if (rows <= 16) {
+    if (ref.once) DWM_COLUMNS(1, 4, true);
+    else DWM_COLUMNS(1, 4, false);
+  } else {
+    if (ref.once) DWM_COLUMNS(2, 3, true);
+    else DWM_COLUMNS(2, 3, false);
+  }
+#undef DWM_COLUMNS
 }
 
 // Grid of a streaming launch: four waves (256 columns) per block, or one
 // where the waves are few, so that every CU gets a block.
 struct StreamGrid {
   unsigned blocks;
-  int wpb;
+  int wpb, max_rt;
 };
 
 static int stream_grid(int64_t M, int64_t N, int64_t E_local, int num_groups, const char *what, StreamGrid &sg) {
   const int64_t G = (N + 63) / 64;
-  // Row tiles: every group that holds rows has at most one partial one.
-  const int64_t max_rt = M / kStreamRows + std::min(std::min(E_local, (int64_t)num_groups), M);
+  // Row tiles of 32 rows: every group that holds rows has at most one partial one.
+  const int64_t max_rt = M / 32 + std::min(std::min(E_local, (int64_t)num_groups), M);
   sg.wpb = max_rt * G >= 4096 ? 4 : 1;
   const int64_t grid = (max_rt * ((G + sg.wpb - 1) / sg.wpb) + 7) / 8 * 8;
   DWM_UNSUPPORTED_IF(grid > (1ll << 31) - 1, "%s: too many tiles (%lld)", what, (long long)grid);
   sg.blocks = (unsigned)grid;
+  sg.max_rt = (int)max_rt;
   return DWM_OK;
 }
 
@@ -258,7 +329,7 @@ int launch_gmm_stream(const uint16_t *lhs, const int32_t *row_idx, int64_t lhs_r
 #define DWM_STREAM(WPB, ACT)                                                                                     \
   hipLaunchKernelGGL((gmm_fp4_stream_kernel<WPB, ACT>), dim3(sg.blocks), dim3(64 * WPB), 0, st, lhs,            \
                      row_idx, lhs_rows, M, (int)K, weight, scale, group_sizes, num_groups, group_offset, E_local, \
-                     (int)N, out, out_f32, ep)
+                     (int)N, out, out_f32, ep, sg.max_rt, device_cu_count())
   if (gated) {
     if (sg.wpb == 4) DWM_STREAM(4, true);
     else DWM_STREAM(1, true);
@@ -276,7 +347,7 @@ int launch_gmm_stream(const uint16_t *lhs, const int32_t *row_idx, int64_t lhs_r
 // (gmm_mx.hip), so the results are theirs bit for bit.
 typedef __attribute__((ext_vector_type(8))) int i32x8_t;
 
-template <int D, bool ACT, bool F4>
+template <int D, bool NT, bool ACT, bool F4>
 __device__ __forceinline__ void mx_stream_columns(const uint8_t *__restrict__ lhs, const uint8_t *__restrict__ lsc,
                                                   const int32_t *__restrict__ row_idx, int64_t lhs_rows, int64_t row0,
                                                   int rows, int K, const uint8_t *__restrict__ w,
@@ -297,7 +368,7 @@ __device__ __forceinline__ void mx_stream_columns(const uint8_t *__restrict__ lh
   auto load = [&](int d, int kb) {
     const uint8_t *const wb = w + (int64_t)kb * 4096;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) wr[d][i] = __builtin_nontemporal_load((const u32x4_t *)(wb + 1024 * i + woff));
+    for (int i = 0; i < 4; ++i) wr[d][i] = load_weights<NT>((const u32x4_t *)(wb + 1024 * i + woff));
     sr[d] = *(const uint32_t *)(s + (int64_t)kb * 256 + soff);
     as[d] = *(const uint32_t *)(lsc + (int64_t)kb * 4 + asoff);
 #pragma unroll
@@ -351,21 +422,23 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(2))) v
     const uint8_t *__restrict__ lhs, const uint8_t *__restrict__ lsc, const int32_t *__restrict__ row_idx,
     int64_t lhs_rows, int64_t M, int K, const uint8_t *__restrict__ wpk, const uint8_t *__restrict__ spk,
     const int32_t *__restrict__ group_sizes, int num_groups, const int32_t *__restrict__ group_offset,
-    int64_t e_local, int N, void *__restrict__ out, int out_f32, GmmEpilogue ep) {
+    int64_t e_local, int N, void *__restrict__ out, int out_f32, GmmEpilogue ep, int max_rt, int ncu) {
   __shared__ __attribute__((aligned(16))) float s_ep[WPB][32 * 72];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int G = (N + 63) >> 6, n_ct = (G + WPB - 1) / WPB;
+  const int G = (N + 63) >> 6;
   const int go = group_offset ? group_offset[0] : 0;
-  int g, rows, ct;
-  int64_t row0;
-  if (!find_stream_tile(group_sizes, num_groups, go, e_local, M, n_ct, g, row0, rows, ct)) return;
-  const int cg = ct * WPB + wave;
-  if (cg >= G) return;
-  const int64_t e = g - go;
+  StreamRef ref;
+  if (!find_stream_tile<true, WPB>(group_sizes, num_groups, go, e_local, M, G, max_rt, ncu, wave, ref)) return;
+  const int rows = ref.rows, cg = ref.cg;
+  const int64_t e = ref.g - go;
   const uint8_t *const w = wpk + (e * G + cg) * (int64_t)(K >> 6) * 2048;
   const uint8_t *const s = spk + (e * G + cg) * (int64_t)(K >> 7) * 256;
-  mx_stream_columns<4, ACT, F4>(lhs, lsc, row_idx, lhs_rows, row0, rows, K, w, s, (int64_t)cg * 64, N, out, out_f32,
-                                expert_bias(ep, e, N), ep, s_ep[wave]);
+#define DWM_COLUMNS(NT)                                                                                          \
+  mx_stream_columns<4, NT, ACT, F4>(lhs, lsc, row_idx, lhs_rows, ref.row0, rows, K, w, s, (int64_t)cg * 64, N, \
+                                    out, out_f32, expert_bias(ep, e, N), ep, s_ep[wave])
+  if (ref.once) DWM_COLUMNS(true);
+  else DWM_COLUMNS(false);
+#undef DWM_COLUMNS
 }
 
 int launch_gmm_mx_stream(const uint8_t *lhs, const uint8_t *lhs_scale, const int32_t *row_idx, int64_t lhs_rows,
@@ -379,7 +452,7 @@ int launch_gmm_mx_stream(const uint8_t *lhs, const uint8_t *lhs_scale, const int
 #define DWM_STREAM(WPB, ACT, F4)                                                                                    \
   hipLaunchKernelGGL((gmm_mx_stream_kernel<WPB, ACT, F4>), dim3(sg.blocks), dim3(64 * WPB), 0, st, lhs, lhs_scale, \
                      row_idx, lhs_rows, M, (int)K, weight, scale, group_sizes, num_groups, group_offset, E_local,   \
-                     (int)N, out, out_f32, ep)
+                     (int)N, out, out_f32, ep, sg.max_rt, device_cu_count())
 #define DWM_STREAM_W(ACT, F4) \
   do {                        \
     if (sg.wpb == 4) DWM_STREAM(4, ACT, F4); \

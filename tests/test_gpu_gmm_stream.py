@@ -35,6 +35,13 @@ CASES = [
     (300, 1408, 1280, [1, 0, 0, 2], None, False, "gather"),
     (300, 128, 1040, [0, 1, 3, 0, 8], (7, 290), False, "f32"),
     (1024, 256, 128, [0, 0, 1], None, True, "gather"),
+    # four-wave blocks that run one (4 experts of 32 rows, 12 of 96) or two waves (24 x 64 column groups), 18 experts
+    # whose one-wave list would not fit the grid, and one large group among single rows (16-row tiles in two rounds)
+    (64, 256, 4096, [32] + [0] * 15, None, False, "none"),
+    (64, 128, 4096, [96] + [0] * 15, None, False, "gather"),
+    (128, 128, 4096, [192] + [0] * 31, None, True, "none"),
+    (64, 128, 4096, [7, 0, 0, 0, 0, 7, 0], None, False, "f32"),
+    (64, 256, 4096, [64] + [1] * 63, None, False, "none"),
 ]
 
 

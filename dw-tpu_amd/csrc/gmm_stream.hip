@@ -28,11 +28,11 @@
 namespace dwm {
 
 // The wave's tile: `rows` rows from row0 of group g, 64-column group cg;
-// once: no other row tile of the group reads the same weights.
+// stream: its weights are loaded with the streaming policy.
 struct StreamRef {
   int64_t row0;
   int g, rows, cg;
-  bool once;
+  bool stream;
 };
 
 // A block's first w waves take w adjacent 64-column groups of one row tile.
@@ -51,10 +51,11 @@ struct StreamRef {
 //
 // Row tiles hold 16 rows (MX: 32, its MFMA's) or 32.  With 16 the waves are
 // alike: while weights stream from HBM, a wave with twice the rows falls
-// behind and ends alone.  32 are taken where most tiles would share their
-// weights with another one anyway (few groups hold all rows: larger tiles
-// read less from L2), where only they fit one round of waves, and where 16
-// would not fit the grid.  Against 32 throughout, us: 384 rows over 64
+// behind and ends alone.  32 are taken in launches of at most half a round of
+// waves (64 Zipf rows over 8 experts, K = 3072, N = 4096 14.3 -> 12.8 us), where
+// most tiles would share their weights with another one anyway (few groups
+// hold all rows: larger tiles read less from L2), where only they fit one
+// round, and where 16 would not fit the grid.  Against 32 throughout, us: 384 rows over 64
 // experts by a Zipf law (1.1), K = N = 4096 100.5 -> 90.5; 192 such rows over
 // 32 experts, K = 2048, N = 7168 50.5 -> 44.0; 32 of 64 rows in one of 32
 // experts, K = 7168 101.5 -> 86.2.  Against 16 throughout: 1536 rows in one
@@ -63,7 +64,7 @@ struct StreamRef {
 // Blocks of four waves share their lhs rows through L1.  A launch of at most
 // one round takes one or two waves a block where that leaves fewer waves on
 // the fullest CU (128 rows in 4 of 64 experts, K = N = 4096 37.6 -> 15.5).
-template <int PL, bool MX, int WPB>
+template <int PL, bool R16, int WPB>
 __device__ __forceinline__ bool stream_tile(const int32_t *__restrict__ group_sizes, int num_groups, int go,
                                             int64_t e_local, int64_t M, int G, int max_rt, int ncu, int wave,
                                             StreamRef &ref) {
@@ -83,11 +84,11 @@ __device__ __forceinline__ bool stream_tile(const int32_t *__restrict__ group_si
     for (int i = 0; i < PL; ++i) {
       v[0] += sz[i];
       v[1] += tiles_of(lane * PL + i, sz[i], 5);
-      if (!MX) v[2] += tiles_of(lane * PL + i, sz[i], 4);
+      if (R16) v[2] += tiles_of(lane * PL + i, sz[i], 4);
     }
 #pragma unroll
     for (int a = 0; a < 3; ++a) own[a] = v[a];
-    wave_inclusive_scan_n<3>(v);  // (MX: v[2] is 0 and folds away)
+    wave_inclusive_scan_n<3>(v);
   };
 #pragma unroll
   for (int i = 0; i < PL; ++i) sz[i] = lane * PL + i < num_groups ? min(max(sz[i], 0), m32) : 0;
@@ -105,9 +106,9 @@ __device__ __forceinline__ bool stream_tile(const int32_t *__restrict__ group_si
     count();
   }
   const int64_t cap = 8 * (int64_t)ncu;  // waves of one round: 256 VGPRs each
-  const int all32 = wave_last(v[1]), all16 = MX ? 0 : wave_last(v[2]);
-  const bool small = !MX && all16 <= max_rt && 2 * (int64_t)all16 < 3 * (int64_t)all32 &&
-                     (all16 * (int64_t)G <= cap || all32 * (int64_t)G > cap);
+  const int all32 = wave_last(v[1]), all16 = R16 ? wave_last(v[2]) : 0;
+  const bool small = R16 && all16 <= max_rt && 2 * (int64_t)all16 < 3 * (int64_t)all32 &&
+                     2 * all32 * (int64_t)G > cap && (all16 * (int64_t)G <= cap || all32 * (int64_t)G > cap);
   const int lg = small ? 4 : 5, all = small ? all16 : all32;
   const int upto = small ? v[2] : v[1], before = upto - (small ? own[2] : own[1]);
   const int j = blockIdx.x >> 3;
@@ -155,23 +156,25 @@ __device__ __forceinline__ bool stream_tile(const int32_t *__restrict__ group_si
   ref.cg = (int)(local / n) * w + wave;
   ref.row0 = (int64_t)rs + ((int64_t)rt << lg);
   ref.rows = min(szg - (rt << lg), 1 << lg);
-  ref.once = n == 1;
+  ref.stream = n == 1 || all * (int64_t)G <= cap;
   return ref.cg < G;
 }
 
-template <bool MX, int WPB>
+template <bool R16, int WPB>
 __device__ __forceinline__ bool find_stream_tile(const int32_t *__restrict__ group_sizes, int num_groups, int go,
                                                  int64_t e_local, int64_t M, int G, int max_rt, int ncu, int wave,
                                                  StreamRef &ref) {
-  if (num_groups <= 64) return stream_tile<1, MX, WPB>(group_sizes, num_groups, go, e_local, M, G, max_rt, ncu, wave, ref);
-  if (num_groups <= 256) return stream_tile<4, MX, WPB>(group_sizes, num_groups, go, e_local, M, G, max_rt, ncu, wave, ref);
-  return stream_tile<kMaxGroups / 64, MX, WPB>(group_sizes, num_groups, go, e_local, M, G, max_rt, ncu, wave, ref);
+  if (num_groups <= 64) return stream_tile<1, R16, WPB>(group_sizes, num_groups, go, e_local, M, G, max_rt, ncu, wave, ref);
+  if (num_groups <= 256) return stream_tile<4, R16, WPB>(group_sizes, num_groups, go, e_local, M, G, max_rt, ncu, wave, ref);
+  return stream_tile<kMaxGroups / 64, R16, WPB>(group_sizes, num_groups, go, e_local, M, G, max_rt, ncu, wave, ref);
 }
 
-// NT: weights that no other row tile of the group reads stream past the caches
-// (the plain policy there: half of 1536 rows in one of 256 experts 512 -> 467
-// us, 384 Zipf rows over 64 experts 107 -> 100, both K = N = 4096; all rows in
-// one or a few experts lose 3-8%).
+// NT: the weights stream past the caches.  Not where other row tiles of the
+// group read them in a later round of waves (plain loads, K = N = 4096: half
+// of 1536 rows in one of 256 experts 512 -> 467 us, 384 Zipf rows over 64
+// experts 107 -> 100); within one round the tiles run side by side and share
+// them anyway, and plain loads lose (64 rows in one of 8 experts, K = 1024, N
+// = 2048 6.3 -> 7.1).
 template <bool NT>
 __device__ __forceinline__ u32x4_t load_weights(const u32x4_t *p) {
   return NT ? __builtin_nontemporal_load(p) : *p;
@@ -270,7 +273,7 @@ __device__ __forceinline__ void stream_columns(const uint16_t *__restrict__ lhs,
   store_halves<NH, ACT, 72>(acc, ep_lds, row0, rows, col0, N, out, out_f32, bias, ep.bias_bf16, ep.act);
 }
 
-template <int WPB, bool ACT>
+template <int WPB, bool R16, bool ACT>
 __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(2))) void gmm_fp4_stream_kernel(
     const uint16_t *__restrict__ lhs, const int32_t *__restrict__ row_idx, int64_t lhs_rows, int64_t M, int K,
     const uint8_t *__restrict__ wpk, const uint8_t *__restrict__ spk, const int32_t *__restrict__ group_sizes,
@@ -281,7 +284,7 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(2))) v
   const int G = (N + 63) >> 6;
   const int go = group_offset ? group_offset[0] : 0;
   StreamRef ref;
-  if (!find_stream_tile<false, WPB>(group_sizes, num_groups, go, e_local, M, G, max_rt, ncu, wave, ref)) return;
+  if (!find_stream_tile<R16, WPB>(group_sizes, num_groups, go, e_local, M, G, max_rt, ncu, wave, ref)) return;
   const int rows = ref.rows, cg = ref.cg;
   const int64_t e = ref.g - go;
   const uint8_t *const w = wpk + (e * G + cg) * (int64_t)(K >> 6) * 2048;
@@ -291,10 +294,10 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(2))) v
   stream_columns<NH, D, NT, ACT>(lhs, row_idx, lhs_rows, ref.row0, rows, K, w, s, (int64_t)cg * 64, N, out, \
                                  out_f32, bias, ep, s_ep[wave])
   if (rows <= 16) {
-    if (ref.once) DWM_COLUMNS(1, 4, true);
+    if (!R16 || ref.stream) DWM_COLUMNS(1, 4, true);
     else DWM_COLUMNS(1, 4, false);
   } else {
-    if (ref.once) DWM_COLUMNS(2, 3, true);
+    if (!R16 || ref.stream) DWM_COLUMNS(2, 3, true);
     else DWM_COLUMNS(2, 3, false);
   }
 #undef DWM_COLUMNS
@@ -326,16 +329,23 @@ int launch_gmm_stream(const uint16_t *lhs, const int32_t *row_idx, int64_t lhs_r
   StreamGrid sg;
   int rc = stream_grid(M, N, E_local, num_groups, "gmm_fp4", sg);
   if (rc != DWM_OK) return rc;
-#define DWM_STREAM(WPB, ACT)                                                                                     \
-  hipLaunchKernelGGL((gmm_fp4_stream_kernel<WPB, ACT>), dim3(sg.blocks), dim3(64 * WPB), 0, st, lhs,            \
+#define DWM_STREAM(WPB, R16, ACT)                                                                                \
+  hipLaunchKernelGGL((gmm_fp4_stream_kernel<WPB, R16, ACT>), dim3(sg.blocks), dim3(64 * WPB), 0, st, lhs,       \
                      row_idx, lhs_rows, M, (int)K, weight, scale, group_sizes, num_groups, group_offset, E_local, \
-                     (int)N, out, out_f32, ep, sg.max_rt, device_cu_count())
+                     (int)N, out, out_f32, ep, sg.max_rt, ncu)
+  // At most half a round of waves never takes 16-row tiles (stream_tile): it
+  // runs the kernel without that choice (0.2 us less search: 8 rows, K =
+  // 2048, N = 7168 12.3 -> 12.0).
+  const int ncu = device_cu_count();
+  const bool r16 = 2 * sg.max_rt * ((N + 63) / 64) > 8 * ncu;
   if (gated) {
-    if (sg.wpb == 4) DWM_STREAM(4, true);
-    else DWM_STREAM(1, true);
+    if (sg.wpb == 4) DWM_STREAM(4, true, true);
+    else if (r16) DWM_STREAM(1, true, true);
+    else DWM_STREAM(1, false, true);
   } else {
-    if (sg.wpb == 4) DWM_STREAM(4, false);
-    else DWM_STREAM(1, false);
+    if (sg.wpb == 4) DWM_STREAM(4, true, false);
+    else if (r16) DWM_STREAM(1, true, false);
+    else DWM_STREAM(1, false, false);
   }
 #undef DWM_STREAM
   return launch_status("gmm_fp4");
@@ -428,7 +438,7 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(2))) v
   const int G = (N + 63) >> 6;
   const int go = group_offset ? group_offset[0] : 0;
   StreamRef ref;
-  if (!find_stream_tile<true, WPB>(group_sizes, num_groups, go, e_local, M, G, max_rt, ncu, wave, ref)) return;
+  if (!find_stream_tile<false, WPB>(group_sizes, num_groups, go, e_local, M, G, max_rt, ncu, wave, ref)) return;
   const int rows = ref.rows, cg = ref.cg;
   const int64_t e = ref.g - go;
   const uint8_t *const w = wpk + (e * G + cg) * (int64_t)(K >> 6) * 2048;
@@ -436,7 +446,7 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(2))) v
 #define DWM_COLUMNS(NT)                                                                                          \
   mx_stream_columns<4, NT, ACT, F4>(lhs, lsc, row_idx, lhs_rows, ref.row0, rows, K, w, s, (int64_t)cg * 64, N, \
                                     out, out_f32, expert_bias(ep, e, N), ep, s_ep[wave])
-  if (ref.once) DWM_COLUMNS(true);
+  if (ref.stream) DWM_COLUMNS(true);
   else DWM_COLUMNS(false);
 #undef DWM_COLUMNS
 }

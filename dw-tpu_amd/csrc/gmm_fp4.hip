@@ -166,7 +166,7 @@ struct WsCfg {
 // Producer wave pw: NA of its A_LOADS lhs row groups hold rows of the tile;
 // the others are zero in every stage and never loaded.  It loads GL of the
 // tile's 64-column weight groups (G_LOADS in a wide tile, half in a narrow one),
-// their weights with cache policy AUX (kAuxStream or 0: launch_gmm_bf16).
+// their weights with cache policy AUX (kAuxStream or 0: gmm_fp4_ws_kernel).
 template <class C, int NA, int GL, int AUX>
 __device__ __forceinline__ void ws_producer(const uint16_t *__restrict__ lhs, const int32_t *__restrict__ row_idx,
                                             int64_t lhs_rows, int64_t row0, int rows, int K, int T,
@@ -521,6 +521,7 @@ __device__ __forceinline__ void ws_produce(int na, const uint16_t *lhs, const in
 
 // NARROW: the tile list may cut its costliest classes into 256-column tiles
 // (find_tile) when the 512-column tiles leave some of the ncu CUs idle.
+// AUX: cache policy of weights that no other row tile reads (kAuxStream or 0).
 template <class C, int MB, bool ACT, bool NARROW, int AUX>
 __global__ __launch_bounds__(C::THREADS) void gmm_fp4_ws_kernel(
     const uint16_t *__restrict__ lhs, const int32_t *__restrict__ row_idx, int64_t lhs_rows, int64_t M, int K,
@@ -579,10 +580,16 @@ __global__ __launch_bounds__(C::THREADS) void gmm_fp4_ws_kernel(
     const uint8_t *const sexp = spk + e * G * KB * 256;
     // Row groups pw + NP i with 8 (pw + NP i) < rows are loaded.
     const int na = min(C::A_LOADS, (rows + 8 * C::NPROD - 1 - 8 * pw) / (8 * C::NPROD));
-    if (NARROW && narrow)
-      ws_produce<C, C::G_LOADS / 2, AUX>(na, lhs, row_idx, lhs_rows, row0, rows, K, T, KB, wexp, sexp, g0, G, s_lds, pw);
-    else
-      ws_produce<C, C::G_LOADS, AUX>(na, lhs, row_idx, lhs_rows, row0, rows, K, T, KB, wexp, sexp, g0, G, s_lds, pw);
+    auto produce = [&](auto gl_c, auto aux_c) {
+      ws_produce<C, decltype(gl_c)::value, decltype(aux_c)::value>(na, lhs, row_idx, lhs_rows, row0, rows, K, T, KB,
+                                                                   wexp, sexp, g0, G, s_lds, pw);
+    };
+    auto by_policy = [&](auto gl_c) {
+      if (AUX != 0 && ref.once) produce(gl_c, IntC<AUX>{});
+      else produce(gl_c, IntC<0>{});
+    };
+    if (NARROW && narrow) by_policy(IntC<C::G_LOADS / 2>{});
+    else by_policy(IntC<C::G_LOADS>{});
     DWM_GS(gs_role(1u | (uint64_t)rows << 8 | (uint64_t)narrow << 24);)
     tl_exit();
     return;
@@ -743,7 +750,7 @@ int launch_gmm_bf16(const uint16_t *lhs, const int32_t *row_idx, int64_t lhs_row
                                                  num_groups, group_offset, E_local, N, out, out_f32, ep, ncu, \
                                                  balanced_tiles(), st)
 #define DWM_GMM_WS_AUX(ACT, NARROW) \
-  (weights_read_once(M, E_local) ? DWM_GMM_WS(ACT, NARROW, kAuxStream) : DWM_GMM_WS(ACT, NARROW, 0))
+  (launch_streams_weights(M, E_local) ? DWM_GMM_WS(ACT, NARROW, kAuxStream) : DWM_GMM_WS(ACT, NARROW, 0))
   if (gated) return narrow ? DWM_GMM_WS_AUX(true, true) : DWM_GMM_WS_AUX(true, false);
   return narrow ? DWM_GMM_WS_AUX(false, true) : DWM_GMM_WS_AUX(false, false);
 #undef DWM_GMM_WS_AUX

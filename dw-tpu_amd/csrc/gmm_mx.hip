@@ -174,10 +174,11 @@ __global__ __launch_bounds__(256) void mx_quant_e2m1_kernel(const uint16_t *__re
 // AF4: the lhs is e2m1 (MXFP4: 32 bytes per row and 64-deep step, one
 // 16-byte A operand per lane, A format 4 in the MFMA) instead of e4m3 (64
 // bytes per row and step).
-// WAUX: cache policy of the weight loads (kAuxStream or 0).
+// WAUX: cache policy of weights that no other row tile reads (kAuxStream or 0).
 template <int MB, int CW, int NP, int NS, int RH, bool AF4, int WAUX>
 struct MxCfg {
   static constexpr int AUX = WAUX;
+  using Plain = MxCfg<MB, CW, NP, NS, RH, AF4, 0>;
   static constexpr int CONS = CW, NPROD = NP, STAGES = NS, HALVES = RH;
   static constexpr bool A_FP4 = AF4;
   static constexpr int GT = CW / RH;                     // 64-column groups per tile
@@ -480,7 +481,11 @@ __global__ __launch_bounds__(C::THREADS) void gmm_mx_kernel(
     int na = 0;
     for (int ga = pw; ga < C::A_GROUPS; ga += NP) na += C::RL * ga < rows ? 1 : 0;
     const bool asl = pw >= NP - C::AS_LOADS;
-    mx_produce<C>(na, asl, lhs, lsc, row_idx, lhs_rows, row0, rows, K, T, KB, wexp, sexp, g0, G, s_lds, pw);
+    if (C::AUX != 0 && !ref.once)
+      mx_produce<typename C::Plain>(na, asl, lhs, lsc, row_idx, lhs_rows, row0, rows, K, T, KB, wexp, sexp, g0, G,
+                                    s_lds, pw);
+    else
+      mx_produce<C>(na, asl, lhs, lsc, row_idx, lhs_rows, row0, rows, K, T, KB, wexp, sexp, g0, G, s_lds, pw);
     return;
   }
   const int cg = wave % C::GT, rb = 32 * CMB * (wave / C::GT);
@@ -515,6 +520,7 @@ __global__ __launch_bounds__(C::THREADS) void gmm_mx_kernel(
 template <int MB, int CW, int NP, int NS, bool AF4, int WAUX>
 struct Mx128Cfg {
   static constexpr int AUX = WAUX;
+  using Plain = Mx128Cfg<MB, CW, NP, NS, AF4, 0>;
   static constexpr int CONS = CW, NPROD = NP, STAGES = NS;
   static constexpr bool A_FP4 = AF4;
   static constexpr int GT = CW;
@@ -737,9 +743,13 @@ __global__ __launch_bounds__(C::THREADS) void gmm_mx128_kernel(
     for (int ga = pw; ga < C::A_GROUPS; ga += NP) na += C::RL * ga < rows ? 1 : 0;
     const bool asl = pw >= NP - C::AS_LOADS;
     auto run = [&](auto na_c, auto asl_c) {
-      mx128_producer<C, (decltype(na_c)::value < C::A_LOADS ? decltype(na_c)::value : C::A_LOADS),
-                     decltype(asl_c)::value != 0>(lhs, lsc, row_idx, lhs_rows, row0, rows, K, T, wexp, sexp, g0, G,
-                                                  s_lds, pw);
+      constexpr int NA = decltype(na_c)::value < C::A_LOADS ? decltype(na_c)::value : C::A_LOADS;
+      constexpr bool ASL = decltype(asl_c)::value != 0;
+      if (C::AUX != 0 && !ref.once)
+        mx128_producer<typename C::Plain, NA, ASL>(lhs, lsc, row_idx, lhs_rows, row0, rows, K, T, wexp, sexp, g0, G,
+                                                   s_lds, pw);
+      else
+        mx128_producer<C, NA, ASL>(lhs, lsc, row_idx, lhs_rows, row0, rows, K, T, wexp, sexp, g0, G, s_lds, pw);
     };
     static_assert(C::A_LOADS <= 3, "at most three lhs row groups per producer");
     if (asl) {
@@ -803,7 +813,7 @@ static int launch_mx_form(const uint8_t *lhs, const uint8_t *lhs_scale, const in
   using S1 = MxCfg<3, 8, 4, 5, 1, AF4, kAuxStream>;
   const bool deep = K >= kMx128MinK;
   const bool halves = !deep && M > 96 * E_local && M <= 192 * E_local;
-  const bool once = weights_read_once(M, E_local);
+  const bool once = launch_streams_weights(M, E_local);
 #define DWM_MX(CFG, TMB, DEEP)                                                                                    \
   launch_mx<CFG, TMB, ACT, DEEP>(lhs, lhs_scale, row_idx, lhs_rows, M, K, weight, scale, group_sizes, num_groups, \
                                  group_offset, E_local, N, out, out_f32, ep, st)

@@ -86,12 +86,13 @@ __device__ __forceinline__ void tile_classes(const int32_t *group_sizes, int num
 }
 
 // The block's tile: (local group g, rows row0 .. row0 + rows - 1) x column
-// tile nt, of the wide tile width, or of half of it when `narrow`.
+// tile nt, of the wide tile width, or of half of it when `narrow`; `once`:
+// no other row tile of the group reads the same weights.
 struct TileRef {
-  int g, rows, nt, narrow;
+  int g, rows, nt, narrow, once;
   int64_t row0;
 };
-constexpr int kTileInfo = 5;  // s_info: g (-1: no tile), row0, rows, nt, narrow
+constexpr int kTileInfo = 6;  // s_info: g (-1: no tile), row0, rows, nt, narrow, once
 
 // The block's work-list entry from the class totals tot(a) (see find_tile):
 // the narrow split, then the class `cls` (-1: no tile) of block (xcd, j),
@@ -142,11 +143,12 @@ __device__ __forceinline__ void class_entry(Tot tot, int n_tiles, int n_tiles_n,
 
 // Rows and column tile of entry `entry` (row tile trow of class cls) in
 // group g of sz rows starting at row rs, whose class-cls row tiles start at
-// cs_g in the class's list.  s_info[1 .. 3] = row0, rows, nt.
+// cs_g in the class's list.  s_info[1 .. 3] = row0, rows, nt; s_info[5] = once.
 template <int MT, int CG>
 __device__ __forceinline__ void tile_rows(int sz, int rs, int cs_g, int cls, int trow, int64_t entry, int per_row,
                                           int bal, int *s_info) {
   const RowSplit<MT, CG> sp(sz, bal);
+  s_info[5] = sp.n == 1;
   if (sp.bal) {
     // (column tile, row tile) with the row tile innermost; tile tt starts
     // after tt * base + min(tt, extra) blocks.
@@ -266,6 +268,7 @@ __device__ __forceinline__ bool find_tile(const int32_t *__restrict__ group_size
   if (ref.g < 0) return false;
   ref.nt = s_info[3];
   ref.narrow = s_info[4];
+  ref.once = s_info[5];
   ref.row0 = s_info[1];
   // group_sizes lives on the device and is not checked by the host: sizes
   // whose sum leaves int32 would give row starts outside [0, M).  Such tiles
@@ -452,10 +455,13 @@ __device__ __forceinline__ void store_halves(const f32x4_t (&acc)[NH][4], float 
 // the 96-row tiles, K = 7168, N = 4096: 512 rows over 32 experts 95.0 -> 83.6
 // us, 1024 rows 102.9 -> 92.8; where two row tiles of an expert share its
 // weights the hint costs (128 rows per expert, K = 2048, N = 7168 146.6 ->
-// 152.3 us; 65536 rows 2.94 -> 3.03 ms), so it is used while the average
-// expert has fewer rows than a tile by a margin for uneven groups.
+// 152.3 us; 65536 rows 2.94 -> 3.03 ms).  A launch uses it while the average
+// expert has fewer rows than a tile by a margin for uneven groups, and in it
+// the tiles whose group has no other row tile (TileRef::once; for every tile
+// the MX tiles lost 25-50% on 192 .. 512 rows in one of 8 experts, K = 3072,
+// N = 4096: e2m1 23.5 -> 35.8 us).
 constexpr int kAuxStream = 2;
-inline bool weights_read_once(int64_t M, int64_t E_local) { return M <= 72 * E_local; }
+inline bool launch_streams_weights(int64_t M, int64_t E_local) { return M <= 72 * E_local; }
 
 // Epilogue inputs every gmm kernel passes through to store_tile.
 struct GmmEpilogue {

@@ -76,41 +76,29 @@ __device__ __forceinline__ bool stream_tile(const int32_t *__restrict__ group_si
   auto tiles_of = [&](int gi, int s, int lg) {
     return gi >= go && (int64_t)gi < (int64_t)go + e_local ? (s >> lg) + ((s & ((1 << lg) - 1)) != 0 ? 1 : 0) : 0;
   };
-  int v[3] = {0, 0, 0}, own[3];  // rows, row tiles of 32 rows, of 16
-  auto count = [&]() {
+  int rows_in = 0, v[2] = {0, 0};  // row tiles of 32 rows, of 16
 #pragma unroll
-    for (int a = 0; a < 3; ++a) v[a] = 0;
-#pragma unroll
-    for (int i = 0; i < PL; ++i) {
-      v[0] += sz[i];
-      v[1] += tiles_of(lane * PL + i, sz[i], 5);
-      if (R16) v[2] += tiles_of(lane * PL + i, sz[i], 4);
-    }
-#pragma unroll
-    for (int a = 0; a < 3; ++a) own[a] = v[a];
-    wave_inclusive_scan_n<3>(v);
-  };
-#pragma unroll
-  for (int i = 0; i < PL; ++i) sz[i] = lane * PL + i < num_groups ? min(max(sz[i], 0), m32) : 0;
-  count();
-  if (__ballot(v[0] < 0 || v[0] > m32) != 0) {
-    // A sum past int32 turns negative there: the lanes after it are past M.
-    const uint64_t neg = __ballot(v[0] < 0);
-    const int start = v[0] - own[0];
-    int left = neg != 0 && lane >= __ffsll((unsigned long long)neg) ? 0 : max(m32 - start, 0);
-#pragma unroll
-    for (int i = 0; i < PL; ++i) {
-      sz[i] = min(sz[i], left);
-      left -= sz[i];
-    }
-    count();
+  for (int i = 0; i < PL; ++i) {
+    sz[i] = lane * PL + i < num_groups ? min(max(sz[i], 0), m32) : 0;
+    rows_in += sz[i];
   }
+  const int start = wave_inclusive_scan(rows_in) - rows_in;  // first row of the lane's first group
+  int left = start >= 0 ? max(m32 - start, 0) : 0;           // (a sum past int32 is past M too)
+#pragma unroll
+  for (int i = 0; i < PL; ++i) {
+    sz[i] = min(sz[i], left);
+    left -= sz[i];
+    v[0] += tiles_of(lane * PL + i, sz[i], 5);
+    if (R16) v[1] += tiles_of(lane * PL + i, sz[i], 4);
+  }
+  const int own[2] = {v[0], v[1]};
+  wave_inclusive_scan_n<2>(v);
   const int64_t cap = 8 * (int64_t)ncu;  // waves of one round: 256 VGPRs each
-  const int all32 = wave_last(v[1]), all16 = R16 ? wave_last(v[2]) : 0;
+  const int all32 = wave_last(v[0]), all16 = R16 ? wave_last(v[1]) : 0;
   const bool small = R16 && all16 <= max_rt && 2 * (int64_t)all16 < 3 * (int64_t)all32 &&
                      2 * all32 * (int64_t)G > cap && (all16 * (int64_t)G <= cap || all32 * (int64_t)G > cap);
   const int lg = small ? 4 : 5, all = small ? all16 : all32;
-  const int upto = small ? v[2] : v[1], before = upto - (small ? own[2] : own[1]);
+  const int upto = small ? v[1] : v[0], before = upto - (small ? own[1] : own[0]);
   const int j = blockIdx.x >> 3;
   if (j >= (all * (int64_t)G + 7) >> 3) return false;  // past the run of every w
   int w = WPB;
@@ -132,7 +120,7 @@ __device__ __forceinline__ bool stream_tile(const int32_t *__restrict__ group_si
   const uint64_t hit = __ballot(before <= trow && trow < upto);
   if (!hit) return false;
   const int sel = __ffsll((unsigned long long)hit) - 1;
-  int rs = __builtin_amdgcn_readlane(v[0] - own[0], sel);  // first row of lane sel's first group
+  int rs = __builtin_amdgcn_readlane(start, sel);  // first row of lane sel's first group
   int tc = __builtin_amdgcn_readlane(before, sel);         // row tiles before it
   int g = -1, szg = 0;
 #pragma unroll

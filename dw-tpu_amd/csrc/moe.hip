@@ -4,7 +4,7 @@
 // one_hot(...).sum(0) (patches/tpu-inference-ext/0405-moe-fast-dispatch.patch:70-98,
 // kernels/tpu_inference/layers/common/moe_fast_dispatch.py:41-44) with a
 // counting sort that is bit-exact to a stable argsort, in three launches
-// (one launch for batches of up to kWideMax ids, dispatch_wide_kernel):
+// (one launch for most batches of up to kWideMax ids, dispatch_wide_kernel):
 //   1. per 1024-id chunk, an LDS histogram -> counts[chunk][expert]
 //   2. one block: group sizes, exclusive offsets, per-(chunk, expert) bases
 //   3. per chunk, in id order (256 ids per step, wave by wave): each lane's
@@ -168,29 +168,44 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_kernel(
 
 // Up to kWideMax ids in one launch: block b of 1024 threads counts all n ids
 // by key in LDS (those before its portion and the rest apart; every block
-// reads the ids from L2), scans the totals, and places its own 1024 ids.
+// reads the ids from L2), scans the totals, and places its own 1024 ids.  One
+// block needs no count: the portion is the batch.
 // What bounds three launches (count, scan, scatter) is their latency, not
 // their work: 24576 ids over 256 experts took 3.9 + 6.5 + 6.4 us and the gaps
-// between them, this kernel one launch.  The repeated count grows with n (64
-// LDS atomics per thread at kWideMax), so larger batches keep the three.
+// between them, this kernel one launch.  The repeated count grows with n and
+// serialises on a hot key (LDS atomics of one wave on one address), so past
+// 8192 ids the counters have 4 copies, from 24576 on 8.  Three launches ->
+// this one, us, even ids / all ids on one expert:
+//   256 experts: 24576 ids 13.8 / 13.9 -> 8.7 / 10.4, 65536 19.3 / 19.2 -> 14.8 / 14.0;
+//   32 experts: 24576 10.7 / 11.0 -> 7.2 / 9.5, 49152 10.8 / 11.2 -> 10.7 / 10.7, 65536 11.2 / 11.6 -> 12.8 / 12.9;
+// (with one copy 65536 hot ids took 58 us), so under 128 experts batches past
+// kWideFew ids keep the three launches, as all do past kWideMax.
 // Few experts and few ids take dispatch_small_kernel below.
-constexpr int kFusedThreads = 1024, kSmallMax = 8192, kWideMax = 65536;
+constexpr int kFusedThreads = 1024, kSmallMax = 8192, kWideFew = 49152, kWideMax = 65536;
+constexpr int kWideCounters = 4112;  // 8 copies of up to 512 keys, 4 of 1025
 
 __global__ __launch_bounds__(kFusedThreads) void dispatch_wide_kernel(const int32_t *ids, int64_t n, int topk, int E,
                                                                       int32_t *perm, int32_t *tok_sorted,
                                                                       int32_t *revert, int32_t *group_sizes,
                                                                       int32_t *group_offsets, int32_t *flags) {
   constexpr int W = kFusedThreads / 64, U = 8;
-  __shared__ int s_bef[kMaxExperts + 1];      // ids of each key before the portion, then the portion's first position
-  __shared__ int s_rest[kMaxExperts + 1];     // the other ids of each key
+  // Ids of each key before the portion (then the portion's first position) and
+  // the other ids of each key, in `copies` copies.
+  __shared__ int s_bef[kWideCounters], s_rest[kWideCounters];
   __shared__ int s_wcnt[W][kMaxExperts + 1];  // the portion's count of each key per wave
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  for (int e = tid; e <= E; e += kFusedThreads) {
-    s_bef[e] = 0;
-    s_rest[e] = 0;
-#pragma unroll
-    for (int w = 0; w < W; ++w) s_wcnt[w][e] = 0;
+  // Copies of the counters, lane % copies counting in its own: an odd stride
+  // apart, so that one key's copies lie in different banks.
+  const int stride = (E + 1) | 1;
+  int copies = n <= kSmallMax ? 1 : n <= 24576 ? 4 : 8;
+  while (copies * stride > kWideCounters) copies >>= 1;
+  const bool many = gridDim.x > 1;
+  const int waves = many ? W : ((int)n + 63) >> 6;  // that hold ids
+  if (many) {
+    for (int e = tid; e < stride * copies; e += kFusedThreads) s_bef[e] = s_rest[e] = 0;
   }
+  for (int e = tid; e <= E; e += blockDim.x)
+    for (int w = 0; w < waves; ++w) s_wcnt[w][e] = 0;
   const int64_t base = (int64_t)blockIdx.x * kFusedThreads, j = base + tid;
   const bool active = j < n;
   bool bad = false;
@@ -206,21 +221,44 @@ __global__ __launch_bounds__(kFusedThreads) void dispatch_wide_kernel(const int3
   const int rank = __popcll(peers & ((1ull << lane) - 1ull));
   __syncthreads();
   if (active && rank == 0) s_wcnt[wave][key] = __popcll(peers);
-  for (int64_t j0 = 0; j0 < n; j0 += U * kFusedThreads) {
-    int id[U];
+  if (many) {
+    const int copy = (lane & (copies - 1)) * stride;
+    for (int64_t j0 = 0; j0 < n; j0 += U * kFusedThreads) {
+      int id[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {  // the loads of a round side by side
-      const int64_t i = j0 + u * kFusedThreads + tid;
-      id[u] = i < n ? ids[i] : 0;
-    }
+      for (int u = 0; u < U; ++u) {  // the loads of a round side by side
+        const int64_t i = j0 + u * kFusedThreads + tid;
+        id[u] = i < n ? ids[i] : 0;
+      }
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t i0 = j0 + u * kFusedThreads;
-      if (i0 + tid < n) atomicAdd(i0 < base ? &s_bef[dispatch_key(id[u], E, &bad)] : &s_rest[dispatch_key(id[u], E, &bad)], 1);
+      for (int u = 0; u < U; ++u) {
+        const int64_t i0 = j0 + u * kFusedThreads;
+        if (i0 + tid < n) atomicAdd((i0 < base ? s_bef : s_rest) + copy + dispatch_key(id[u], E, &bad), 1);
+      }
     }
   }
   if (bad && flags && blockIdx.x == 0) atomicOr(flags, 1);
   __syncthreads();
+  if (!many) {
+    for (int e = tid; e <= E; e += blockDim.x) {
+      int r = 0;
+      for (int w = 0; w < waves; ++w) r += s_wcnt[w][e];
+      s_bef[e] = 0;
+      s_rest[e] = r;
+    }
+    __syncthreads();
+  } else if (copies > 1) {
+    for (int e = tid; e <= E; e += kFusedThreads) {
+      int b = s_bef[e], r = s_rest[e];
+      for (int c = 1; c < copies; ++c) {
+        b += s_bef[c * stride + e];
+        r += s_rest[c * stride + e];
+      }
+      s_bef[e] = b;
+      s_rest[e] = r;
+    }
+    __syncthreads();
+  }
   if (wave == 0) {
     int carry = 0;
     for (int b = 0; b <= E; b += 64) {
@@ -562,10 +600,14 @@ static int dispatch_launch(const int32_t *topk_ids, int64_t n, int topk, int num
                        num_experts, perm, tok_sorted, revert, group_sizes, group_offsets, flags);
     return launch_status("moe_dispatch");
   }
-  if (n <= kWideMax) {
-    hipLaunchKernelGGL(dispatch_wide_kernel, dim3((unsigned)((n + kFusedThreads - 1) / kFusedThreads)),
-                       dim3(kFusedThreads), 0, st, topk_ids, n, topk, num_experts, perm, tok_sorted, revert,
-                       group_sizes, group_offsets, flags);
+  // (Without counters there is only this kernel: dwm_moe_dispatch_noalloc.)
+  if (n <= kWideMax && (!counts || n <= kWideFew || num_experts >= 128)) {
+    // One block: no more waves than the ids or the keys need.
+    const unsigned blocks = (unsigned)((n + kFusedThreads - 1) / kFusedThreads);
+    const int64_t most = n > num_experts + 1 ? n : num_experts + 1;
+    const unsigned threads = blocks > 1 || most >= kFusedThreads ? kFusedThreads : (unsigned)((most + 63) / 64 * 64);
+    hipLaunchKernelGGL(dispatch_wide_kernel, dim3(blocks), dim3(threads), 0, st, topk_ids, n, topk, num_experts, perm,
+                       tok_sorted, revert, group_sizes, group_offsets, flags);
     return launch_status("moe_dispatch");
   }
   hipLaunchKernelGGL(dispatch_count_kernel, dim3((unsigned)nchunks), dim3(kDispThreads), 0, st,
@@ -661,8 +703,8 @@ extern "C" int dwm_moe_dispatch_noalloc(const int32_t *topk_ids, int64_t T, int 
                      "moe_dispatch_noalloc: %lld ids over %d experts need %lld counter words, more than the "
                      "%lld of its static scratch (use dwm_moe_dispatch with a workspace)",
                      (long long)n, num_experts, (long long)words, (long long)kNoAllocWords);
-  // Only the three-launch path (n > kWideMax) uses the counters: smaller
-  // batches never look the array up, so their first call on a device does
+  // Only batches past kWideMax use the counters here: smaller
+  // ones never look the array up, so their first call on a device does
   // no runtime lookup (e.g. inside a stream capture).
   int32_t *counts = nullptr;
   if (n > kWideMax) {

@@ -1,8 +1,9 @@
 """The one-launch dispatch over several blocks (dispatch_wide_kernel in
 csrc/moe.hip) and its neighbours, bit for bit against a stable argsort:
-portions of 1024 ids, the rounds of 8192 ids each block counts, the largest
-batch of one launch (65536 ids), the three launches above it, and ids outside
-the experts."""
+portions of 1024 ids (one portion in a block of fewer waves), the rounds of
+8192 ids each block counts, 1, 4 and 8 copies of the counters, the largest
+batches of one launch (49152 ids under 128 experts, else 65536), the three
+launches above them, and ids outside the experts."""
 import numpy as np
 import pytest
 import torch
@@ -14,7 +15,9 @@ pytestmark = pytest.mark.gpu
     (1, 1, 64), (341, 3, 64), (512, 2, 256), (205, 5, 1024),    # 1, 1023, 1024 and 1025 ids
     (4096, 2, 63), (8193, 1, 63), (8193, 1, 64), (1365, 6, 256),  # 8192 ids over few experts, 8193, 8190
     (4096, 6, 256), (5461, 12, 8), (8192, 8, 1024),              # 24576, 65532 and 65536 ids
-    (65537, 1, 100), (9000, 8, 32),                              # past one launch
+    (8192, 3, 1024), (8192, 3, 128), (24577, 1, 300), (200, 2, 70),  # 24576 and 24577 ids; 400
+    (49152, 1, 64), (49153, 1, 64), (49153, 1, 128),             # both sides of the limit under 128 experts
+    (65537, 1, 100), (65537, 1, 1024), (9000, 8, 32),            # past one launch
 ])
 @pytest.mark.parametrize("skew", [False, True])
 def test_dispatch_is_a_stable_argsort(dev, T, topk, E, skew):

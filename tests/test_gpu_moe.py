@@ -17,18 +17,19 @@ def _dispatch(dev, ids, E, check=False):
     return [t.cpu().numpy() for t in d]
 
 
-# Batches of up to 8192 ids take a one-block kernel (with at most 63
-# experts the register-count kernel, E = 63 and a ragged last round here;
-# with more the LDS-histogram one, E = 64 here), larger ones the
-# three-launch path: both sides of each boundary are covered.  In the
-# three-launch path the scan splits the chunk counters into runs per expert
-# column (E + 1 <= 512 columns: 2 .. 1024 runs), or walks whole columns
-# (E = 1024: more columns than the scan's threads).
+# Batches of up to 8192 ids over at most 63 experts take the register-count
+# kernel (E = 63 and a ragged last round here), others of up to 65536 ids (49152
+# under 128 experts) the one-launch kernel, larger ones the three launches: both
+# sides of each boundary are covered.  In the three launches the scan splits
+# the chunk counters into runs per expert column (E + 1 <= 512 columns: 65 or
+# more chunks in up to 1024 runs), or walks whole columns (E = 1024: more
+# columns than the scan's threads).
 @pytest.mark.parametrize("T,topk,E", [(1, 1, 1), (3, 2, 8), (64, 2, 8), (256, 8, 32), (512, 8, 32),
                                       (1000, 6, 256), (8192, 8, 32), (130, 8, 1024), (4096, 1, 3),
                                       (1024, 8, 1024), (8192, 1, 5), (8193, 1, 7), (2731, 3, 64),
                                       (2048, 8, 1024), (16384, 8, 256), (65536, 8, 32), (9000, 1, 1),
-                                      (1000, 5, 63), (700, 8, 64), (1, 7, 2), (8191, 1, 1)])
+                                      (1000, 5, 63), (700, 8, 64), (1, 7, 2), (8191, 1, 1), (8200, 8, 1024), (8200, 8, 256),
+                                      (65537, 1, 1), (49153, 1, 3), (7000, 7, 127), (7000, 9, 128)])
 def test_dispatch_bit_exact(dev, rng, T, topk, E):
     ids = rng.integers(0, E, (T, topk)).astype(np.int32)
     got = _dispatch(dev, ids, E)
@@ -64,14 +65,15 @@ def test_dispatch_skewed_and_invalid_ids(dev, rng):
     assert gs.sum() == valid.sum() and off[-1] == valid.sum()
     assert set(perm[off[-1]:]) == set(np.nonzero(~valid)[0])  # invalid ids last
     assert np.array_equal(perm[rev], np.arange(bad.size))
-    # the same on the three-launch path (more than 8192 ids): invalid ids sort
-    # as one extra key E after every valid one, stably
-    big = rng.integers(0, 8, (3000, 3)).astype(np.int32)
-    big[5, 2], big[2999, 0], big[1500, 1] = 8, -3, 100
-    got = _dispatch(dev, big, 8)
-    perm, tok, rev, gs, off = moe.dispatch(np.where((big >= 0) & (big < 8), big, 8), 9)
-    for g, w in zip(got, (perm, tok, rev, gs[:8], off[:9])):
-        assert np.array_equal(g, w)
+    # the same in the one-launch kernel (9000 ids) and the three launches (66000):
+    # invalid ids sort as one extra key E after every valid one, stably
+    for T in (3000, 22000):
+        big = rng.integers(0, 8, (T, 3)).astype(np.int32)
+        big[5, 2], big[2999, 0], big[1500, 1] = 8, -3, 100
+        got = _dispatch(dev, big, 8)
+        perm, tok, rev, gs, off = moe.dispatch(np.where((big >= 0) & (big < 8), big, 8), 9)
+        for g, w in zip(got, (perm, tok, rev, gs[:8], off[:9])):
+            assert np.array_equal(g, w)
 
 
 @pytest.mark.parametrize("T,H,dtype", [(64, 1024, torch.bfloat16), (513, 7168, torch.bfloat16),

@@ -1,8 +1,8 @@
 """dwm_moe_dispatch_noalloc (the dispatch without a workspace or any
 allocation) through the C ABI against dwm_moe_dispatch with a workspace:
-bit-identical outputs on two calls in a row, the second smaller, both on
-the three-launch path that uses the static counters; and the size limit
-rejected on the host before any device work."""
+bit-identical outputs on calls in a row, each smaller than the one before, the
+first two on the three launches that use the static counters (more than 65536
+ids); and the size limit rejected on the host before any device work."""
 import ctypes
 
 import numpy as np
@@ -37,7 +37,8 @@ def _dispatch(ids, T, topk, E, dev, noalloc):
 def test_noalloc_dispatch_matches_workspace_dispatch(dev):
     rng = np.random.default_rng(11)
     E, topk = 256, 8
-    for T in (6000, 1500):  # 48000 then 12000 ids: both above the one-block path
+    # 96000 then 72000 ids: three launches on the static counters; 48000 and 12000: one launch
+    for T in (12000, 9000, 6000, 1500):
         ids_np = rng.integers(0, E, (T, topk)).astype(np.int32)
         ids_np[0, 0] = E + 3  # an invalid id: flagged and ordered last
         ids = torch.from_numpy(ids_np).to(dev)
@@ -69,16 +70,17 @@ def test_noalloc_dispatch_under_graph_capture(dev):
     ids copied in, eager work and synchronisations between the replays; every
     replay bit-identical to dwm_moe_dispatch with a workspace.  The 2048-id
     batch is captured with no earlier no-alloc call of its size class (it
-    never looks the static array up); the 20,000-id batch (three launches
-    on the static counters) is captured after one eager call, as the header
-    asks of batches above 8192 ids."""
+    never looks the static array up), and so are the 20,000-id one and, over
+    few experts, one of 60,000 ids, all of one launch; the 70,000-id batch
+    (three launches on the static counters) is captured after one eager call,
+    as the header asks of batches above 65536 ids."""
     rng = np.random.default_rng(5)
-    for T, topk, E in ((256, 8, 32), (2500, 8, 256)):
+    for T, topk, E in ((256, 8, 32), (2500, 8, 256), (7500, 8, 32), (8750, 8, 256)):
         n = T * topk
         ids = torch.zeros((T, topk), dtype=torch.int32, device=dev)
         outs = _static_outs(n, E, dev)
         args = lambda: (_lib.ptr(ids), T, topk, E) + tuple(_lib.ptr(t) for t in outs)  # noqa: E731
-        if n > 8192:
+        if n > 65536:
             _lib.call("dwm_moe_dispatch_noalloc", *args(), _lib.stream_handle(dev))
             torch.cuda.synchronize()
         g = torch.cuda.CUDAGraph()

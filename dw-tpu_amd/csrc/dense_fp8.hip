@@ -416,7 +416,7 @@ __global__ __launch_bounds__(64 * KS) void dense_fp8_skinny_kernel(
 // the block's weights through L1.  W8A8's row scales of the block's K run are
 // transposed into LDS once ([K block][row], so a lane's four rows are one
 // read).
-constexpr int kRowsKb = 32;  // K blocks per block at most (W8A8's row-scale buffer)
+constexpr int kRowsKb = 64;  // K blocks per block at most (W8A8's row-scale buffer)
 
 typedef __attribute__((ext_vector_type(8))) int i32x8_t;
 typedef i32x8_t __attribute__((aligned(16))) i32x8_a16_t;
@@ -1122,45 +1122,84 @@ static int rows_halves(int64_t M) { return M > 64 ? 2 : 1; }
 constexpr int rows_groups(int mb) { return mb == 2 ? 4 : 2; }
 static int rows_blocks(int64_t M) { return (int)(((M + 15) / 16 + rows_halves(M) - 1) / rows_halves(M)); }
 
+static bool rows_ok(int64_t M, int64_t K, int64_t N, bool a8) {
+  return M > 16 && M <= (a8 ? kRowsMax : 32) && (!a8 || N % 128 == 0) && dense_offsets_ok(M, K, N, 128);
+}
+
+// K runs of the rows kernel: at most one block per CU while every wave keeps a
+// K block (one and a bit rounds cost two: 32 W8A16 rows, K = 5120, N = 4608 18.3
+// us with 288 blocks, 12.4 with 216; K = 2048, N = 12288 17.7 -> 9.9).  Where
+// kRowsKb forces more blocks than CUs, as many as two rounds hold; past one
+// round of column tiles, runs of at most 32 K blocks (32 rows, K = 7168, N =
+// 20016 46.4 -> 42.4).
+static int rows_runs(int64_t M, int64_t KB, int64_t ct) {
+  const int64_t waves = 8 / rows_halves(M), most = ct > 256 ? 32 : kRowsKb, least = (KB + most - 1) / most;
+  int64_t ks = 256 / ct < KB / waves ? 256 / ct : KB / waves;
+  if (ks < 1) ks = 1;
+  if (ks < least) ks = 512 / ct > least ? 512 / ct : least;
+  return whole_runs(KB, (int)ks);
+}
+
+// K runs of the MFMA tiles: doubled until the grid covers the 256 CUs.
+static int mfma_runs(int64_t KB, int64_t tiles) {
+  int ks = 1;
+  while (tiles * ks < 256 && ks * 2 <= KB && ks < 16) ks *= 2;
+  return whole_runs(KB, ks);
+}
+
 // Measured against the 128-row MFMA tiles (K = 7168, N = 4096, reduce
 // included), W8A8: M = 17 16.4 -> 11.1 us, 32 17.0 -> 11.6, 48 18.9 -> 12.8, 64
 // 19.2 -> 14.8, 65 19.4 -> 17.7; past 96 rows it loses (100 rows 20.8 ->
 // 21.6).  Above 32 rows a second round of its one-per-CU blocks loses too
 // (64 rows, K = 1024, N = 32768 16.8 -> 27.3), so the column tiles must fit
-// one; up to 32 rows it wins there as well (20 rows 15.0 -> 11.7).
-// W8A16 takes it up to 32 rows (17 rows 14.3 -> 10.9, 32 14.9 -> 11.8; K =
-// 1024, N = 32768 20.8 -> 14.6): its lhs fragments are 64 bytes a lane, half
-// lines of every row, and from 48 rows on they cost more than the tiles' LDS
-// copies (48 rows 15.9 -> 16.4, 64 16.7 -> 19.7); off the 128-column grid it
-// replaces the general tiled kernel (32 rows, N = 4048 18.0 -> 12.1).
-static bool rows_rule(int64_t M, int64_t N, bool a8) {
-  return M <= 32 || (a8 && M <= kRowsMax && N / (16 * rows_groups(rows_blocks(M))) <= 256);
-}
-static bool rows_ok(int64_t M, int64_t K, int64_t N, bool a8) {
-  return M > 16 && M <= (a8 ? kRowsMax : 32) && (!a8 || N % 128 == 0) && dense_offsets_ok(M, K, N, 128);
+// one; above 64 the whole grid must, and runs of more than 32 K blocks lose to
+// tiles that fill one round exactly (96 rows, K = 7168, N = 8192 27.7 -> 31.5).
+// Up to 32 rows a second round wins (20 rows 15.0 -> 11.7), but not over one
+// round of tiles under 4 K blocks (32 rows, K = 256, N = 32768 8.4 -> 10.3).
+// W8A16 takes it up to 32 rows (17 rows 14.3 -> 10.9, 32 14.9 -> 11.8): its lhs
+// fragments are 64 bytes a lane, half lines of every row, and from 48 rows on
+// they cost more than the tiles' LDS copies (48 rows 15.9 -> 16.4, 64 16.7 ->
+// 19.7).  Against the 64-row MFMA tiles it loses where most of its waves idle
+// (up to three K blocks: 17 rows, K = 256, N = 4096 4.7 -> 5.3; 32 rows 4.9 ->
+// 6.5), in a second round of up to eight (32 rows, K = 1024, N = 32768 10.8 ->
+// 15.5), and on narrow products (under 64 blocks and 32 K blocks: 32 rows, K =
+// 2048, N = 1024 7.1 -> 8.8; under 16 K blocks only with under 32 blocks and
+// over 24 rows: K = 1024, N = 512 17 rows 5.9 -> 5.4, 32 6.1 -> 6.5).  Off the 128-column grid it replaces the
+// general tiled kernel (32 rows, N = 4048 18.0 -> 12.1), which stays for one K
+// block (32 rows 4.7 -> 6.5) and for two in a second round (K = 256, N = 20016
+// 10.0 -> 12.6).
+static bool rows_rule(int64_t M, int64_t K, int64_t N, bool a8) {
+  const int64_t KB = K / 128, tn = 16 * rows_groups(rows_blocks(M)), ct = (N + tn - 1) / tn;
+  const int64_t blocks = ct * rows_runs(M, KB, ct);
+  if (a8) {
+    if (M <= 32) return KB >= 4 || N / 128 < 256;
+    if (M <= 64) return ct <= 256;
+    const int64_t tiles = N / 128;
+    return M <= kRowsMax && blocks <= 256 && (KB * ct <= 32 * blocks || tiles * mfma_runs(KB, tiles) > 256);
+  }
+  if (M > 32) return false;
+  if (N % 128 != 0) return KB > 2 || (KB == 2 && ct <= 256);
+  return KB > 3 && (ct <= 256 || KB > 8) && (blocks >= 64 || KB >= 32 || (KB < 16 && (M <= 24 || blocks >= 32)));
 }
 
 static dwm_dense_plan default_plan(int64_t M, int64_t K, int64_t N, bool a8) {
   const int64_t KB = K / 128;
-  if (rows_ok(M, K, N, a8) && rows_rule(M, N, a8)) {
-    // One block per CU, while every wave keeps a K block; at most kRowsKb per block.
+  if (rows_ok(M, K, N, a8) && rows_rule(M, K, N, a8)) {
     const int tn = 16 * rows_groups(rows_blocks(M));
-    const int64_t ct = (N + tn - 1) / tn, waves = 8 / rows_halves(M);
-    int64_t ks = (256 + ct - 1) / ct;
-    if (ks > KB / waves) ks = KB / waves;
-    if (ks < (KB + kRowsKb - 1) / kRowsKb) ks = (KB + kRowsKb - 1) / kRowsKb;
-    return {DWM_DENSE_ROWS, 16 * rows_blocks(M) * rows_halves(M), tn, whole_runs(KB, (int)ks), 2};
+    return {DWM_DENSE_ROWS, 16 * rows_blocks(M) * rows_halves(M), tn, rows_runs(M, KB, (N + tn - 1) / tn), 2};
   }
   if (dense_mfma_ok(M, K, N, 128)) {
     const int tm = (a8 && M >= 256) ? 256 : (!a8 && M <= 64) ? 64 : 128;
     const int64_t tiles = (N / 128) * ((M + tm - 1) / tm);
-    int ks = 1;
-    while (tiles * ks < 256 && ks * 2 <= KB && ks < 16) ks *= 2;
-    ks = whole_runs(KB, ks);
+    int ks = mfma_runs(KB, tiles);
     if (a8) return {DWM_DENSE_MFMA, tm, 128, ks, tm == 256 ? 3 : 4};
     // 33 .. 64 rows: half the MFMAs, lhs copies and barrier partners of a
     // 128-row tile (K = 7168, N = 4096: 48 rows 15.3 -> 13.9 us, 64 16.1 ->
     // 14.4; K = 1024, N = 32768 22.3 -> 12.0; twice the K runs lost, 17.7).
+    // Up to 32 rows only the products that rows_rule leaves: shallow ones in
+    // one run (17 rows, K = 256, N = 4096 4.7 us, two runs 6.1), narrow ones in
+    // runs of two K blocks (32 rows, K = 2048, N = 1024 7.1, of one 7.8).
+    if (M <= 32) ks = KB <= 8 && (KB <= 3 || tiles > 128) ? 1 : whole_runs(KB, KB >= 16 && ks > KB / 2 ? KB / 2 : ks);
     if (tm == 64) return {DWM_DENSE_MFMA, 64, 128, ks, 4};
     // Enough rows for 256 x 128 tiles to fill the grid: half the weight
     // re-reads of 128-row tiles (8 waves, one block per CU).
@@ -1172,9 +1211,7 @@ static dwm_dense_plan default_plan(int64_t M, int64_t K, int64_t N, bool a8) {
   if (!a8 && dense_edge_ok(M, K, N, 128)) {
     const int64_t ct = (N + 127) / 128;
     if (ct * ((M + 255) / 256) >= 256) return {DWM_DENSE_EDGE, 256, 128, 1, 3};
-    int ks = 1;
-    while (ct * ((M + 127) / 128) * ks < 256 && ks * 2 <= KB && ks < 16) ks *= 2;
-    return {DWM_DENSE_EDGE, 128, 128, whole_runs(KB, ks), 3};
+    return {DWM_DENSE_EDGE, 128, 128, mfma_runs(KB, ct * ((M + 127) / 128)), 3};
   }
   // 16 waves split K, two K blocks (weights, lhs fragments and scales) in
   // flight per wave; 4/8/16 waves x 2..7 blocks in flight all measured

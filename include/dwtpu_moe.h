@@ -417,7 +417,7 @@ enum dwm_dense_kernel {
   DWM_DENSE_TILED = 3,
   /* 17 <= M <= 32 (W8A8: 96, N % 128 == 0): M rounded up to 32 rows x 64
    * columns, or 48, 64 or 96 rows x 32 columns per block, operands
-   * straight from memory to registers (ring depth 2), at most 32 K blocks per
+   * straight from memory to registers (ring depth 2), at most 64 K blocks per
    * K run. */
   DWM_DENSE_ROWS = 4,
   /* W8A16, M > 64, N > 128, N % 128 != 0: the 128 x 128 or 256 x 128 MFMA

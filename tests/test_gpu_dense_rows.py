@@ -35,6 +35,8 @@ def _check(out, y64, ap, K):
     (96, 640, 8320, (2, 128, 128, 3, 4)),  # 260: the MFMA tiles
     (97, 1024, 256, (2, 128, 128, 8, 4)),
     (32, 256, 16640, (4, 32, 64, 1, 2)),   # two rounds of column tiles
+    (32, 256, 32768, (2, 128, 128, 1, 4)),  # under 4 K blocks: one round of MFMA tiles instead
+    (80, 4224, 8192, (2, 128, 128, 4, 4)),  # past 64 rows, 33 K blocks in one run against one round of tiles
 ])
 def test_w8a8_rows_plans_against_oracle(dev, M, K, N, plan):
     from dw_tpu_amd.dense_fp8 import last_plan, matmul_w8a8
@@ -53,17 +55,23 @@ def test_w8a8_rows_plans_against_oracle(dev, M, K, N, plan):
 
 
 @pytest.mark.parametrize("M,K,N,plan", [
-    (17, 128, 128, (4, 32, 64, 1, 2)),
+    (17, 512, 128, (4, 32, 64, 1, 2)),
     (32, 4224, 256, (4, 32, 64, 4, 2)),
-    (31, 1152, 384, (4, 32, 64, 1, 2)),
-    (24, 2176, 128, (4, 32, 64, 2, 2)),
-    (32, 256, 16640, (4, 32, 64, 1, 2)),
+    (24, 1152, 384, (4, 32, 64, 1, 2)),
+    (32, 1152, 16640, (4, 32, 64, 1, 2)),   # two rounds of column tiles
+    # up to three K blocks, up to eight in a second round, narrow products: 64-row MFMA tiles
+    (17, 128, 128, (2, 64, 128, 1, 4)),
+    (32, 256, 16640, (2, 64, 128, 1, 4)),
+    (31, 1152, 384, (2, 64, 128, 5, 4)),
+    (24, 2176, 128, (2, 64, 128, 6, 4)),    # 17 K blocks in runs of 3, 3, 3, 3, 3, 2
     (33, 1024, 256, (2, 64, 128, 8, 4)),   # past 32 rows: 64-row MFMA tiles
     (64, 1152, 128, (2, 64, 128, 5, 4)),   # runs of 2, 2, 2, 2, 1 K blocks: two steps in a four-stage ring
     (48, 384, 33024, (2, 64, 128, 1, 4)),
     (65, 1024, 256, (2, 128, 128, 8, 3)),
     # widths off the 128 grid: rows kernel, general tiles (33 .. 64 rows), MFMA tiles with a part-filled last one
     (17, 256, 16, (4, 32, 64, 1, 2)),
+    (17, 128, 16, (3, 64, 128, 1, 2)),      # one K block: general tiles
+    (32, 256, 16400, (3, 64, 128, 2, 2)),   # two in a second round
     (32, 2048, 208, (4, 32, 64, 2, 2)),
     (29, 384, 4080, (4, 32, 64, 1, 2)),
     (64, 512, 144, (3, 64, 128, 4, 2)),
@@ -90,6 +98,40 @@ def test_w8a16_rows_plans_against_oracle(dev, M, K, N, plan):
     t = plan_to_tile(p, K)
     again = matmul(x, pw, s, mode=t.mode, tm=t.tm, tk=t.tk, tn=t.tn, stages=t.stages)
     assert torch.equal(again.view(torch.int16), out.view(torch.int16)) and last_plan().astuple() == plan
+
+
+@pytest.mark.parametrize("a8,M,K,N,plan", [
+    (False, 17, 128, 128, (4, 32, 64, 1, 2)),   # one K block: seven of eight waves have none
+    (False, 31, 1152, 384, (4, 32, 64, 1, 2)),
+    (False, 24, 2176, 128, (4, 32, 64, 2, 2)),  # runs of 9 and 8 K blocks
+    (False, 32, 256, 16640, (4, 32, 64, 1, 2)),
+    (False, 20, 8192, 64, (4, 32, 64, 1, 2)),   # 64 K blocks in one run, the most
+    (True, 20, 8192, 128, (4, 32, 64, 1, 2)),
+    (True, 48, 8192, 128, (4, 48, 32, 1, 2)),
+    (True, 64, 8320, 128, (4, 64, 32, 2, 2)),   # runs of 33 and 32
+    (True, 96, 8192, 128, (4, 96, 32, 1, 2)),
+])
+def test_rows_kernel_by_plan(dev, a8, M, K, N, plan):
+    """The rows kernel where the library's own rule takes other tiles."""
+    from dw_tpu_amd import _lib
+    from dw_tpu_amd.dense_fp8 import last_plan, matmul, matmul_w8a8
+    from dw_tpu_amd.dense_fp8_tiles import plan_to_tile
+    from dw_tpu_amd.workloads import make_dense_workload
+    wl = make_dense_workload(M, K, N, seed=M + K + 3)
+    t = plan_to_tile(_lib.DensePlan(*plan), K)
+    if a8:
+        out = matmul_w8a8(*(torch.from_numpy(v).to(dev) for v in (wl.xq, wl.sx, wl.wq, wl.sw)), tile=t)
+        y64, ap = (f(wl.xq, wl.sx, wl.wq, wl.sw, **kw) for f, kw in (
+            (odf.matmul_w8a8, {"out_dtype": "float64"}), (odf.abs_product_w8a8, {})))
+    else:
+        xf = bf16_to_f32(wl.x_bits)
+        out = matmul(bf16_tensor(wl.x_bits, dev), torch.from_numpy(wl.wq).to(dev).view(torch.float8_e4m3fn),
+                     torch.from_numpy(wl.s_w8a16).to(dev), mode=t.mode, tm=t.tm, tk=t.tk, tn=t.tn, stages=t.stages)
+        y64 = odf.matmul_w8a16(xf, wl.wq, wl.s_w8a16, out_dtype="float64")
+        ap = odf.abs_product_w8a16(xf, wl.wq, wl.s_w8a16)
+    torch.cuda.synchronize()
+    assert last_plan().astuple() == plan
+    _check(out, y64, ap, K)
 
 
 @pytest.mark.parametrize("a8", [False, True])

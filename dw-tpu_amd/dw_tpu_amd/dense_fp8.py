@@ -61,17 +61,20 @@ def prepack_fp8(weight: torch.Tensor) -> Fp8Weight:
 
 
 @functools.lru_cache(maxsize=4096)
-def _default_workspace(m, k, n):
-    """Workspace bytes of the library's own plans (host arithmetic on the sizes alone)."""
+def _default_workspace(m, k, n, w8a8):
+    """Workspace bytes of the library's own plan (host arithmetic on the sizes
+    alone).  ``dwm_dense_fp8_workspace_size`` covers every variant's plan, the
+    "pre" mode's too: up to 32 MB more than the one that runs."""
     b = ctypes.c_int64(0)
-    _lib.call("dwm_dense_fp8_workspace_size", m, k, n, ctypes.byref(b))
+    plan = default_plan(m, k, n, w8a8)
+    _lib.call("dwm_dense_fp8_plan_workspace_size", m, k, n, ctypes.byref(plan), ctypes.byref(b))
     return b.value
 
 
 def _plan_and_workspace(m, k, n, dev, tile, w8a8):
     """(plan pointer or None, workspace tensor or None, workspace bytes)."""
     if tile is None:
-        plan, need = None, _default_workspace(m, k, n)
+        plan, need = None, _default_workspace(m, k, n, bool(w8a8))
     else:
         p = tile_to_plan(tile, max(m, 1), k, n, w8a8)
         b = ctypes.c_int64(0)

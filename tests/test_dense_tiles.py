@@ -128,3 +128,15 @@ def test_try_dense_fp8_fail_closed_on_host():
     assert dense_fp8.try_dense_fp8(x, w, s.double()) is None           # scale not f32
     assert dense_fp8.try_dense_fp8(x, w, torch.ones((2, 128))) is None # scale shape
     assert dense_fp8.try_dense_fp8(x, w, s) is None                    # host tensors: no kernel
+
+
+@pytest.mark.parametrize("m,k,n,a16,a8", [
+    (0, 7168, 4096, 0, 0), (1, 7168, 4096, 0, 0), (16, 1024, 32768, 0, 0),   # one launch, nothing to sum
+    (100, 7168, 4096, 8, 8), (1000, 7168, 4096, 1, 2), (4096, 7168, 4096, 1, 1),
+])
+def test_default_launches_take_no_more_workspace_than_their_plan(m, k, n, a16, a8):
+    """A launch with no tile allocates what its own plan needs (``a16`` and
+    ``a8`` K runs of f32 partials, none for a single run), not the largest need
+    of every variant."""
+    for w8a8, runs in ((False, a16), (True, a8)):
+        assert dense_fp8._default_workspace(m, k, n, w8a8) == (4 * runs * m * n if runs > 1 else 0)

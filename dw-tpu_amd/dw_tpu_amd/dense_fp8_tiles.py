@@ -94,6 +94,8 @@ def tile_to_plan(tile, m, k, n, w8a8=False):
         kernel = _lib.DENSE_EDGE if stages == 3 else kernel
     else:
         kernel = (_lib.DENSE_SKINNY if (tm, tn) == (16, 16) else _lib.DENSE_ROWS if tn in (32, 64) else _lib.DENSE_MFMA)
+    if w8a8 and kernel == _lib.DENSE_MFMA and tm == 64:
+        tm = 128  # W8A8's smallest MFMA tile: W8A16's of up to 64 rows names that launch
     if kernel == _lib.DENSE_SKINNY:
         if tk != k:
             raise ValueError(f"the skinny kernel covers all of K in one block: tk must be {k}")

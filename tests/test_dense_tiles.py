@@ -140,3 +140,12 @@ def test_default_launches_take_no_more_workspace_than_their_plan(m, k, n, a16, a
     of every variant."""
     for w8a8, runs in ((False, a16), (True, a8)):
         assert dense_fp8._default_workspace(m, k, n, w8a8) == (4 * runs * m * n if runs > 1 else 0)
+
+
+@pytest.mark.parametrize("k,n", [(7168, 4096), (2048, 1024), (256, 512), (512, 20480)])
+@pytest.mark.parametrize("m", [1, 16, 17, 25, 32, 33, 48, 64, 65, 96, 128])
+def test_select_tile_names_a_w8a8_launch_too(m, k, n):
+    """``matmul_w8a8(..., tile=select_tile(m, k, n))`` runs (up to 64 rows the
+    W8A16 choice can be a 64-row tile, which W8A8 does not have)."""
+    plan = tiles.tile_to_plan(dense_fp8.select_tile(m, k, n), m, k, n, w8a8=True)
+    assert plan.kernel != _lib.DENSE_MFMA or plan.tile_m >= 128

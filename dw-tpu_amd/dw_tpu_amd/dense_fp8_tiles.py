@@ -16,8 +16,9 @@ What they mean here is a launch of this library's kernels
                    tn = 64 or 32: the rows kernel (17 <= M <= 32, W8A8 <= 96; tm
                    = M rounded up to 32 (tn = 64), 48, 64 or 96 (32));
   mode "megablox"  the general tiled kernel, tm x tn = 16 x 64, 64 x 128 or
-                   128 x 128 (any N % 16 == 0); with "stages" 3 the MFMA tiles
-                   of a width off the 128 grid (M > 64, tm = 128 or 256);
+                   128 x 128 (any N % 16 == 0); with "stages" 3, or tm = 256,
+                   the MFMA tiles of a width off the 128 grid (M > 64, tm =
+                   128 or 256);
   tk               the K depth one block covers: K / tk blocks share an
                    output tile and their f32 partials are added in order;
   "stages"         optional ring depth (LDS stages of the MFMA kernel);
@@ -65,7 +66,7 @@ def _usual_stages(kernel, tile_m, w8a8):
         if w8a8:
             return 4 if tile_m == 128 else 3
         return {64: 4, 128: 3}.get(tile_m, 2)
-    return 2
+    return 3 if kernel == _lib.DENSE_EDGE else 2
 
 
 def plan_to_tile(plan, k):
@@ -91,7 +92,8 @@ def tile_to_plan(tile, m, k, n, w8a8=False):
         raise ValueError(f"tk={tk} must be a positive multiple of 128 (the scale block)")
     kernel = _KERNEL_OF_MODE[mode]
     if kernel is not None:
-        kernel = _lib.DENSE_EDGE if stages == 3 else kernel
+        # Only the edge tiles have 256 rows, so those need no "stages" to be told apart.
+        kernel = _lib.DENSE_EDGE if stages == 3 or (stages == 0 and tm == 256) else kernel
     else:
         kernel = (_lib.DENSE_SKINNY if (tm, tn) == (16, 16) else _lib.DENSE_ROWS if tn in (32, 64) else _lib.DENSE_MFMA)
     if w8a8 and kernel == _lib.DENSE_MFMA and tm == 64:

@@ -149,3 +149,16 @@ def test_select_tile_names_a_w8a8_launch_too(m, k, n):
     W8A16 choice can be a 64-row tile, which W8A8 does not have)."""
     plan = tiles.tile_to_plan(dense_fp8.select_tile(m, k, n), m, k, n, w8a8=True)
     assert plan.kernel != _lib.DENSE_MFMA or plan.tile_m >= 128
+
+
+@pytest.mark.parametrize("m", [1, 16, 24, 64, 100, 256, 700, 1024, 4096])
+@pytest.mark.parametrize("n", [144, 4000, 4096, 7184])
+def test_select_tile_needs_no_stages(m, n):
+    """The plain 4-tuple of a selected tile, and a file's entry without
+    "stages", name a launch too: of the same tile, with the usual ring."""
+    k = 2048
+    mode, tm, tk, tn = tuple(dense_fp8.select_tile(m, k, n))
+    plan = tiles.tile_to_plan((mode, tm, tk, tn), m, k, n)
+    assert (plan.tile_m, plan.tile_n) == (tm, tn)
+    table = tiles.parse_table(_doc([{"m": m, "k": k, "n": n, "mode": mode, "tm": tm, "tk": tk, "tn": tn}]))
+    assert table[(m, k, n)] == (mode, tm, tk, tn)

@@ -126,6 +126,7 @@ class MoeBlockGraph:
         plain = dev.index == torch.cuda.current_device() and all(
             type(src) is torch.Tensor and src.device == dst.device == dev and src.dtype == dst.dtype
             and src.is_contiguous() and dst.is_contiguous() and not (src.requires_grad or dst.requires_grad)
+            and not (src.is_neg() or dst.is_neg())  # a lazy sign is not in the bytes
             for src, dst in pairs)
         if plain and pairs:
             n = len(pairs)

@@ -71,3 +71,23 @@ def test_graph_inputs_of_other_forms(dev, rng):
         assert torch.equal(got.view(torch.int16), want.view(torch.int16)), form
     with pytest.raises(ValueError, match="captured"):
         graph(h[:8], ids, w)
+
+
+@pytest.mark.gpu
+def test_graph_inputs_with_a_lazy_sign(dev, rng):
+    """A negated view's bytes are those of its base: torch's copy resolves it."""
+    from dw_tpu_amd import MoeBlockGraph, fp4_weight_to_codes, moe_block
+    T, E, topk, H, I = 24, 8, 2, 256, 128
+    fp4 = lambda *s: torch.from_numpy(rng.integers(0, 256, s, dtype=np.uint8)).to(dev)  # noqa: E731
+    sc = lambda *s: torch.from_numpy(rng.integers(120, 126, s, dtype=np.uint8)).to(dev)  # noqa: E731
+    w13 = fp4_weight_to_codes(fp4(E, H, I), sc(E, H // 32, 1, 2 * I), gate_up=True)
+    w2 = fp4_weight_to_codes(fp4(E, I, H // 2), sc(E, I // 32, 1, H))
+    h = torch.from_numpy(rng.standard_normal((T, H)).astype(np.float32)).to(dev)
+    ids = torch.from_numpy(rng.integers(0, E, (T, topk)).astype(np.int32)).to(dev)
+    w = torch.from_numpy(rng.random((T, topk)).astype(np.float32)).to(dev)
+    graph = MoeBlockGraph(h.bfloat16(), ids, w, w13, w2, E)
+    neg = torch._neg_view(w)
+    assert neg.is_neg() and neg.is_contiguous()
+    got = graph(h.bfloat16(), ids, neg)
+    want = moe_block(h.bfloat16(), ids, -w, w13, w2, E)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))

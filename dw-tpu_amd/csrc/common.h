@@ -15,6 +15,8 @@ namespace dwm {
 
 void set_error(const char *fmt, ...);
 void clear_error();
+// What dwm_last_kernel reports on this thread (a string literal).
+void note_kernel(const char *name);
 
 #define DWM_CHECK_ARG(cond, ...)        \
   do {                                  \
@@ -31,6 +33,9 @@ void clear_error();
       return DWM_ERR_UNSUPPORTED;       \
     }                                   \
   } while (0)
+
+// Compute units of the current device (gmm_fp4.hip).
+int device_cu_count();
 
 // Reports the launch status of the kernels just enqueued.
 int launch_status(const char *what);

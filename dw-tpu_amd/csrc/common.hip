@@ -18,6 +18,10 @@ void set_error(const char *fmt, ...) {
 
 void clear_error() { g_last_error.clear(); }
 
+static thread_local const char *g_last_kernel = "";
+
+void note_kernel(const char *name) { g_last_kernel = name; }
+
 int launch_status(const char *what) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
@@ -32,3 +36,5 @@ int launch_status(const char *what) {
 extern "C" int dwm_version(void) { return 100; }
 
 extern "C" const char *dwm_last_error(void) { return dwm::g_last_error.c_str(); }
+
+extern "C" const char *dwm_last_kernel(void) { return dwm::g_last_kernel; }

@@ -1213,10 +1213,11 @@ static dwm_dense_plan default_plan(int64_t M, int64_t K, int64_t N, bool a8) {
     if (ct * ((M + 255) / 256) >= 256) return {DWM_DENSE_EDGE, 256, 128, 1, 3};
     return {DWM_DENSE_EDGE, 128, 128, mfma_runs(KB, ct * ((M + 127) / 128)), 3};
   }
-  // 16 waves split K, two K blocks (weights, lhs fragments and scales) in
-  // flight per wave; 4/8/16 waves x 2..7 blocks in flight all measured
-  // within 0.5 us at K=7168, N=4096: the 29 MB stream plus launch and
-  // start-up latency sets the time (8 us at M = 1).
+  // 16 waves split K past 1024, two K blocks (weights, lhs fragments and
+  // scales) in flight per wave; 4/8/16 waves x 2..7 blocks in flight all
+  // measured within 0.5 us at K=7168, N=4096: the 29 MB stream plus launch and
+  // start-up latency sets the time (8 us at M = 1).  run_dense gives a
+  // shallower K the form that fits it; all of them are this plan.
   if (M <= 16) return {DWM_DENSE_SKINNY, 16, 16, 16, 2};
   dwm_dense_plan p = tiled_default(M, K, N);
   p.ksplit = whole_runs(KB, p.ksplit);
@@ -1227,7 +1228,7 @@ static int check_plan(int64_t M, int64_t K, int64_t N, bool a8, const dwm_dense_
   const int64_t KB = K / 128;
   const char *const v = a8 ? "w8a8" : "w8a16";
   if (p.kernel == DWM_DENSE_SKINNY) {
-    // Its 16 waves split K inside the block (idle waves when K/128 < 16).
+    // One plan for all of its forms (run_dense): their sums are the same.
     DWM_UNSUPPORTED_IF(M > 16, "dense_fp8 plan: the skinny kernel takes M <= 16 (M=%lld)", (long long)M);
     DWM_UNSUPPORTED_IF(p.tile_m != 16 || p.tile_n != 16 || p.ksplit != 16 || p.stages != 2,
                        "dense_fp8 plan: the skinny kernel runs 16 x 16 tiles, 16 K runs, ring depth 2");
@@ -1360,21 +1361,30 @@ static int run_dense(const void *x, const float *sx, int64_t M, int64_t K, int64
   float *const partial = need ? (float *)workspace : nullptr;
   const int ks = p.ksplit;
   if (p.kernel == DWM_DENSE_SKINNY) {
-    // One K block per wave up to K = 2048: no more waves than K blocks, so that
-    // none is idle and more blocks share a CU (the same sums in the same order).
-    // Wide and shallow (at least two blocks per CU of 64 columns), a block
-    // takes four column groups.
+    // The plan names the kernel; its form is chosen here by size.  Up to K =
+    // 512, 1024 and 2048, 4, 8 and 16 waves take one K block each (the last
+    // ones none where K has fewer blocks); fewer waves let more blocks share a
+    // CU, and the sums and their order do not change.  Wide and shallow, a block
+    // takes four column groups and reads the lhs once for all of them, from two
+    // such blocks per CU on.  Measured, one group against four, us: K = 512, N
+    // = 32768, 16 rows 7.3 -> 5.7, one row 4.7 -> 5.2; N = 16384, one row
+    // 3.5 -> 3.9, 16 rows 4.8 -> 4.4; K = 1024, N = 65536, 16 rows 21.5 ->
+    // 18.4.  16 waves of one group, for all, against these, one row: K = 512, N
+    // = 32768 12.3 -> 5.2; K = 128, N = 16384 5.5 -> 2.1, N = 24576 8.2 -> 2.65,
+    // N = 65536 19.8 -> 5.0.
 #define DWM_SKINNY(KS, D, NB)                                                                                   \
   hipLaunchKernelGGL((dense_fp8_skinny_kernel<KS, D, NB, A8>), dim3((unsigned)(N / (16 * NB))), dim3(64 * KS), 0, \
-                     st, x, sx, (int)M, (int)K, (int)N, w, sw, sw_ld, out)
-    const bool wide = N % 64 == 0 && N / 64 >= 512;
-    if (K <= 512 && wide) DWM_SKINNY(4, 1, 4);
-    else if (K <= 512) DWM_SKINNY(4, 1, 1);
-    else if (K <= 1024 && wide) DWM_SKINNY(8, 1, 4);
-    else if (K <= 1024) DWM_SKINNY(8, 1, 1);
-    else DWM_SKINNY(16, 2, 1);
+                     st, x, sx, (int)M, (int)K, (int)N, w, sw, sw_ld, out);                                    \
+  note_kernel("dense_skinny/" #KS "/" #D "/" #NB)
+    const bool wide = N % 64 == 0 && N / 64 >= 2 * device_cu_count();
+    if (K <= 512 && wide) { DWM_SKINNY(4, 1, 4); }
+    else if (K <= 512) { DWM_SKINNY(4, 1, 1); }
+    else if (K <= 1024 && wide) { DWM_SKINNY(8, 1, 4); }
+    else if (K <= 1024) { DWM_SKINNY(8, 1, 1); }
+    else { DWM_SKINNY(16, 2, 1); }
 #undef DWM_SKINNY
   } else if (p.kernel == DWM_DENSE_ROWS) {
+    note_kernel("dense_rows");
     if (p.tile_m == 32) launch_rows<2, 1, A8>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
     if constexpr (A8) {
       if (p.tile_m == 48) launch_rows<3, 1, true>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
@@ -1382,6 +1392,7 @@ static int run_dense(const void *x, const float *sx, int64_t M, int64_t K, int64
       else if (p.tile_m == 96) launch_rows<3, 2, true>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
     }
   } else if (p.kernel == DWM_DENSE_MFMA || p.kernel == DWM_DENSE_EDGE) {
+    note_kernel(p.kernel == DWM_DENSE_EDGE ? "dense_edge" : "dense_mfma");
     if constexpr (A8) {
       if (p.tile_m == 256) launch_mfma<DenseMfmaCfg<4, 2, true>, true, 3>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
       else if (p.stages == 3) launch_mfma<DenseMfmaCfg<2, 2, true>, true, 3>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
@@ -1395,6 +1406,7 @@ static int run_dense(const void *x, const float *sx, int64_t M, int64_t K, int64
       else launch_mfma<DenseMfmaCfg<2, 4, false, 1>, false, 4>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
     }
   } else {
+    note_kernel("dense_tiled");
     if (p.tile_m == 16) launch_tiled<1, 1, A8>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
     else if (p.tile_m == 64) launch_tiled<4, 2, A8>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
     else launch_tiled<8, 2, A8>(x, sx, M, K, N, w, sw, sw_ld, ks, out, partial, st);
@@ -1536,6 +1548,7 @@ extern "C" int dwm_dense_fp8_w8a16_pre(const uint16_t *x, int64_t M, int64_t K, 
   float *const partial = need ? (float *)workspace : nullptr;
   hipStream_t st = as_stream(stream);
   const int ks = p.ksplit;
+  note_kernel("dense_tiled");
   if (p.tile_m == 16) launch_tiled<1, 1, false, true>(x, nullptr, M, K, N, w, s, (int)N, ks, out, partial, st);
   else if (p.tile_m == 64) launch_tiled<4, 2, false, true>(x, nullptr, M, K, N, w, s, (int)N, ks, out, partial, st);
   else launch_tiled<8, 2, false, true>(x, nullptr, M, K, N, w, s, (int)N, ks, out, partial, st);

@@ -657,8 +657,10 @@ int launch_gmm_zero_rows(const int32_t *group_sizes, int num_groups, const int32
   return launch_status("gmm zero rows");
 }
 
-// Compute units of the current device (looked up once per device).  It only
-// sizes the narrow split; any positive value gives correct results.
+// Compute units of the current device (looked up once per device).  It sizes
+// the narrow split and the streaming kernel's tiles and blocks, and draws the
+// lines at which gmm_streams and the dense skinny kernel change form; any
+// positive value gives correct results.
 int device_cu_count() {
   constexpr int kMaxDev = 64;
   static std::atomic<int> cache[kMaxDev];
@@ -694,6 +696,7 @@ static int launch_gmm_ws(const uint16_t *lhs, const int32_t *row_idx, int64_t lh
   DWM_UNSUPPORTED_IF(K > (1 << 24), "gmm_fp4: K <= 2^24 required");
   hipLaunchKernelGGL((gmm_fp4_ws_kernel<C, MB, ACT, NARROW, AUX>), dim3((unsigned)grid), dim3(C::THREADS), 0, st, lhs,
                      row_idx, lhs_rows, M, (int)K, w, s, gs, ng, go, e_local, (int)N, out, out_f32, ep, ncu, bal);
+  note_kernel("gmm_ws");
   return launch_status("gmm_fp4");
 }
 

@@ -788,6 +788,7 @@ static int launch_mx(const uint8_t *lhs, const uint8_t *lsc, const int32_t *row_
   else
     hipLaunchKernelGGL((gmm_mx_kernel<C, ACT>), dim3((unsigned)grid), dim3(C::THREADS), 0, st, lhs, lsc, row_idx,
                        lhs_rows, M, (int)K, w, s, gs, ng, go, e_local, (int)N, out, out_f32, ep);
+  note_kernel(STEP128 ? "gmm_mx128" : "gmm_mx");
   return launch_status("gmm_fp4_mx");
 }
 

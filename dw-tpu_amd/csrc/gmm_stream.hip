@@ -336,6 +336,7 @@ int launch_gmm_stream(const uint16_t *lhs, const int32_t *row_idx, int64_t lhs_r
     else DWM_STREAM(1, false, false);
   }
 #undef DWM_STREAM
+  note_kernel("gmm_stream");
   return launch_status("gmm_fp4");
 }
 
@@ -465,6 +466,7 @@ int launch_gmm_mx_stream(const uint8_t *lhs, const uint8_t *lhs_scale, const int
   }
 #undef DWM_STREAM_W
 #undef DWM_STREAM
+  note_kernel("gmm_mx_stream");
   return launch_status("gmm_fp4_mx");
 }
 

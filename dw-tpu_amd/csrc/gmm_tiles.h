@@ -486,8 +486,6 @@ int launch_gmm_bf16(const uint16_t *lhs, const int32_t *row_idx, int64_t lhs_row
                     const uint8_t *weight, const uint8_t *scale, const int32_t *group_sizes, int num_groups,
                     const int32_t *group_offset, int64_t E_local, int64_t N, void *out, int out_f32, bool gated,
                     const GmmEpilogue &ep, hipStream_t st);
-// Compute units of the current device.
-int device_cu_count();
 // Whether a launch takes the streaming kernel (gmm_stream.hip; the rule and
 // its figures stand in gmm_fp4.hip).
 bool gmm_streams(int64_t M, int64_t N, int64_t E_local);

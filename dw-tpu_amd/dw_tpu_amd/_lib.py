@@ -35,6 +35,7 @@ _p = ctypes.c_void_p
 SIGNATURES = {
     "dwm_version": [],
     "dwm_last_error": [],
+    "dwm_last_kernel": [],
     "dwm_e2m1_to_codes": [_p, _p, _i64, _p],
     "dwm_fp4_decode": [_p, _i32, _i64, _p, _p, _p, _p],
     "dwm_gmm_fp4_prepack_size": [_i64, _i64, _i64, _p, _p],
@@ -72,7 +73,7 @@ SIGNATURES = {
     "dwm_route_topk": [_p, _i32, _i64, _i64, _i32, _i32, _p, _p, _i32, _p, _p, _i32, _p, _p],
     "dwm_dedupe_topk": [_p, _p, _i64, _i32, _i64, _p, _p, _p],
 }
-_RESTYPES = {"dwm_last_error": ctypes.c_char_p}
+_RESTYPES = {"dwm_last_error": ctypes.c_char_p, "dwm_last_kernel": ctypes.c_char_p}
 
 # enum dwm_dense_kernel
 DENSE_SKINNY, DENSE_MFMA, DENSE_TILED, DENSE_ROWS, DENSE_EDGE = 1, 2, 3, 4, 5
@@ -142,6 +143,11 @@ def call(name, *args):
     if rc == ERR_UNSUPPORTED:
         raise Unsupported(msg)
     raise RuntimeError(msg)
+
+
+def last_kernel():
+    """Name of the kernel this thread's last grouped or dense matmul launched."""
+    return load().dwm_last_kernel().decode()
 
 
 def ptr(t):

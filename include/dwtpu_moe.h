@@ -77,6 +77,13 @@ int dwm_version(void);
 /* Message of the last failed call on this thread ("" if none). */
 const char *dwm_last_error(void);
 
+/* The kernel that this thread's last grouped or dense matmul launched (for
+ * tests and traces; "" before the first): "gmm_ws" or "gmm_stream" (bf16 lhs),
+ * "gmm_mx", "gmm_mx128" or "gmm_mx_stream" (MX lhs), "dense_mfma",
+ * "dense_edge", "dense_rows", "dense_tiled", or "dense_skinny/W/D/G" (W waves
+ * split K, ring depth D, G groups of 16 columns per block). */
+const char *dwm_last_kernel(void);
+
 /* ---------------------------------------------------------------------- */
 /* FP4 weight codes.                                                       */
 /* ---------------------------------------------------------------------- */
@@ -405,8 +412,11 @@ int dwm_dense_fp8_w8a8(const uint8_t *xq, const float *sx, int64_t M, int64_t K,
  * dense_fp8_tiles.py:11-58) and matmul's tm/tk/tn (dense_fp8.py:15-76) choose
  * there, expressed in this library's kernels. */
 enum dwm_dense_kernel {
-  /* M <= 16: one block per 16 columns; its 16 waves split K (ksplit = 16)
-   * and add their f32 partial sums in wave order; register ring depth 2. */
+  /* M <= 16: waves split K inside a block and add their f32 partial sums in
+   * wave order.  One plan, 16 x 16 with ksplit 16 and stages 2, for every form
+   * the library gives it by size: 16 waves, two K blocks in flight, past
+   * K = 1024; 8 up to there, 4 up to K = 512; 64 columns per block in place of
+   * 16 for a wide shallow launch (dwm_last_kernel names the form). */
   DWM_DENSE_SKINNY = 1,
   /* tile_m x 128 tiles (tile_m 128 or 256; 64 for W8A16), 32x32 MFMA (bf16 for W8A16, fp8
    * for W8A8) fed by an LDS ring of `stages` K steps.  Needs M > 16 and

@@ -138,6 +138,7 @@ def test_rows_kernel_by_plan(dev, a8, M, K, N, plan):
 @pytest.mark.parametrize("M,K,N", [(1, 128, 48), (16, 512, 128), (5, 640, 256), (16, 1024, 80), (7, 1152, 128),
                                    (3, 256, 32768), (16, 512, 32832), (9, 896, 32768), (16, 1024, 33024)])
 def test_skinny_forms_against_oracle(dev, a8, M, K, N):
+    from dw_tpu_amd import _lib
     from dw_tpu_amd.dense_fp8 import last_plan, matmul, matmul_w8a8
     from dw_tpu_amd.workloads import make_dense_workload
     if a8:
@@ -164,4 +165,7 @@ def test_skinny_forms_against_oracle(dev, a8, M, K, N):
         ap = odf.abs_product_w8a16(xf, wc, sc)
     torch.cuda.synchronize()
     assert last_plan().astuple() == (1, 16, 16, 16, 2)
+    waves = 4 if K <= 512 else 8 if K <= 1024 else 16
+    wide = K <= 1024 and N % 64 == 0 and N >= 128 * torch.cuda.get_device_properties(dev).multi_processor_count
+    assert _lib.last_kernel() == f"dense_skinny/{waves}/{2 if waves == 16 else 1}/{4 if wide else 1}"
     _check(out[:, torch.from_numpy(cols).to(dev)], y64, ap, K)

@@ -500,16 +500,18 @@ def test_gmm_acceptance_policy_full_size(dev, rng, name, mx):
 
 
 @pytest.mark.parametrize("mx", [False, True])
-@pytest.mark.parametrize("num_groups,go,e_local", [(256, 96, 32), (1024, 1016, 8), (130, 0, 130)])
-def test_gmm_many_groups_window(dev, rng, mx, num_groups, go, e_local):
+@pytest.mark.parametrize("num_groups,go,e_local,N,most,tiles", [
+    (256, 96, 32, 64, 5, False), (1024, 1016, 8, 64, 5, True), (130, 0, 130, 64, 5, False),
+    (256, 96, 32, 1024, 5, True), (130, 0, 130, 1024, 24, True)])
+def test_gmm_many_groups_window(dev, rng, mx, num_groups, go, e_local, N, most, tiles):
     """Many global groups (DeepSeek's 256 experts, the 1024 maximum, and 130
     local ones): the device tile list's group scans run over several 64-group
     chunks.  Sizes are ragged with empty groups; the window's rows match the
     oracle (bf16 bound, or the MX bound) and every other row is zero."""
-    from dw_tpu_amd import fp4_weight_to_codes, gmm_v2
+    from dw_tpu_amd import _lib, fp4_weight_to_codes, gmm_v2
     from oracle import quant
-    K, N = 128, 64
-    sizes = rng.integers(0, 6, num_groups).astype(np.int32)
+    K = 128
+    sizes = rng.integers(0, most + 1, num_groups).astype(np.int32)
     sizes[rng.random(num_groups) < 0.3] = 0
     sizes[go] = 97  # a multi-tile local group
     M = int(sizes.sum())
@@ -519,6 +521,7 @@ def test_gmm_many_groups_window(dev, rng, mx, num_groups, go, e_local):
     pw = fp4_weight_to_codes(torch.from_numpy(rhs).to(dev), torch.from_numpy(sc).to(dev))
     out = gmm_v2(bf16_tensor(lhs_bits, dev), pw, torch.from_numpy(sizes).to(dev), group_offset=go,
                  preferred_element_type=torch.float32, lhs_quant_dtype=torch.float8_e4m3fn if mx else None)
+    assert _lib.last_kernel() == ("gmm_mx" if mx else "gmm_ws" if tiles else "gmm") + ("" if tiles else "_stream")
     torch.cuda.synchronize()
     a = bf16_to_f32(lhs_bits)
     if mx:

@@ -55,10 +55,14 @@ def _run(dev, lhs_bits, rhs, sc, gs, bias, act, mx, out_dtype=torch.bfloat16, bi
 @pytest.mark.parametrize("act", ACTS)
 @pytest.mark.parametrize("K", [256, 4096])
 @pytest.mark.parametrize("mx", [False, True])
-def test_bias_and_activation(dev, rng, mx, K, act):
+@pytest.mark.parametrize("sizes", [[40, 0, 70, 33], [140, 0, 97, 33]])
+def test_bias_and_activation(dev, rng, sizes, mx, K, act):
+    from dw_tpu_amd import _lib
     N = 192
-    lhs_bits, rhs, sc, gs, bias = _case(rng, [40, 0, 70, 33], K, N)
+    lhs_bits, rhs, sc, gs, bias = _case(rng, sizes, K, N)
     out = _run(dev, lhs_bits, rhs, sc, gs, bias, act, mx)
+    kernels = ("gmm_mx_stream", "gmm_mx128" if K >= 4096 else "gmm_mx") if mx else ("gmm_stream", "gmm_ws")
+    assert _lib.last_kernel() == kernels[sum(sizes) > 64 * len(sizes)]
     a = bf16_to_f32(lhs_bits)
     if mx:
         a = quant.mx_dequantize(*quant.mx_quantize_e4m3(a))

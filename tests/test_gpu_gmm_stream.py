@@ -42,16 +42,23 @@ CASES = [
     (128, 128, 4096, [192] + [0] * 31, None, True, "none"),
     (64, 128, 4096, [7, 0, 0, 0, 0, 7, 0], None, False, "f32"),
     (64, 256, 4096, [64] + [1] * 63, None, False, "none"),
+    # more rows per expert, in launches too small to fill the chip with tiles: 33 .. 64 rows of all, one and both
+    # clauses' edges (12 and 64 rows per expert), a window
+    (4, 384, 640, [50, 0, 64, 33], None, False, "none"),
+    (8, 256, 2560, [12], None, True, "none"),
+    (3, 640, 272, [64], None, False, "f32"),
+    (40, 128, 80, [0, 70, 16, 31], (5, 30), False, "gather"),
+    (2, 1408, 1040, [65, 63], None, False, "bias"),
 ]
 
 
 @pytest.mark.parametrize("E,K,N,pattern,window,act,form", CASES)
 def test_stream_kernel_against_oracle_and_tiles(dev, rng, E, K, N, pattern, window, act, form):
-    from dw_tpu_amd import fp4_weight_to_codes, gmm_v2
+    from dw_tpu_amd import _lib, fp4_weight_to_codes, gmm_v2
     sizes = _sizes(E, pattern)
     go, e_local = window if window else (0, E)
     M = int(sizes.sum())
-    assert 0 < M <= 6 * e_local, "the launch takes the streaming kernel"
+    assert 0 < M <= 64 * e_local
     rhs = rng.integers(0, 256, (e_local, K, N // 2), dtype=np.uint8)
     sc = rng.integers(123, 130, (e_local, K // 32, 1, N), dtype=np.uint8)
     pw = fp4_weight_to_codes(torch.from_numpy(rhs).to(dev), torch.from_numpy(sc).to(dev), gate_up=act)
@@ -69,6 +76,7 @@ def test_stream_kernel_against_oracle_and_tiles(dev, rng, E, K, N, pattern, wind
         y = gmm_v2(bf16_tensor(src, dev), pw, gs, lhs_row_indices=torch.from_numpy(idx).to(dev), **kw)
     else:
         y = gmm_v2(lhs, pw, gs, **kw)
+    assert _lib.last_kernel() == "gmm_stream"
     # The same rows at the head of groups padded to more than 72 rows each.
     pad = 80
     big = sizes + pad
@@ -79,6 +87,7 @@ def test_stream_kernel_against_oracle_and_tiles(dev, rng, E, K, N, pattern, wind
     rows[at] = bits
     at = torch.from_numpy(at).to(dev)
     yb = gmm_v2(bf16_tensor(rows, dev), pw, torch.from_numpy(big).to(dev), **kw)[at]
+    assert _lib.last_kernel() == "gmm_ws"
     torch.cuda.synchronize()
     assert torch.equal(y.view(torch.int32 if form == "f32" else torch.int16),
                        yb.view(torch.int32 if form == "f32" else torch.int16))
@@ -101,13 +110,13 @@ def test_stream_kernel_against_oracle_and_tiles(dev, rng, E, K, N, pattern, wind
 def test_mx_stream_kernel_equals_tiles(dev, rng, E, K, N, pattern, window, act, form, fmt):
     """The MX form gives the bits of the MX tiles (both K step depths: K below
     and from 4096 on) for every group and epilogue form above."""
-    from dw_tpu_amd import MxLhs, fp4_weight_to_codes, gmm_v2, mx_quantize
+    from dw_tpu_amd import MxLhs, _lib, fp4_weight_to_codes, gmm_v2, mx_quantize
     if E == 4:
         K = 4224
     sizes = _sizes(E, pattern)
     go, e_local = window if window else (0, E)
     M = int(sizes.sum())
-    assert 0 < M <= 6 * e_local
+    assert 0 < M <= 64 * e_local
     pw = fp4_weight_to_codes(torch.from_numpy(rng.integers(0, 256, (e_local, K, N // 2), dtype=np.uint8)).to(dev),
                              torch.from_numpy(rng.integers(123, 130, (e_local, K // 32, 1, N), dtype=np.uint8)).to(dev),
                              gate_up=act)
@@ -123,6 +132,7 @@ def test_mx_stream_kernel_equals_tiles(dev, rng, E, K, N, pattern, window, act, 
         y = gmm_v2(MxLhs(codes, scales, fmt), pw, torch.from_numpy(sizes).to(dev), lhs_row_indices=p, **kw)
     else:
         y = gmm_v2(x, pw, torch.from_numpy(sizes).to(dev), **kw)
+    assert _lib.last_kernel() == "gmm_mx_stream"
     big = sizes + 80
     assert big.sum() > 64 * e_local
     starts = np.concatenate([[0], np.cumsum(big)[:-1]])
@@ -131,9 +141,30 @@ def test_mx_stream_kernel_equals_tiles(dev, rng, E, K, N, pattern, window, act, 
     scales = torch.full((int(big.sum()), x.scales.shape[1]), 127, dtype=torch.uint8, device=dev)
     codes[at], scales[at] = x.codes, x.scales
     yb = gmm_v2(MxLhs(codes, scales, fmt), pw, torch.from_numpy(big).to(dev), **kw)[at]
+    assert _lib.last_kernel() == ("gmm_mx128" if K >= 4096 else "gmm_mx")
     torch.cuda.synchronize()
     v = torch.int32 if form == "f32" else torch.int16
     assert torch.equal(y.view(v), yb.view(v)) and bool((y != 0).any())
+
+
+@pytest.mark.parametrize("E,M,N,mx,kernel", [
+    (32, 192, 4096, False, "gmm_stream"),   # 6 rows per expert
+    (32, 193, 8192, False, "gmm_ws"),       # 33 tiles x 32 column tiles: past half of the CUs
+    (8, 512, 2304, True, "gmm_mx_stream"),  # 64 rows per expert, 13 x 9 tiles of 128 allowed
+    (8, 513, 2304, True, "gmm_mx"),
+    (8, 512, 2560, False, "gmm_ws"),        # 13 x 10
+    (8, 300, 2816, False, "gmm_stream"),    # 11 x 11
+])
+def test_stream_rule(dev, rng, E, M, N, mx, kernel):
+    from dw_tpu_amd import _lib, fp4_weight_to_codes, gmm_v2
+    K = 128
+    pw = fp4_weight_to_codes(torch.zeros((E, K, N // 2), dtype=torch.uint8, device=dev),
+                             torch.full((E, K // 32, 1, N), 127, dtype=torch.uint8, device=dev))
+    gs = torch.from_numpy(rng.multinomial(M, np.ones(E) / E).astype(np.int32)).to(dev)
+    y = gmm_v2(torch.ones((M, K), dtype=torch.bfloat16, device=dev), pw, gs,
+               lhs_quant_dtype=torch.float8_e4m3fn if mx else None)
+    assert _lib.last_kernel() == kernel
+    assert not y.any()
 
 
 def test_stream_kernel_skips_rows_past_m(dev, rng):

@@ -146,14 +146,20 @@ CASES = [  # K < 4096: the 64-deep kernel; K >= 4096: the 128-deep one
     ([1, 0, 15, 16, 17, 95, 97], 4096, 96),
     ([127, 0, 129, 8], 4224, 656),
 ]
+# The launches above of up to 64 rows per group take the streaming kernel: one
+# more group takes the same rows to the tiles.
+CASES += [(sizes + [64 * (len(sizes) + 1)], K, N) for sizes, K, N in CASES if 0 < sum(sizes) <= 64 * len(sizes)]
 
 
 @pytest.mark.parametrize("sizes,K,N", CASES)
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
 def test_gmm_mx_random_shapes(dev, rng, sizes, K, N, out_dtype):
+    from dw_tpu_amd import _lib
     lhs_bits, rhs, sc, gs = _mx_case(rng, sizes, K, N)
     out = _gmm_mx(dev, lhs_bits, rhs, sc, gs, out_dtype=out_dtype)
     if out.shape[0]:
+        tiles = "gmm_mx128" if K >= 4096 else "gmm_mx"
+        assert _lib.last_kernel() == (tiles if sum(sizes) > 64 * len(sizes) else "gmm_mx_stream")
         y64, ap, _ = _oracle_mx(lhs_bits, _w(rhs, sc), gs)
         print(sizes, K, N, _check(out, y64, ap, K, out_dtype), flush=True)
 

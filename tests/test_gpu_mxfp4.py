@@ -133,15 +133,21 @@ CASES = [
     ([31, 32, 33, 0, 3], 256, 272),
     ([127, 128, 129, 0, 3], 256, 272),   # 97 .. 192-row groups: stacked row halves
     ([200, 7, 0, 90], 1024, 512),
-    ([40, 75, 3], 4096, 512),            # the 64-deep kernel at K >= 4096 too
+    ([40, 75, 3], 4096, 512),            # K >= 4096: the 128-deep kernel (with the further group below)
 ]
+# The launches above of up to 64 rows per group take the streaming kernel: one
+# more group takes the same rows to the tiles.
+CASES += [(sizes + [64 * (len(sizes) + 1)], K, N) for sizes, K, N in CASES if 0 < sum(sizes) <= 64 * len(sizes)]
 
 
 @pytest.mark.parametrize("sizes,K,N", CASES)
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
 def test_mxfp4_gmm_random_shapes(dev, rng, sizes, K, N, out_dtype):
+    from dw_tpu_amd import _lib
     lhs_bits, rhs, sc, gs = _case(rng, sizes, K, N)
     out = _gmm(dev, lhs_bits, rhs, sc, gs, out_dtype)
+    tiles = "gmm_mx128" if K >= 4096 else "gmm_mx"
+    assert _lib.last_kernel() == (tiles if sum(sizes) > 64 * len(sizes) else "gmm_mx_stream")
     y64, terms, _ = _oracle(lhs_bits, _w(rhs, sc), gs)
     print(sizes, K, N, out_dtype, _check(out, y64, terms, K, out_dtype), flush=True)
 

@@ -169,3 +169,36 @@ def test_skinny_forms_against_oracle(dev, a8, M, K, N):
     wide = K <= 1024 and N % 64 == 0 and N >= 128 * torch.cuda.get_device_properties(dev).multi_processor_count
     assert _lib.last_kernel() == f"dense_skinny/{waves}/{2 if waves == 16 else 1}/{4 if wide else 1}"
     _check(out[:, torch.from_numpy(cols).to(dev)], y64, ap, K)
+
+
+def test_w8a8_rows_in_block_accumulation(dev):
+    """The 16x16x128 fp8 MFMA of the rows kernel on rows that cancel inside
+    one K block (448, -448 at some distance, then small values; weights and
+    scales 1): it loses what the 32x32x64 MFMA of the tiles loses.  That is the
+    alignment of small products to a large one, up to 2^-12 of it (the scaled
+    MFMA's measured figure, see ``gmm.mx_error_bound``), here for two large
+    ones, next to the bf16 output's half ulp."""
+    from dw_tpu_amd import _lib
+    from dw_tpu_amd.dense_fp8 import matmul_w8a8
+    from dw_tpu_amd.dense_fp8_tiles import DenseTile
+    K, N = 128, 128
+    rows = []
+    for v in (1.0, 0.375, 0.0625, 0.046875, 2.0 ** -5, 2.0 ** -6, 2.0 ** -7, 2.0 ** -9, 3 * 2.0 ** -9):
+        for at in (1, 9, 17, 33, 40, 65, 100, 127):
+            r = np.full(K, v, np.float32)
+            r[0], r[at] = 448.0, -448.0
+            rows.append(r)
+    x = torch.from_numpy(np.stack(rows)).to(dev).to(torch.float8_e4m3fn)
+    M = len(rows)
+    assert 65 <= M <= 96
+    args = (x, torch.ones((M, 1), device=dev), torch.ones((K, N), device=dev).to(torch.float8_e4m3fn),
+            torch.ones((1, 1), device=dev))
+    want = x.float().double().sum(1).cpu().numpy()
+    err = {}
+    for tile in (None, DenseTile("native", 128, 128, 128, 4)):
+        y = matmul_w8a8(*args, **({} if tile is None else dict(tile=tile)))
+        y = y[:, 0].float().cpu().numpy().astype(np.float64)
+        err[_lib.last_kernel()] = np.maximum(0, np.abs(y - want) - 2.0 ** -9 * np.abs(want)) / 448.0
+    print({k: float(e.max()) for k, e in err.items()})
+    assert np.array_equal(err["dense_rows"], err["dense_mfma"])
+    assert err["dense_rows"].max() <= 2 * 2.0 ** -12

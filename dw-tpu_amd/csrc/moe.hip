@@ -169,7 +169,9 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_kernel(
 // Up to kWideMax ids in one launch: block b of 1024 threads counts all n ids
 // by key in LDS (those before its portion and the rest apart; every block
 // reads the ids from L2), scans the totals, and places its own 1024 ids.  One
-// block needs no count: the portion is the batch.
+// block needs no count, the portion is the batch: the waves' counts are added
+// up as they are ranked (summing them per key after a barrier took 0.3 us at
+// 256 experts, 0.7 at 1024).
 // What bounds three launches (count, scan, scatter) is their latency, not
 // their work: 24576 ids over 256 experts took 3.9 + 6.5 + 6.4 us and the gaps
 // between them, this kernel one launch.  The repeated count grows with n and
@@ -204,8 +206,10 @@ __global__ __launch_bounds__(kFusedThreads) void dispatch_wide_kernel(const int3
   if (many) {
     for (int e = tid; e < stride * copies; e += kFusedThreads) s_bef[e] = s_rest[e] = 0;
   }
-  for (int e = tid; e <= E; e += blockDim.x)
+  for (int e = tid; e <= E; e += blockDim.x) {
+    if (!many) s_bef[e] = s_rest[e] = 0;
     for (int w = 0; w < waves; ++w) s_wcnt[w][e] = 0;
+  }
   const int64_t base = (int64_t)blockIdx.x * kFusedThreads, j = base + tid;
   const bool active = j < n;
   bool bad = false;
@@ -220,7 +224,11 @@ __global__ __launch_bounds__(kFusedThreads) void dispatch_wide_kernel(const int3
   }
   const int rank = __popcll(peers & ((1ull << lane) - 1ull));
   __syncthreads();
-  if (active && rank == 0) s_wcnt[wave][key] = __popcll(peers);
+  if (active && rank == 0) {
+    const int mine = __popcll(peers);
+    s_wcnt[wave][key] = mine;
+    if (!many) atomicAdd(&s_rest[key], mine);  // the portion is the batch
+  }
   if (many) {
     const int copy = (lane & (copies - 1)) * stride;
     for (int64_t j0 = 0; j0 < n; j0 += U * kFusedThreads) {
@@ -239,15 +247,7 @@ __global__ __launch_bounds__(kFusedThreads) void dispatch_wide_kernel(const int3
   }
   if (bad && flags && blockIdx.x == 0) atomicOr(flags, 1);
   __syncthreads();
-  if (!many) {
-    for (int e = tid; e <= E; e += blockDim.x) {
-      int r = 0;
-      for (int w = 0; w < waves; ++w) r += s_wcnt[w][e];
-      s_bef[e] = 0;
-      s_rest[e] = r;
-    }
-    __syncthreads();
-  } else if (copies > 1) {
+  if (many && copies > 1) {
     for (int e = tid; e <= E; e += kFusedThreads) {
       int b = s_bef[e], r = s_rest[e];
       for (int c = 1; c < copies; ++c) {

@@ -298,7 +298,8 @@ def prep_dispatch_combine(dev, steps, warmup):
         assert keep
         res = {}
         ms = time_steps(lambda i: call(lib.dwm_moe_dispatch, disp_args), steps, warmup)
-        res["dispatch"] = {"ms": round(ms, 5), "ids": n, "experts": wl.E, "kernels": 1 if n <= 65536 else 3,
+        one_launch = n <= (65536 if wl.E >= 128 else 49152)
+        res["dispatch"] = {"ms": round(ms, 5), "ids": n, "experts": wl.E, "kernels": 1 if one_launch else 3,
                            "note": "launch-latency bound"}
         ms = time_steps(lambda i: call(lib.dwm_row_gather, gargs[i % gc]), steps, warmup)
         gb = wl.T * wl.K * 2 + n * wl.K * 2 + n * 4

@@ -9,11 +9,12 @@
 // acc += part * (sx[m, kb] * sw[kb, n / 128]).
 //
 // Kernels:
-// - M > 16, N % 128 == 0: dense_fp8_mfma_kernel.  W8A16 decodes e4m3 -> bf16
+// - Larger M, N % 128 == 0: dense_fp8_mfma_kernel.  W8A16 decodes e4m3 -> bf16
 //   (exact: 3 mantissa bits, exponents inside bf16's range) for bf16 MFMA
 //   32x32x16; W8A8 runs the fp8 MFMA 32x32x64 on the codes.
 // - M <= 16: dense_fp8_skinny_kernel (see below).
-// - 17 <= M <= 32, or W8A8 up to 96 (its N % 128 == 0): dense_fp8_rows_kernel (see below).
+// - 17 <= M <= 32, or W8A8 up to 96 (its N % 128 == 0): dense_fp8_rows_kernel,
+//   except where the tiles are faster (rows_rule; see below).
 // - W8A16, M > 64, other N: the MFMA tiles with a clamped last column tile.
 // - Other shapes: dense_fp8_kernel, bf16 MFMA 16x16x32 on decoded codes.
 // Every product is the exact fp8 (or bf16 x fp8) product; the 128-K partial

@@ -717,15 +717,27 @@ static int balanced_tiles() {
   return (*end == 0 && v >= 0 && v <= (1l << 30)) ? (int)v : kGmmBalancedTiles;
 }
 
-// Few rows per expert: the streaming kernel (gmm_stream.hip).  Measured
-// against the tiles below (both with streaming weight loads), us:
-//   32 experts, K = 7168, N = 4096: 1 token 49 -> 23; 4 rows an expert 81 -> 79, 10 rows 82 -> 91;
-//   256 experts, K = N = 4096: 3 rows an expert 398 -> 339, 7 rows 414 -> 386, 12 rows 412 -> 446;
-//   e4m3 lhs, 32 experts, K = 7168, N = 4096: half a row an expert 57 -> 40, 4 rows 83 -> 81, 10 rows 85 -> 92;
-// so it is taken up to 6 rows per local expert; and, while an expert's rows
-// make one tile, also where even 256-column tiles would leave half of the CUs
-// idle (8 experts of 50 rows, K = 3072, N = 2560: 31 -> 26, e4m3 lhs 34 -> 24;
-// K = 1024, N = 640: 16 -> 8, 17 -> 10).
+// Few rows per expert: the streaming kernel (gmm_stream.hip).  Tiles below ->
+// it, us, at 6 rows per local expert, where the rule ends (even groups / half
+// of the rows in one / all in four):
+//   32 experts, K = 7168, N = 4096: bf16 86 / 133 / 47 -> 74 / 100 / 34,
+//     e4m3 86 / 117 / 50 -> 73 / 95 / 27, e2m1 85 / 117 / 49 -> 74 / 80 / 23;
+//   256 experts, K = N = 4096: bf16 420 / 432 / 85 -> 347 / 374 / 107,
+//     e4m3 395 / 401 / 43 -> 341 / 356 / 70, e2m1 394 / 401 / 41 -> 338 / 346 / 51.
+// (10 even rows per expert: 82 -> 91 and 85 -> 92 in the first shape, 12 in
+// the second 412 -> 446.)  The last column is what it costs that the host does
+// not know the sizes: from about 600 rows on that all fall on four experts the
+// tiles are faster, and every spread of 256 experts' rows gains more than that.
+// Rows are counted against the local experts, also where the launch is one
+// window of many more groups (an expert-parallel shard) and M holds the rows
+// of all shards: M bounds what the window can hold, and such launches keep the
+// tiles.
+// It is taken too where at most 64 rows per expert, on average, make so few
+// tiles that even 256-column ones leave half of the CUs idle.  Even groups /
+// half of the rows in one:
+//   8 experts of 50 rows, K = 3072, N = 2560: bf16 26 / 26 -> 23 / 22, e4m3 27 / 27 -> 18 / 17, e2m1 26 / 25 -> 14 / 15;
+//   8 of 64, K = 1024, N = 640: bf16 12 / 14 -> 6.8 / 7.1, e4m3 10 / 13 -> 5.2 / 5.5, e2m1 10 / 12 -> 4.7 / 5.1;
+//   (the worst seen: 4 of 64, Zipf, K = 3072, N = 5120, bf16: 8% slower).
 bool gmm_streams(int64_t M, int64_t N, int64_t E_local) {
   if (M <= 6 * E_local) return true;
   return M <= 64 * E_local && (M / 96 + E_local) * ((N + 255) / 256) <= device_cu_count() / 2;

@@ -304,7 +304,8 @@ int dwm_moe_dispatch_workspace_size(int64_t n, int num_experts, int64_t *bytes);
  *   group_offsets (nullable) = [0, cumsum(group_sizes)]  (num_experts + 1 entries)
  * Bit-exact.  Ids outside [0, num_experts) are rejected on the device:
  * `flags` (device int32[1], nullable) gets bit 0 ORed in and such ids are
- * ordered after every valid id. */
+ * ordered after every valid id.  The outputs must not overlap topk_ids (every
+ * block of a launch reads all of the ids). */
 int dwm_moe_dispatch(const int32_t *topk_ids, int64_t T, int topk, int num_experts,
                      int32_t *perm, int32_t *tok_sorted, int32_t *revert, int32_t *group_sizes,
                      int32_t *group_offsets, int32_t *flags, void *workspace, void *stream);
@@ -469,7 +470,8 @@ int dwm_dense_fp8_w8a8_plan(const uint8_t *xq, const float *sx, int64_t M, int64
                             void *workspace, int64_t workspace_bytes, void *stream);
 
 /* The plan of the last dense GEMM this thread launched (all zero before the
- * first), so callers and tests can see which configuration ran. */
+ * first), so callers and tests can see which configuration ran (of the skinny
+ * kernel's forms dwm_last_kernel tells which). */
 int dwm_dense_fp8_last_plan(dwm_dense_plan *plan);
 
 /* ---------------------------------------------------------------------- */

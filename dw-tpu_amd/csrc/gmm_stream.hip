@@ -321,11 +321,13 @@ int launch_gmm_stream(const uint16_t *lhs, const int32_t *row_idx, int64_t lhs_r
   hipLaunchKernelGGL((gmm_fp4_stream_kernel<WPB, R16, ACT>), dim3(sg.blocks), dim3(64 * WPB), 0, st, lhs,       \
                      row_idx, lhs_rows, M, (int)K, weight, scale, group_sizes, num_groups, group_offset, E_local, \
                      (int)N, out, out_f32, ep, sg.max_rt, ncu)
-  // At most half a round of waves never takes 16-row tiles (stream_tile): it
-  // runs the kernel without that choice (0.2 us less search: 8 rows, K =
+  // 16-row tiles are taken (stream_tile) past half a round of waves, and make
+  // a difference with a group of more than 16 rows: a launch too small for
+  // both runs the kernel without that choice (0.2 us less search: 8 rows, K =
   // 2048, N = 7168 12.3 -> 12.0).
   const int ncu = device_cu_count();
-  const bool r16 = 2 * sg.max_rt * ((N + 63) / 64) > 8 * ncu;
+  const int64_t half = 4 * (int64_t)ncu / ((N + 63) / 64);  // row tiles in half a round
+  const bool r16 = sg.max_rt > half && M > 16 + half;
   if (gated) {
     if (sg.wpb == 4) DWM_STREAM(4, true, true);
     else if (r16) DWM_STREAM(1, true, true);

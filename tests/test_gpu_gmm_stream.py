@@ -42,6 +42,9 @@ CASES = [
     (128, 128, 4096, [192] + [0] * 31, None, True, "none"),
     (64, 128, 4096, [7, 0, 0, 0, 0, 7, 0], None, False, "f32"),
     (64, 256, 4096, [64] + [1] * 63, None, False, "none"),
+    # one-wave blocks with the choice of 16-row tiles (a group of 20 among single rows) and just too small for it
+    (32, 256, 4096, [20] + [1] * 20 + [0] * 11, None, False, "none"),
+    (32, 256, 4096, [16] + [1] * 16 + [0] * 15, None, True, "none"),
     # more rows per expert, in launches too small to fill the chip with tiles: 33 .. 64 rows of all, one and both
     # clauses' edges (12 and 64 rows per expert), a window
     (4, 384, 640, [50, 0, 64, 33], None, False, "none"),

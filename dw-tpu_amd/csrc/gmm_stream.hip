@@ -58,7 +58,8 @@ struct StreamRef {
 // round, and where 16 would not fit the grid.  Against 32 throughout, us: 384 rows over 64
 // experts by a Zipf law (1.1), K = N = 4096 100.5 -> 90.5; 192 such rows over
 // 32 experts, K = 2048, N = 7168 50.5 -> 44.0; 32 of 64 rows in one of 32
-// experts, K = 7168 101.5 -> 86.2.  Against 16 throughout: 1536 rows in one
+// experts, K = 7168 101.5 -> 86.2 (but 20 of 40 rows there 55.4 -> 61.2, the
+// tiles of gmm_fp4.hip 65.8).  Against 16 throughout: 1536 rows in one
 // of 256 experts 121 -> 109; 192 Zipf rows over 32 experts, K = 7168 94 -> 88.
 //
 // Blocks of four waves share their lhs rows through L1.  A launch of at most
